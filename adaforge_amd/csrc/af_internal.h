@@ -195,6 +195,19 @@ int set_error(int code, std::string msg);
 // ilogb of the block's max |x|) as two fp16 halves, hi = f16(u) and lo = f16(u - hi):
 //   hi  fp16 [nb][Tp][32], then lo fp16 [nb][Tp][32], then the scales 2^(e - 14) as float [nb][Tp]
 constexpr uint32_t kBatchMax = 32;   // tokens per batch (crates/cuda-backend/src/batch.rs:10 MAX_BATCH)
+// Prompt positions per prefill pass.  A pass of more than kBatchMax positions takes the wide GEMM
+// (wide_gemm_kernel), whose input image is laid out as its MFMAs read it and holds one scale per
+// token: with G = ceil(T / M) M / 16 groups of 16 tokens (M = wide_tokens(T)),
+//   fp16 [nb][G][hi, lo][64 lanes][8], then the tokens' scales 2^(e - 14) as float [16 G]
+// where lane 16 q + t % 16 holds elements 4 q + {0, 2}, 16 + 4 q + {0, 2}, 4 q + {1, 3}, 16 + 4 q +
+// {1, 3} of token t's block: the order in which a dword of four code bytes unpacks.
+constexpr uint32_t kPassMax = 512;
+// Tokens of a wide GEMM workgroup's tile: 128, or 64 when a tile of 128 would be half padding.
+__host__ __device__ inline uint32_t wide_tokens(uint32_t T) { return T % 128 == 0 || T % 128 > 64 ? 128u : 64u; }
+__host__ __device__ inline uint32_t wide_groups(uint32_t T) {
+    const uint32_t m = wide_tokens(T);
+    return (T + m - 1) / m * (m / 16);
+}
 constexpr uint32_t kVerifyMax = 16;  // tokens per speculative verification pass (batch.rs:13 MAX_VERIFY)
 
 enum BatchInputKind : int { BI_PLAIN = 0, BI_RESID = 1, BI_EMBED = 2 };
@@ -224,6 +237,7 @@ struct BatchIn {
     const float* part;
     uint32_t parts;
     size_t part_row;
+    uint32_t part_tp;       // Tp of the planes
     int8_t* img;
 };
 
@@ -243,21 +257,25 @@ constexpr uint32_t kDeferParts = 16, kDeferPairParts = 4;
 
 // Attention of a batch over the KV cache after the append pass (batch_attention_kernel): the
 // tokens' queries q[t][q_heads][D], token t at position pos0 + t seeing keys [max(0, pos0 + t + 1 -
-// window), pos0 + t] (window 0: from 0).  Keys [klo, pos0 + T) go in nchunks chunks of span keys
-// (a multiple of the kernel's sub-chunk); chunk partials (sum p v, max, sum p) per (token, head).
+// window), pos0 + t] (window 0: from 0).  A query tile's keys go in nchunks chunks (whole sub-chunks of
+// the kernel); chunk partials (sum p v, max, sum p) per (token, head).
 struct BatchAttn {
     const float* q;
     const uint16_t* kcache;
     const uint16_t* vcache;
     uint32_t ring, window, T, pos0, kv_heads, group;
     float scale;
-    uint32_t klo, span, nchunks;
+    uint32_t nchunks;
     float* part;             // [T q_heads][nchunks][D + 2]
     float* out;              // [T][out_stride]: head qh at qh D
     size_t out_stride;
 };
-constexpr uint32_t kBatchAttnChunks = 32;  // chunk partials per (token, head) at most
+constexpr uint32_t kBatchAttnChunks = 32;  // chunk partials per (token, head) at most, and in all at most
+                                           // kBatchAttnChunks kBatchMax tokens' worth of each head
 
+// Tokens of a batch's split-K partial planes (its padded tokens).
+uint32_t batch_padded(uint32_t tokens);
+// Largest input image of a batch of at most `tokens` tokens.
 size_t batch_image_bytes(uint32_t blocks, uint32_t tokens);
 hipError_t launch_batch_attention(BatchAttn a, uint32_t head_width, hipStream_t s);
 size_t batch_gemm_part_bytes(uint32_t rows, uint32_t blocks, uint32_t tokens, bool gelu_pair);

@@ -978,11 +978,15 @@ struct af_session {
     bool poisoned = false;
     bool use_graphs = true;
     KernelTimer* timer = nullptr;  // set during af_session_profile
-    // Batched prefill (batch.hip): prompt positions run through the layers up to kBatchMax at a time,
-    // every weight read once per batch.  prefill_batch: positions per batch for generation
-    // (AF_PREFILL_BATCH, default kBatchMax; 0 or 1 prefills one position per step-kernel launch);
-    // trace_batch: the same for af_session_trace (AF_TRACE_BATCH, default 0: the step kernel).
-    uint32_t prefill_batch = kBatchMax, trace_batch = 0;
+    // Batched prefill (batch.hip): prompt positions run through the layers up to kPassMax at a time,
+    // every weight read once per pass.  prefill_batch: positions per pass for generation
+    // (AF_PREFILL_BATCH; 0 or 1 prefills one position per step-kernel launch); trace_batch: the same
+    // for af_session_trace (AF_TRACE_BATCH, default 0: the step kernel).
+    uint32_t prefill_batch = kPassMax, trace_batch = 0;
+    // The longest batched pass of this session: the batch buffers' tokens, and the slots a sliding
+    // window's ring has beyond the window.  At least a verification pass or kBatchMax, and no longer
+    // than the positions the session can hold.
+    uint32_t pass_max() const { return std::min(std::max({prefill_batch, trace_batch, kBatchMax}), std::max(capacity, kBatchMax)); }
     // Greedy speculative decoding with prompt-lookup drafts (AF_SPECULATIVE=1; AF_SPEC_DEPTH draft
     // tokens at most, default 11, at most kVerifyMax - 1): the draft and the pending token run through
     // the batched layers in one pass and the head checks the positions, up to four per launch.
@@ -1323,12 +1327,12 @@ struct af_session {
         uint32_t blocks = std::max({hidden, max_q, intermediate}) / 32;
         size_t part = 4;
         for (const LayerDev& L : layers) {
-            part = std::max({part, batch_gemm_part_bytes(L.qkv.rows, hidden / 32, kBatchMax, false),
-                             batch_gemm_part_bytes(L.o.rows, L.qn / 32, kBatchMax, false),
-                             batch_gemm_part_bytes(L.gate.rows, hidden / 32, kBatchMax, true),
-                             batch_gemm_part_bytes(L.down.rows, intermediate / 32, kBatchMax, false)});
+            part = std::max({part, batch_gemm_part_bytes(L.qkv.rows, hidden / 32, pass_max(), false),
+                             batch_gemm_part_bytes(L.o.rows, L.qn / 32, pass_max(), false),
+                             batch_gemm_part_bytes(L.gate.rows, hidden / 32, pass_max(), true),
+                             batch_gemm_part_bytes(L.down.rows, intermediate / 32, pass_max(), false)});
         }
-        const size_t T = kBatchMax;
+        const size_t T = pass_max();
         struct {
             DevMem* m;
             size_t bytes;
@@ -1336,8 +1340,9 @@ struct af_session {
             {&XB, T * hidden * 4},        {&HB, T * hidden * 4},  {&QKVB, T * max_qkv * 4},
             {&ATTB, T * max_q * 4},       {&QB, T * max_q * 4},   {&PROJB, T * hidden * 4},
             {&ACTB, T * intermediate * 4},
-            {&DB, T * hidden * 4},        {&BIMG, batch_image_bytes(blocks, kBatchMax)}, {&BGEMM, part},
-            {&BPART, T * kBatchAttnChunks * max_qh_part * 4}, {&BCOUNT, T * std::max<uint32_t>(max_qh, 64) * 4},
+            {&DB, T * hidden * 4},        {&BIMG, batch_image_bytes(blocks, (uint32_t)T)}, {&BGEMM, part},
+            {&BPART, (size_t)kBatchMax * kBatchAttnChunks * max_qh_part * 4},
+            {&BCOUNT, T * std::max<uint32_t>(max_qh, 64) * 4},
         };
         for (auto& b : bufs) {
             int rc = dev_alloc(*b.m, b.bytes, "batch buffer");
@@ -1380,6 +1385,7 @@ struct af_session {
     // deferred its reduce (parts > 0), else y.
     BatchIn resid_input(uint32_t T, const float* y, uint32_t parts) {
         BatchIn in = batch_in(BI_RESID, T, hidden, y, hidden);
+        in.part_tp = batch_padded(T);
         if (parts) {
             in.part = BGEMM.as<float>();
             in.parts = parts;
@@ -1455,7 +1461,7 @@ struct af_session {
                 aa.raw_part = BGEMM.as<float>();
                 aa.raw_parts = qkv_parts;
                 aa.raw_prow = (L.qkv.rows + 15) / 16 * 16;
-                aa.raw_tp = (T + 15) / 16 * 16;
+                aa.raw_tp = batch_padded(T);
             }
             if ((e = launch_attention(aa, aa.group, L.width, stream, T)) != hipSuccess) return e;
             BatchAttn ba{};
@@ -1491,6 +1497,7 @@ struct af_session {
             if ((e = batch_gemm(L.gate, &L.up, T, ACTB.as<float>(), intermediate, &ff_parts)) != hipSuccess) return e;
 
             in = batch_in(BI_PLAIN, T, intermediate, ACTB.as<float>(), intermediate);
+            in.part_tp = batch_padded(T);
             if (ff_parts) {
                 in.part = BGEMM.as<float>();
                 in.parts = ff_parts;
@@ -1753,9 +1760,9 @@ int open_session(const af_layer_weights* layers, uint32_t n_layers, const af_out
     // layer l's down projection) waits for one arrival more than the grid makes, and times out.
     if (const char* fp = std::getenv("AF_STEP_FAIL_PHASE")) s->fail_phase = (uint32_t)std::strtoul(fp, nullptr, 10);
     if (const char* pb = std::getenv("AF_PREFILL_BATCH"))
-        s->prefill_batch = std::min<uint32_t>((uint32_t)std::strtoul(pb, nullptr, 10), kBatchMax);
+        s->prefill_batch = std::min<uint32_t>((uint32_t)std::strtoul(pb, nullptr, 10), kPassMax);
     if (const char* tb = std::getenv("AF_TRACE_BATCH"))
-        s->trace_batch = std::min<uint32_t>((uint32_t)std::strtoul(tb, nullptr, 10), kBatchMax);
+        s->trace_batch = std::min<uint32_t>((uint32_t)std::strtoul(tb, nullptr, 10), kPassMax);
     if (const char* sp = std::getenv("AF_SPECULATIVE")) s->speculative = std::strcmp(sp, "1") == 0;
     if (const char* sd = std::getenv("AF_SPEC_DEPTH"))
         s->spec_depth = std::max<uint32_t>(1, std::min<uint32_t>((uint32_t)std::strtoul(sd, nullptr, 10), kVerifyMax - 1));
@@ -1797,10 +1804,10 @@ int open_session(const af_layer_weights* layers, uint32_t n_layers, const af_out
         if ((rc = dev_upload(L.post_ffn, w.ffn.post.weights, (size_t)hidden * 4, "norm upload"))) return rc;
         std::vector<double> f = inverse_frequencies(w.rope);
         if ((rc = dev_upload(L.inv_freq, f.data(), f.size() * 8, "RoPE upload"))) return rc;
-        // Sliding-window layers keep a ring of window + kBatchMax slots (crates/cuda-backend/src/
-        // stack.rs:94-102): a batch appends up to kBatchMax positions before any of them attends,
+        // Sliding-window layers keep a ring of window + pass_max() slots (crates/cuda-backend/src/
+        // stack.rs:94-102): a pass appends up to pass_max() positions before any of them attends,
         // and the first still sees its window - 1 predecessors.
-        L.ring = L.window ? std::min(L.window + kBatchMax, capacity) : capacity;
+        L.ring = L.window ? (uint32_t)std::min<uint64_t>((uint64_t)L.window + s->pass_max(), capacity) : capacity;
         const size_t kv = (size_t)L.kv_heads * L.ring * L.width * 2;
         if ((rc = dev_alloc(L.kcache, kv, "K cache"))) return rc;
         if ((rc = dev_alloc(L.vcache, kv, "V cache"))) return rc;
@@ -1933,7 +1940,7 @@ std::vector<uint32_t> draft_lookup(const std::vector<uint32_t>& h, size_t limit)
 // the batched layers at once, the head runs over the positions (up to kHeadBatchMax per launch, the
 // table read once per launch) until the first prediction that differs from the draft, the
 // matching draft tokens are emitted, and the caches keep only their
-// positions (the rest are overwritten later: a local ring holds window + kBatchMax slots).  The
+// positions (the rest are overwritten later: a local ring holds at least window + kBatchMax slots).  The
 // emitted ids are the greedy ids of plain decoding, up to the arithmetic of the batched layers.
 int speculate(af_session* s, const uint32_t* prompt, size_t n_prompt, const uint32_t* stop, size_t n_stop,
               uint32_t max_new, af_token_fn on_token, void* user, uint32_t* ids_out, size_t* n_out,
@@ -2451,7 +2458,7 @@ int af_session_trace(af_session* s, const uint32_t* ids, size_t n, float* layer_
     if (s->trace_batch > 1) {
         // every position through the batched layers: layer outputs and appended K/V per batch
         if ((rc = s->ensure_batch())) return rc;
-        if (layer_outputs && (rc = grow(s->SNAP, (size_t)kBatchMax * nl * H * 4, false, "trace buffer"))) return rc;
+        if (layer_outputs && (rc = grow(s->SNAP, (size_t)std::max(kBatchMax, s->trace_batch) * nl * H * 4, false, "trace buffer"))) return rc;
         const uint32_t B = s->trace_batch, first = s->consumed + (uint32_t)pend;
         HIP_OK(s->prefill_batched(s->consumed, first, B), "trace batch");
         uint32_t T = 0;

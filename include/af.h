@@ -247,8 +247,8 @@ int af_session_open(const af_layer_weights* layers, uint32_t n_layers, const af_
  * session's cached tokens; at most max_new (1..AF_MAX_NEW_TOKENS) greedy ids, stopping before
  * any id in `stop` (non-empty).  on_token may be NULL.  ids_out holds >= max_new ids.
  * Environment switches read at af_session_open: AF_PREFILL_BATCH (prompt positions per batched
- * pass, default 32; 0 or 1: one decode step per position, as ADAFORGE_BATCH_PREFILL=0,
- * stack.rs:982-987); AF_SPECULATIVE=1 with AF_SPEC_DEPTH (default 11, at most 15): greedy
+ * pass, at most and by default 512; 0 or 1: one decode step per position, as
+ * ADAFORGE_BATCH_PREFILL=0, stack.rs:982-987); AF_SPECULATIVE=1 with AF_SPEC_DEPTH (default 11, at most 15): greedy
  * speculative decoding with prompt-lookup drafts verified in one batched pass (ADAFORGE_SPECULATIVE,
  * ADAFORGE_SPEC_DEPTH, stack.rs:1252-1338, 1485-1511).  A verification pass predicts each position
  * from the batched layers, which sum in another order than the decode step (the reference's batched

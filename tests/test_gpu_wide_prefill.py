@@ -1,0 +1,67 @@
+"""Prefill passes of more than 32 positions (wide_gemm_kernel, its input images and the batched
+attention over whole passes) against the CPU oracle, teacher-forced per layer."""
+import os
+
+import numpy as np
+import pytest
+
+import oracle
+from adaforge_amd import synth
+from tests.test_gpu_batch import THREADS, open_with_env
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("q_heads,kv_heads,window,intermediate,n,batch", [
+    (16, 8, 16, 2048, 33, 33),     # one 64-token tile, nearly half padding
+    (16, 8, 100, 2080, 64, 64),    # a full 64-token tile; FFN rows and columns off every tile
+    (8, 8, 24, 1056, 150, 65),     # a 128-token tile, then one that ends a pass of 65 + 65 + 20
+    (16, 4, 64, 2048, 280, 128),   # full 128-token tiles; two passes and a narrow remainder
+    (16, 8, 40, 2080, 330, 161),   # three 64-token tiles; the window's ring wraps inside the pass
+    (16, 8, 1024, 2048, 530, 512), # the largest pass, then a narrow one
+])
+def test_wide_trace_teacher_forced(q_heads, kv_heads, window, intermediate, n, batch):
+    """Layer outputs within the oracle's tolerance (|gpu - ref| <= 1e-4 + 1e-4 |ref|) and K/V within one
+    fp16 ulp at tile, window and pass boundaries."""
+    model = synth.model(name=f"wide{q_heads}x{kv_heads}", layers=3, hidden=1024, intermediate=intermediate,
+                        q_heads=q_heads, kv_heads=kv_heads, head_width=256, vocabulary=2048, window=window,
+                        global_every=3)
+    ids = [int(i) for i in synth.prompt_ids(n, model.vocabulary, name=f"wide{n}.ids")]
+    with open_with_env(model, n + 8, AF_TRACE_BATCH=batch) as s:
+        outputs, kv, logits, hidden = s.trace(ids, kv_rows=kv_heads * 256)
+    marks = {0, 1, 15, 16, 31, 32, 63, 64, 127, 128, window - 1, window, batch - 1, batch, batch + 1, n - 1}
+    positions = sorted(p for p in marks if 0 <= p < n)
+    ratio, ulps, differ = oracle.check_layer_stack(model, ids, outputs, kv, threads=THREADS, positions=positions)
+    print(f"wide trace n={n} batch={batch}: layer ratio {ratio:.3f}, K/V ratio {ulps:.3f}, {differ} fp16 values differ",
+          flush=True)
+    nrm = oracle.rmsnorm(model.final_norm, model.final_eps, hidden).astype(np.float32)
+    oracle.compare(oracle.q6_matvec(model.table, model.hidden, model.vocabulary, nrm, threads=THREADS), logits)
+
+
+def test_wide_trace_gemma4_width_512_shared_v():
+    """The 512-wide global layer (16 query heads on one KV head, V from K's weights) in wide passes."""
+    model = synth.gemma4_model(name="gemma4-wide", layers=6, hidden=1024, intermediate=2048, local_q=(16, 8, 256),
+                               global_q=(16, 1, 512), vocabulary=2048, window=48)
+    n = 150
+    ids = [int(i) for i in synth.prompt_ids(n, model.vocabulary, name="gemma4-wide.ids")]
+    kv_rows = max(L.kv_heads * L.head_width for L in model.layers)
+    with open_with_env(model, n + 8, AF_TRACE_BATCH=100) as s:
+        outputs, kv, _, _ = s.trace(ids, kv_rows=kv_rows, logits=False, hidden=False)
+    positions = [0, 1, 15, 16, 47, 48, 63, 64, 99, 100, 101, 147, 149]
+    ratio, ulps, differ = oracle.check_layer_stack(model, ids, outputs, kv, threads=THREADS, positions=positions)
+    print(f"gemma4 wide: layer ratio {ratio:.3f}, K/V ratio {ulps:.3f}, {differ} fp16 values differ", flush=True)
+
+
+def test_wide_prefill_ids_match_one_position_at_a_time():
+    """Greedy ids after a 300-token prompt: one wide pass against one step-kernel launch per position, and
+    again on a follow-up turn whose pass starts in the middle of the ring."""
+    model = synth.model(name="wide-gen", layers=3, hidden=1024, intermediate=2048, q_heads=16, kv_heads=8,
+                        head_width=256, vocabulary=2048, window=64, global_every=3)
+    prompt = [int(i) for i in synth.prompt_ids(300, model.vocabulary, name="wide-gen.prompt")]
+    more = [int(i) for i in synth.prompt_ids(90, model.vocabulary, name="wide-gen.more")]
+    got = []
+    for batch in (512, 0):
+        with open_with_env(model, 420, AF_PREFILL_BATCH=batch) as s:
+            first = s.generate(prompt, [2047], 8)
+            got.append((first.ids, s.generate(prompt + first.ids + more, [2047], 8).ids))
+    assert got[0] == got[1]
