@@ -190,10 +190,6 @@ int set_error(int code, std::string msg);
 
 // ---- batched prefill (batch.hip) ---------------------------------------------------------------
 //
-// Input image of T vectors of nb 32-element blocks for the batched GEMM, with the tokens padded to
-// Tp = 16 ceil(T / 16) (padding tokens all zero): block b of vector t scaled by 2^(14 - e) (e =
-// ilogb of the block's max |x|) as two fp16 halves, hi = f16(u) and lo = f16(u - hi):
-//   hi  fp16 [nb][Tp][32], then lo fp16 [nb][Tp][32], then the scales 2^(e - 14) as float [nb][Tp]
 constexpr uint32_t kBatchMax = 32;   // tokens per batch (crates/cuda-backend/src/batch.rs:10 MAX_BATCH)
 // Prompt positions per prefill pass.  A pass of more than kBatchMax positions takes the wide GEMM
 // (wide_gemm_kernel), whose input image is laid out as its MFMAs read it and holds one scale per
@@ -230,30 +226,28 @@ struct BatchIn {
     const uint32_t* ids;
     uint32_t pos0;          // BI_EMBED: vector t is row ids[pos0 + t]
     float emb_scale;
-    // parts > 0: x comes from the split-K partial planes part[(k Tp + t) part_row + i] that
-    // batch_gemm_kernel left (its reduce deferred), summed in split order: BI_RESID, planes
-    // k < parts; BI_PLAIN without w_n, a gate/up pair: x = gelu(sum of gate planes 2 k) * (sum of up
-    // planes 2 k + 1)
+    // parts > 0 (BI_RESID): x comes from the split-K partial planes part[(k part_tp + t) part_row + i]
+    // that the GEMM left (its reduce deferred), summed in split order
     const float* part;
     uint32_t parts;
     size_t part_row;
-    uint32_t part_tp;       // Tp of the planes
-    int8_t* img;
+    uint32_t part_tp;       // tokens per plane (batch_padded)
+    int8_t* img;            // out: floats [T][K], or above kBatchMax vectors the wide GEMM's image
 };
 
 struct BatchGemm {
     Q4View w, w2;           // w2: the up matrix of a gate/up pair
-    const int8_t* img;      // input image of T vectors of w.blocks blocks (fp16 halves and scales)
+    const float* x;         // up to kBatchMax tokens: the inputs [T][x_stride]
+    size_t x_stride;
+    const int8_t* img;      // above: their image (launch_batch_input)
     uint32_t T;
     float* y;               // y[t * y_stride + r], r < w.rows (gate/up: f32(gelu(gate)) * up)
     size_t y_stride;
-    const float* add;       // optional residual added to y (same layout)
     float* part;            // split-K partials (batch_gemm_part_bytes)
-    bool defer;             // no add: with a split-K plan of at most kDeferParts (a single matrix)
-                            // or kDeferPairParts (a gate/up pair) splits, leave the partials for
-                            // the input kernel of the next GEMM (no y)
+    uint32_t* counters;     // batch_gemm_counters words, zero between launches
+    bool defer;             // a single matrix split over K: leave the partials for the next kernel (no y)
 };
-constexpr uint32_t kDeferParts = 16, kDeferPairParts = 4;
+constexpr uint32_t kDeferParts = 16;  // K splits at most
 
 // Attention of a batch over the KV cache after the append pass (batch_attention_kernel): the
 // tokens' queries q[t][q_heads][D], token t at position pos0 + t seeing keys [max(0, pos0 + t + 1 -
@@ -279,6 +273,7 @@ uint32_t batch_padded(uint32_t tokens);
 size_t batch_image_bytes(uint32_t blocks, uint32_t tokens);
 hipError_t launch_batch_attention(BatchAttn a, uint32_t head_width, hipStream_t s);
 size_t batch_gemm_part_bytes(uint32_t rows, uint32_t blocks, uint32_t tokens, bool gelu_pair);
+size_t batch_gemm_counters(uint32_t rows, bool gelu_pair);
 hipError_t launch_batch_input(const BatchIn& in, hipStream_t s);
 // Returns through parts the splits whose partials were left in a.part (0: y written).
 hipError_t launch_batch_gemm(const BatchGemm& a, bool gelu_pair, hipStream_t s, uint32_t* parts = nullptr);

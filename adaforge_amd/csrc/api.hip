@@ -398,7 +398,7 @@ float median_of(std::vector<float> t) {
 struct Scratch {
     std::mutex mu;
     DevMem head_partial, head_counter, attn_part, attn_counters;
-    DevMem batch_image, batch_part;     // digit image and split-K partials of af_q4_gemm
+    DevMem batch_part, batch_counters;  // split-K partials and tickets of af_q4_gemm
     DevMem attn_freq;                   // the last RoPE inverse frequencies of af_attention_decode
     std::vector<double> attn_freq_host; // their host copy (re-uploaded only when they change)
 };
@@ -501,27 +501,20 @@ int af_q4_gemm(const af_q4* m, const float* x, uint32_t tokens, float* y, void* 
     const Q4View w = m->m.view();
     std::lock_guard<std::mutex> lock(g_scratch.mu);
     int rc;
-    if ((rc = grow(g_scratch.batch_image, batch_image_bytes(w.blocks, kBatchMax), false, "batch digit image")))
-        return rc;
     if ((rc = grow(g_scratch.batch_part, batch_gemm_part_bytes(w.rows, w.blocks, kBatchMax, false) + 4, false,
                    "batch partials")))
         return rc;
+    if ((rc = grow(g_scratch.batch_counters, batch_gemm_counters(w.rows, false) * 4, true, "batch counters"))) return rc;
     const hipStream_t s = (hipStream_t)stream;
-    BatchIn in{};
-    in.mode = BI_PLAIN;
-    in.T = tokens;
-    in.K = w.blocks * 32;
-    in.stride = in.K;
-    in.x = x;
-    in.img = g_scratch.batch_image.as<int8_t>();
-    HIP_OK(launch_batch_input(in, s), "batched GEMV input digits");
     BatchGemm g{};
     g.w = w;
-    g.img = in.img;
+    g.x = x;
+    g.x_stride = w.blocks * 32;
     g.T = tokens;
     g.y = y;
     g.y_stride = w.rows;
     g.part = g_scratch.batch_part.as<float>();
+    g.counters = g_scratch.batch_counters.as<uint32_t>();
     HIP_OK(launch_batch_gemm(g, false, s), "batched GEMV launch");
     return AF_OK;
 }
@@ -994,7 +987,7 @@ struct af_session {
     uint32_t spec_depth = 11;
     uint64_t spec_passes = 0, spec_drafted = 0, spec_accepted = 0;  // since open (af_session_speculation)
     uint32_t max_qh = 0, max_qh_part = 0;
-    DevMem XB, HB, QKVB, QB, ATTB, PROJB, ACTB, DB, BIMG, BGEMM, BPART, BCOUNT;
+    DevMem XB, HB, QKVB, QB, ATTB, PROJB, ACTB, DB, BIMG, BGEMM, BTICKETS, BPART, BCOUNT;
 
     // Launches f(); when profiling, brackets it with an event pair tagged with its kind and bytes.
     template <typename F>
@@ -1325,8 +1318,10 @@ struct af_session {
     int ensure_batch() {
         if (XB.p) return AF_OK;
         uint32_t blocks = std::max({hidden, max_q, intermediate}) / 32;
-        size_t part = 4;
+        size_t part = 4, tickets = 1;
         for (const LayerDev& L : layers) {
+            tickets = std::max({tickets, batch_gemm_counters(L.qkv.rows, false), batch_gemm_counters(L.o.rows, false),
+                                batch_gemm_counters(L.gate.rows, true), batch_gemm_counters(L.down.rows, false)});
             part = std::max({part, batch_gemm_part_bytes(L.qkv.rows, hidden / 32, pass_max(), false),
                              batch_gemm_part_bytes(L.o.rows, L.qn / 32, pass_max(), false),
                              batch_gemm_part_bytes(L.gate.rows, hidden / 32, pass_max(), true),
@@ -1342,17 +1337,18 @@ struct af_session {
             {&ACTB, T * intermediate * 4},
             {&DB, T * hidden * 4},        {&BIMG, batch_image_bytes(blocks, (uint32_t)T)}, {&BGEMM, part},
             {&BPART, (size_t)kBatchMax * kBatchAttnChunks * max_qh_part * 4},
-            {&BCOUNT, T * std::max<uint32_t>(max_qh, 64) * 4},
+            {&BCOUNT, T * std::max<uint32_t>(max_qh, 64) * 4}, {&BTICKETS, tickets * 4},
         };
         for (auto& b : bufs) {
             int rc = dev_alloc(*b.m, b.bytes, "batch buffer");
             if (rc) return rc;
         }
         HIP_OK(hipMemsetAsync(BCOUNT.p, 0, BCOUNT.bytes, stream), "batch counters clear");
+        HIP_OK(hipMemsetAsync(BTICKETS.p, 0, BTICKETS.bytes, stream), "batch counters clear");
         return AF_OK;
     }
 
-    // Digit image of T vectors for the GEMV of matrix m (see BatchIn).
+    // The input of a GEMM over T vectors (see BatchIn), into BIMG.
     BatchIn batch_in(int mode, uint32_t T, uint32_t K, const float* x, size_t stride) {
         BatchIn in{};
         in.mode = mode;
@@ -1365,18 +1361,27 @@ struct af_session {
         return in;
     }
 
-    // parts non-null: the split-K partials may stay in BGEMM for the next input kernel, which then
-    // sums them; *parts tells it how many (0: y written).
+    // y = W x over the batch (m2: the up matrix of a gate/up pair) for the inputs in BIMG, or a plain
+    // input x (K floats per token).  parts non-null: the split-K partials may stay in BGEMM for the next
+    // kernel, which then sums them; *parts tells it how many (0: y written).
     hipError_t batch_gemm(const Q4Dev& m, const Q4Dev* m2, uint32_t T, float* y, size_t y_stride,
-                          uint32_t* parts = nullptr) {
+                          uint32_t* parts = nullptr, const float* x = nullptr) {
+        const uint32_t K = m.columns;
+        if (x && T > kBatchMax) {
+            hipError_t e = launch_batch_input(batch_in(BI_PLAIN, T, K, x, K), stream);
+            if (e != hipSuccess) return e;
+        }
         BatchGemm g{};
         g.w = m.view();
         if (m2) g.w2 = m2->view();
+        g.x = x ? x : BIMG.as<float>();
+        g.x_stride = K;
         g.img = BIMG.as<int8_t>();
         g.T = T;
         g.y = y;
         g.y_stride = y_stride;
         g.part = BGEMM.as<float>();
+        g.counters = BTICKETS.as<uint32_t>();
         g.defer = parts != nullptr;
         return launch_batch_gemm(g, m2 != nullptr, stream, parts);
     }
@@ -1480,10 +1485,8 @@ struct af_session {
             ba.out_stride = L.qn;
             if ((e = launch_batch_attention(ba, L.width, stream)) != hipSuccess) return e;
 
-            in = batch_in(BI_PLAIN, T, L.qn, ATTB.as<float>(), L.qn);
-            if ((e = launch_batch_input(in, stream)) != hipSuccess) return e;
             uint32_t o_parts = 0;
-            if ((e = batch_gemm(L.o, nullptr, T, PROJB.as<float>(), H, &o_parts)) != hipSuccess) return e;
+            if ((e = batch_gemm(L.o, nullptr, T, PROJB.as<float>(), H, &o_parts, ATTB.as<float>())) != hipSuccess) return e;
 
             in = resid_input(T, PROJB.as<float>(), o_parts);
             in.res = XB.as<float>();
@@ -1493,20 +1496,10 @@ struct af_session {
             in.eps_n = L.ffn_eps;
             in.x_out = HB.as<float>();
             if ((e = launch_batch_input(in, stream)) != hipSuccess) return e;
-            uint32_t ff_parts = 0;
-            if ((e = batch_gemm(L.gate, &L.up, T, ACTB.as<float>(), intermediate, &ff_parts)) != hipSuccess) return e;
-
-            in = batch_in(BI_PLAIN, T, intermediate, ACTB.as<float>(), intermediate);
-            in.part_tp = batch_padded(T);
-            if (ff_parts) {
-                in.part = BGEMM.as<float>();
-                in.parts = ff_parts;
-                in.part_row = (size_t)(intermediate + 15) / 16 * 16;
-            }
-            if ((e = launch_batch_input(in, stream)) != hipSuccess) return e;
+            if ((e = batch_gemm(L.gate, &L.up, T, ACTB.as<float>(), intermediate)) != hipSuccess) return e;
             // the last layer's down output stays in DB for the caller
-            if ((e = batch_gemm(L.down, nullptr, T, DB.as<float>(), H, l + 1 < nl ? &down_parts : nullptr)) !=
-                hipSuccess)
+            if ((e = batch_gemm(L.down, nullptr, T, DB.as<float>(), H, l + 1 < nl ? &down_parts : nullptr,
+                                ACTB.as<float>())) != hipSuccess)
                 return e;
         }
         if (!snap) return hipSuccess;

@@ -26,37 +26,14 @@ typedef _Float16 v2h __attribute__((ext_vector_type(2)));
 
 namespace {
 
-constexpr uint32_t kGemmThreads = 256;  // four waves splitting the blocks of the workgroup's K range
-constexpr uint32_t kGemmTargetGrid = 512;
-
-uint32_t padded_tokens(uint32_t T) { return (T + 15) / 16 * 16; }
-
-// Work split of a GEMM: R row tiles per workgroup, S workgroups along K (partials summed by
-// batch_reduce_kernel), so that about kGemmTargetGrid workgroups share the weight stream and each
-// wave keeps at least two blocks.
-struct GemmPlan {
-    uint32_t R, S;
-};
-// The input image is read by every workgroup of a K range, R row tiles at a time, so R sets its
-// reuse: up to 8 tiles (4 of each matrix of a gate/up pair) while at least 32 row groups remain.
-GemmPlan gemm_plan(uint32_t rows, uint32_t blocks, bool pair) {
-    const uint32_t tiles = (rows + 15) / 16, r_max = pair ? 4 : 8;
-    uint32_t R = 1;
-    while (R < r_max && tiles >= 64 * R) R *= 2;
-    const uint32_t wgs = (tiles + R - 1) / R;
-    uint32_t S = std::max<uint32_t>(1, std::min<uint32_t>(32, (kGemmTargetGrid + wgs - 1) / wgs));
-    S = std::max<uint32_t>(1, std::min(S, blocks / 8));
-    return GemmPlan{R, S};
-}
+uint32_t padded_tokens(uint32_t T) { return T <= 8 ? 8 : (T + 15) / 16 * 16; }
 
 }  // namespace
 
 // ---- input images of a batch --------------------------------------------------------------------
 //
-// Image of K = 32 nb inputs for Tp tokens: hi [nb][Tp][32] fp16, then lo [nb][Tp][32] fp16, then
-// [nb][Tp] floats 2^(e - 14) (0 for an all-zero block and for padding tokens).  A quad of threads
-// writes one block, thread p of it elements 4 p .. + 3 and 16 + 4 p .. + 3 (v[0..3], v[4..7]): the
-// eight that one lane of the wide GEMM's operand holds (wide_halves).
+// Elements are taken in octets: part p of a block is elements 4 p .. 4 p + 3 and 16 + 4 p .. + 3, the
+// eight that one lane of an MFMA operand holds.
 
 // x 2^sh as two fp16 halves: hi = f16(u), lo = f16(u - hi), packed in pairs (x0, x1).
 __device__ __forceinline__ void split_pair(float x0, float x1, int sh, uint32_t& hi, uint32_t& lo) {
@@ -67,40 +44,27 @@ __device__ __forceinline__ void split_pair(float x0, float x1, int sh, uint32_t&
     lo = (uint32_t)__builtin_bit_cast(uint16_t, l0) | (uint32_t)__builtin_bit_cast(uint16_t, l1) << 16;
 }
 
-// The halves and the scale of block b of token t from the 8 elements v of part p (all four lanes of
-// the quad take part).
-__device__ __forceinline__ void block_halves(const float (&v)[8], uint32_t b, uint32_t p, uint32_t t, uint32_t Tp,
-                                             _Float16* hi, _Float16* lo, float* inv) {
-    float m, sum;
-    quad_stats(v, m, sum);
-    const int e = m > 0.0f ? ilogbf(m) : 0;
-    uint32_t hw[4], lw[4];
-#pragma unroll
-    for (int k = 0; k < 4; ++k) split_pair(v[2 * k], v[2 * k + 1], 14 - e, hw[k], lw[k]);
-    const size_t at = ((size_t)b * Tp + t) * 32 + 4 * p;
-    *reinterpret_cast<v2u*>(hi + at) = v2u{hw[0], hw[1]};
-    *reinterpret_cast<v2u*>(hi + at + 16) = v2u{hw[2], hw[3]};
-    *reinterpret_cast<v2u*>(lo + at) = v2u{lw[0], lw[1]};
-    *reinterpret_cast<v2u*>(lo + at + 16) = v2u{lw[2], lw[3]};
-    if (p == 0) inv[(size_t)b * Tp + t] = m > 0.0f ? ldexpf(1.0f, e - 14) : 0.0f;
-}
-
-// Part p of block b of token t into the wide GEMM's image of G 16-token groups, scaled by 2^sh: the
-// halves of one operand lane, in the order in which a dword of code bytes unpacks (nibbles_f16).
-__device__ __forceinline__ void wide_halves(const float (&v)[8], int sh, uint32_t b, uint32_t p, uint32_t t, uint32_t G,
-                                            v4u* img) {
+// The halves of an octet (elements 4 p .. + 3 and 16 + 4 p .. + 3 of a block) scaled by 2^sh: one
+// operand lane, in the order in which a dword of code bytes unpacks (unpack_dword).
+__device__ __forceinline__ void octet_halves(const float (&v)[8], int sh, v4u& hi, v4u& lo) {
     uint32_t h0, h1, h2, h3, l0, l1, l2, l3;
     split_pair(v[0], v[2], sh, h0, l0);
     split_pair(v[4], v[6], sh, h1, l1);
     split_pair(v[1], v[3], sh, h2, l2);
     split_pair(v[5], v[7], sh, h3, l3);
-    v4u* at = img + ((size_t)b * G + t / 16) * 128 + 16 * p + t % 16;
-    at[0] = v4u{h0, h1, h2, h3};
-    at[64] = v4u{l0, l1, l2, l3};
+    hi = v4u{h0, h1, h2, h3};
+    lo = v4u{l0, l1, l2, l3};
 }
 
-// One workgroup per token t < Tp (tokens T..Tp-1 write zeros).  The input vector of the GEMV that
-// follows:
+// Part p of block b of token t into the wide GEMM's image of G 16-token groups.
+__device__ __forceinline__ void wide_halves(const float (&v)[8], int sh, uint32_t b, uint32_t p, uint32_t t, uint32_t G,
+                                            v4u* img) {
+    v4u* at = img + ((size_t)b * G + t / 16) * 128 + 16 * p + t % 16;
+    octet_halves(v, sh, at[0], at[64]);
+}
+
+// One workgroup per token.  The input vector of the GEMM that follows (as floats [T][K], or as the wide
+// GEMM's image):
 //   BI_PLAIN: x_t (f32(rms(x_t) w_n) with w_n);
 //   BI_RESID: v_t = (f32(rms(x_t) w_a) + res_t) * scale (w_a null: (x_t + res_t) * scale), stored to
 //             x_out_t (the residual stream), then f32(rms(v_t) w_n);
@@ -118,24 +82,9 @@ __global__ __launch_bounds__(512) void batch_input_kernel(BatchIn in) {
     extern __shared__ __align__(16) float xs[];  // [K], BI_EMBED only
     __shared__ double red[8];
     __shared__ float redf[8];
-    const uint32_t tid = threadIdx.x, K = in.K, nb = K / 32, no = K / 8, Tp = gridDim.x;
+    const uint32_t tid = threadIdx.x, K = in.K, nb = K / 32, no = K / 8, WG = wide_groups(in.T);
     const uint32_t t = WIDE ? blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8 : blockIdx.x;
-    _Float16* hi = reinterpret_cast<_Float16*>(in.img);
-    _Float16* lo = hi + (size_t)nb * Tp * 32;
-    float* inv = reinterpret_cast<float*>(lo + (size_t)nb * Tp * 32);
-    const uint32_t WG = wide_groups(in.T);
-    if constexpr (WIDE) inv = reinterpret_cast<float*>(in.img + (size_t)nb * WG * 2048);
-    if (WIDE && t >= in.T) return;
-    if (t >= in.T) {
-        for (uint32_t o = tid; o < nb * 4; o += blockDim.x) {
-            const uint32_t b = o >> 2, p = o & 3;
-            const size_t at = ((size_t)b * Tp + t) * 32 + 8 * p;
-            *reinterpret_cast<v4u*>(hi + at) = v4u{0u, 0u, 0u, 0u};
-            *reinterpret_cast<v4u*>(lo + at) = v4u{0u, 0u, 0u, 0u};
-            if (p == 0) inv[(size_t)b * Tp + t] = 0.0f;
-        }
-        return;
-    }
+    if (t >= in.T) return;
     const bool resid = in.mode == BI_RESID, embed = in.mode == BI_EMBED;
     const float4 z4 = make_float4(0.f, 0.f, 0.f, 0.f);
     float4 x[NO][2], r[NO][2], wa[NO][2], wn[NO][2];
@@ -242,8 +191,7 @@ __global__ __launch_bounds__(512) void batch_input_kernel(BatchIn in) {
         for (int j = 0; j < NO; ++j) ss += sq4(x[j][0]) + sq4(x[j][1]);
         rn = inv_rms(block_sum_d(ss, red), K, in.eps_n);
     }
-    // the GEMV's input, in place of x; a quad of threads holds one 32-element block (no is a multiple
-    // of 4: whole quads take part)
+    // the GEMM's input
     float v[NO][8];
     float m = 0.0f;
 #pragma unroll
@@ -262,246 +210,391 @@ __global__ __launch_bounds__(512) void batch_input_kernel(BatchIn in) {
     if constexpr (WIDE) {
         m = block_max_f(m, redf);
         e = m > 0.0f ? ilogbf(m) : 0;
+        float* inv = reinterpret_cast<float*>(in.img + (size_t)nb * WG * 2048);
         if (tid == 0) inv[t] = m > 0.0f ? ldexpf(1.0f, e - 14) : 0.0f;
     }
 #pragma unroll
     for (int j = 0; j < NO; ++j) {
         const uint32_t o = tid + 512 * j;
         if (o >= no) continue;
-        if constexpr (WIDE) wide_halves(v[j], 14 - e, o >> 2, o & 3, t, WG, reinterpret_cast<v4u*>(in.img));
-        else block_halves(v[j], o >> 2, o & 3, t, Tp, hi, lo, inv);
+        if constexpr (WIDE) {
+            wide_halves(v[j], 14 - e, o >> 2, o & 3, t, WG, reinterpret_cast<v4u*>(in.img));
+        } else {
+            v4f* y = reinterpret_cast<v4f*>(reinterpret_cast<float*>(in.img) + (size_t)t * K) + 8 * (o >> 2) + (o & 3);
+            y[0] = v4f{v[j][0], v[j][1], v[j][2], v[j][3]};
+            y[4] = v4f{v[j][4], v[j][5], v[j][6], v[j][7]};
+        }
     }
-}
-
-// BI_PLAIN inputs without a norm: one thread per 8-element octet, grid (Tp, octets / 256).  PS: the
-// input is gelu(gate) * up from a gate/up pair's deferred split-K partials.
-template <bool PS>
-__global__ __launch_bounds__(256) void batch_plain_input_kernel(BatchIn in) {
-    const uint32_t t = blockIdx.x, o = blockIdx.y * 256 + threadIdx.x, nb = in.K / 32, Tp = gridDim.x;
-    if (o >= nb * 4) return;  // whole quads: nb * 4 is a multiple of 4
-    const uint32_t i0 = 8 * (o >> 2) + (o & 3);  // the octet's float4: i0 and i0 + 4
-    _Float16* hi = reinterpret_cast<_Float16*>(in.img);
-    _Float16* lo = hi + (size_t)nb * Tp * 32;
-    float* inv = reinterpret_cast<float*>(lo + (size_t)nb * Tp * 32);
-    float v[8];
-    if (PS && t < in.T) {
-        // every plane's loads first, then each matrix's sums in split order, then gelu(gate) * up
-        const float* p0 = in.part + (size_t)t * in.part_row;
-        const size_t plane = (size_t)in.part_tp * in.part_row;
-        float4 pv[kDeferPairParts][2][2];
-#pragma unroll
-        for (int k = 0; k < (int)kDeferPairParts; ++k)
-            if ((uint32_t)k < in.parts)
-#pragma unroll
-                for (int q = 0; q < 2; ++q)
-#pragma unroll
-                    for (int h = 0; h < 2; ++h) pv[k][q][h] = reinterpret_cast<const float4*>(p0 + (2 * k + q) * plane)[i0 + 4 * h];
-        float s[2][8];
-#pragma unroll
-        for (int q = 0; q < 2; ++q)
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                s[q][4 * h] = pv[0][q][h].x;
-                s[q][4 * h + 1] = pv[0][q][h].y;
-                s[q][4 * h + 2] = pv[0][q][h].z;
-                s[q][4 * h + 3] = pv[0][q][h].w;
-            }
-#pragma unroll
-        for (int k = 1; k < (int)kDeferPairParts; ++k)
-            if ((uint32_t)k < in.parts)
-#pragma unroll
-                for (int q = 0; q < 2; ++q)
-#pragma unroll
-                    for (int h = 0; h < 2; ++h) {
-                        s[q][4 * h] += pv[k][q][h].x;
-                        s[q][4 * h + 1] += pv[k][q][h].y;
-                        s[q][4 * h + 2] += pv[k][q][h].z;
-                        s[q][4 * h + 3] += pv[k][q][h].w;
-                    }
-#pragma unroll
-        for (int i = 0; i < 8; ++i) v[i] = gelu_mul(s[0][i], s[1][i]);
-    } else if (t < in.T) {
-        const float4* x = reinterpret_cast<const float4*>(in.x + (size_t)t * in.stride);
-        const float4 u0 = x[i0], u1 = x[i0 + 4];
-        v[0] = u0.x; v[1] = u0.y; v[2] = u0.z; v[3] = u0.w;
-        v[4] = u1.x; v[5] = u1.y; v[6] = u1.z; v[7] = u1.w;
-    } else {
-#pragma unroll
-        for (int k = 0; k < 8; ++k) v[k] = 0.0f;
-    }
-    block_halves(v, o >> 2, o & 3, t, Tp, hi, lo, inv);
 }
 
 // ---- Q4_0 GEMM over a batch ---------------------------------------------------------------------
+//
+// Up to kBatchMax tokens: bound by the weight stream (66 MB of a gate/up pair in about 10 us), so that
+// everything else has to stay out of its way.  A workgroup of 16 waves takes 64 RW rows (RW waves
+// of four 16-row tiles) over one of S ranges of K, its KW = 16 / RW waves of the same rows dealing
+// the range's 4-block super-tiles among them:
+// - Each wave requests its first super-tiles' weights (one 16-byte load per lane and tile), then the
+//   workgroup turns its range of the fp32 inputs into fp16 halves in LDS (one or two waves a token),
+//   scaled by a power of two per token and range: no image is read or written in memory, and no
+//   launch makes one.
+// - The dwords of a lane's 16 code bytes (block lane / 16, row lane % 16) are exchanged between the
+//   four lanes of a row in registers (lane swaps), so that dword b holds the lane's k-slots of block
+//   b; nine operations then unpack eight weights (unpack_dword), and each product is folded with one
+//   FMA per token and row.
+// - Up to 8 tokens (PACK) the hi and lo halves are rows 0-7 and 8-15 of one MFMA operand, otherwise of two.
+// The waves' sums are added in LDS.  With S > 1 the ranges' sums go to planes in memory, and the last
+// workgroup of a row group to finish adds them (in split order) and writes y, unless the next kernel
+// does (defer) or the planes are many (kFuseSplits: batch_reduce_kernel).
+//
+// 3840 -> 15360, 32 tokens: 21.9 us against 34.3 us for the separate input-image, GEMM and reduce launches
+// this replaced (16 operations per eight weights, a per-block input scale, operands from L2 one block
+// ahead); 15360 -> 3840, 5 tokens: 15.0 against 26.2 us.
 
 namespace {
 
-// A block's input operands for a wave: the hi and lo halves of its G token groups (lane l: token
-// 16 g + l % 16, elements 8 (l / 16) .. + 7) and the block scales of tokens 16 g + 4 (l / 16) + e
-// (the lane's outputs).  They come from L2 (the image is shared by all
-// workgroups) and are loaded one block ahead.
-template <int G>
-struct InOps {
-    v4u hi[G], lo[G];
-    v4f sc[G];  // the block scales 2^(e - 14) of the four tokens whose outputs the lane folds
+constexpr int kThrough = 16;        // buffer access policy sc1: through to (or from) the memory side
+constexpr int kWaitVm0 = 0x0F70;    // s_waitcnt vmcnt(0), expcnt and lgkmcnt unconstrained
+constexpr uint32_t kGemmLds = 128 * 1024;   // the range's input halves at most
+// Ranges whose sums the last workgroup of a row group adds itself: with 32 tokens its 256 rows' planes are
+// 32 KB each, and one CU takes longer over more of them than another launch does.
+constexpr uint32_t kFuseSplits = 4;
+
+// Work split of a GEMM: workgroups of W waves take 64 RW rows (of both matrices together for a gate/up
+// pair, groups of them in all) over one of S ranges of K, so that about one workgroup per CU shares
+// the weight stream, a range's input halves fit LDS and each wave has a super-tile.
+// - Up to 8 tokens W 8, RW 1: the halves are cheap to make (8 KB per 1,024 columns), so a workgroup per 64 rows
+//   makes its own (16 waves, 15360 -> 3840, 5 tokens: 15.6 us against 14.9; 4096 -> 3840: 11.0 against 8.9).
+// - Above, W 16 and RW 2 or 4 (up to 16 tokens, or 32) share them among more rows, where the matrix has
+//   kGemmLarge units of 64 rows x 128 columns, one wave's share of a super-tile, or more; below, such
+//   workgroups would leave most CUs idle and their sums take longer to add: W 8, RW 1, and two groups
+//   of 16 tokens (tg) that read the weights twice rather than one of 32.  4096 -> 3840, 32 tokens: 12.7 us
+//   against 17.0 with W 16, RW 4; 1024 -> 1000, 30 tokens: 7.1 against 9.3 with one group of 32.
+struct GemmPlan {
+    uint32_t rw, waves, tg, groups, S;
 };
-
-// A block's weights for R row tiles of P matrices (lane l: row l % 16, bytes 8 ((l / 16) & 1) .. + 7 of
-// the block's 16 code bytes, and the row's fp16 scale).  They stream from HBM and are loaded
-// kCodeAhead blocks ahead.
-template <int P, int R>
-struct WOps {
-    uint2 code[R][P];
-    uint16_t d[R][P];
-};
-
-// weight blocks in flight per wave: 8, or 2 when a block spans 4 or more tiles
-template <int P, int R>
-constexpr int code_ahead() { return R * P >= 4 ? 2 : 8; }
-
-template <int G>
-__device__ __forceinline__ void load_in(InOps<G>& o, const BatchGemm& a, uint32_t b, uint32_t lane) {
-    constexpr uint32_t Tp = 16 * G;
-    const uint32_t m = lane & 15, kq = lane >> 4;
-    const _Float16* hi = reinterpret_cast<const _Float16*>(a.img);
-    const _Float16* lo = hi + (size_t)a.w.blocks * Tp * 32;
-    const float* inv = reinterpret_cast<const float*>(lo + (size_t)a.w.blocks * Tp * 32);
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-        const size_t at = ((size_t)b * Tp + 16 * g + m) * 32 + 8 * kq;
-        o.hi[g] = *gp(reinterpret_cast<const v4u*>(hi + at));
-        o.lo[g] = *gp(reinterpret_cast<const v4u*>(lo + at));
-        o.sc[g] = *gp(reinterpret_cast<const v4f*>(inv + (size_t)b * Tp + 16 * g + 4 * kq));
-    }
+constexpr uint32_t kGemmLarge = 3200;
+GemmPlan gemm_plan(uint32_t rows, uint32_t blocks, uint32_t T, bool pair) {
+    const uint32_t tiles = (rows + 15) / 16 * (pair ? 2 : 1), nst = (blocks + 3) / 4;
+    const bool large = T > 8 && (uint64_t)tiles * nst >= 4 * kGemmLarge;
+    const uint32_t rw = !large ? 1 : T <= 16 ? 2 : 4, waves = large ? 16 : 8, tg = !large && T > 16 ? 2 : 1;
+    const uint32_t groups = (tiles + 4 * rw - 1) / (4 * rw) * tg;
+    const uint32_t most = kGemmLds / (4096u * (T <= 8 ? 1 : T <= 16 || tg == 2 ? 2 : 4));  // super-tiles of a range
+    const uint32_t need = (nst + most - 1) / most, want = std::max(1u, std::min((256 + groups / 2) / groups, large ? nst / (waves / rw) : (nst + 7) / 8));
+    return GemmPlan{rw, waves, tg, groups, std::max(need, std::min(want, kDeferParts))};
 }
 
-template <int P, int R>
-__device__ __forceinline__ void load_w(WOps<P, R>& o, const BatchGemm& a, uint32_t b, uint32_t rt0, uint32_t last_tile,
-                                       uint32_t lane) {
-    const uint32_t m = lane & 15, kq = lane >> 4;
-    const uint32_t per_tile = a.w.nst * 4;  // block records per row tile (tiled layout, Q4View)
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-        const size_t rec = (size_t)min(rt0 + r, last_tile) * per_tile + b;
-#pragma unroll
-        for (int q = 0; q < P; ++q) {
-            const Q4View& w = q ? a.w2 : a.w;
-            o.code[r][q] = ld_stream(reinterpret_cast<const uint2*>(w.codes + rec * 256 + m * 16 + 8 * (kq & 1)));
-            o.d[r][q] = gp(w.scales)[rec * 16 + m];
-        }
-    }
-}
-
-// Four nibbles (one per byte of c) as fp16 (n - 8), in two pairs: n into the mantissa of 1024 + n
-// (0x6400 | n), then 1032 subtracted, exactly.
-__device__ __forceinline__ void nibbles_f16(uint32_t c, v2h& p0, v2h& p1) {
-    const v2h bias = {(_Float16)1032.0f, (_Float16)1032.0f};
-    p0 = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0u, c, 0x0c010c00u) | 0x64006400u) - bias;
-    p1 = __builtin_bit_cast(v2h, __builtin_amdgcn_perm(0u, c, 0x0c030c02u) | 0x64006400u) - bias;
-}
-
-template <int P, int G, int R>
-__device__ __forceinline__ void mfma_block(const InOps<G>& x, const WOps<P, R>& w, uint32_t kq,
-                                           float (&acc)[R][P][G][4]) {
-    const uint32_t sh = kq >= 2 ? 4u : 0u;  // k 0..15: low nibbles, 16..31: high nibbles
-    const v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-    for (int r = 0; r < R; ++r)
-#pragma unroll
-        for (int q = 0; q < P; ++q) {
-            v2h f0, f1, f2, f3;
-            nibbles_f16((w.code[r][q].x >> sh) & 0x0F0F0F0Fu, f0, f1);
-            nibbles_f16((w.code[r][q].y >> sh) & 0x0F0F0F0Fu, f2, f3);
-            const v8h B = {f0.x, f0.y, f1.x, f1.y, f2.x, f2.y, f3.x, f3.y};
-            const float d = h2f(w.d[r][q]);
-#pragma unroll
-            for (int g = 0; g < G; ++g) {
-                v4f D = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, x.hi[g]), B, zero, 0, 0, 0);
-                D = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, x.lo[g]), B, D, 0, 0, 0);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) acc[r][q][g][e] = fmaf(d * x.sc[g][e], D[e], acc[r][q][g][e]);
-            }
-        }
-}
-
-template <int P>
-__device__ __forceinline__ void gemm_epilogue(const BatchGemm& a, uint32_t t, uint32_t row, const float (&v)[P]) {
-    float* y = a.y + (size_t)t * a.y_stride + row;
-    if constexpr (P == 2) *y = gelu_mul(v[0], v[1]);
-    else if (a.add) *y = __fadd_rn(v[0], a.add[(size_t)t * a.y_stride + row]);
-    else *y = v[0];
-}
+// Super-tiles [s0, s1) of range k of S.
+__host__ __device__ inline uint32_t range_begin(uint32_t nst, uint32_t S, uint32_t k) { return (uint32_t)((uint64_t)nst * k / S); }
 
 }  // namespace
 
-// Grid (ceil(tiles / R), S): workgroup (x, s) takes row tiles R x .. R x + R - 1 (for a gate/up pair,
-// those tiles of both matrices) over K range s of S; its four waves split the range's blocks and add
-// their partials in LDS in wave order.  Each wave streams its blocks through a two-stage register
-// pipeline (the next block's loads in flight while the current block's MFMAs run).  With S = 1 the
-// workgroup writes y; otherwise it writes its partials for batch_reduce_kernel.
-template <int P, int G, int R>
-__global__ __launch_bounds__(256) void batch_gemm_kernel(BatchGemm a) {
-    constexpr uint32_t Tp = 16 * G;
-    __shared__ float red[4][R][P][Tp][16];
-    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = wave_id(), kq = lane >> 4;
-    const uint32_t tiles = (a.w.rows + 15) / 16, rt0 = blockIdx.x * R, S = gridDim.y, split = blockIdx.y;
-    const uint32_t nb = a.w.blocks;
-    const uint32_t s0 = nb * split / S, s1 = nb * (split + 1) / S;
-    const uint32_t b0 = s0 + (s1 - s0) * wave / 4, b1 = s0 + (s1 - s0) * (wave + 1) / 4;
-    float acc[R][P][G][4];
+// One lane's eight fp16 weights n - 8 of a block from the dword of its code bytes 4 q .. 4 q + 3: the
+// nibbles' bits in the mantissa of 1024 + n (or 1024 + 16 n), then 1032 subtracted (or scaled by 1/16
+// and 72 subtracted), exactly.  Weights 4 q + {0, 2}, 16 + 4 q + {0, 2}, 4 q + {1, 3}, 16 + 4 q + {1, 3}.
+__device__ __forceinline__ v4u unpack_dword(uint32_t c) {
+    const v2h bias = {(_Float16)1032.0f, (_Float16)1032.0f}, hb = {(_Float16)-72.0f, (_Float16)-72.0f},
+              sixteenth = {(_Float16)0.0625f, (_Float16)0.0625f};
+    // (the constants in registers, the mask's scalar: v_and_or_b32 takes no literals)
+    uint32_t low = 0x000F000Fu, high = 0x00F000F0u, magic = 0x64006400u;
+    asm("" : "+s"(low), "+s"(high), "+v"(magic));
+    const uint32_t c8 = c >> 8;
+    const v2h a = __builtin_bit_cast(v2h, (c & low) | magic) - bias;
+    const v2h b = __builtin_elementwise_fma(__builtin_bit_cast(v2h, (c & high) | magic), sixteenth, hb);
+    const v2h e = __builtin_bit_cast(v2h, (c8 & low) | magic) - bias;
+    const v2h f = __builtin_elementwise_fma(__builtin_bit_cast(v2h, (c8 & high) | magic), sixteenth, hb);
+    return v4u{__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), __builtin_bit_cast(uint32_t, e),
+               __builtin_bit_cast(uint32_t, f)};
+}
+
+// Lane group g (lanes 16 g .. + 15) holding dwords v[0..3] of its column: afterwards dword b of lane
+// group g is dword g of lane group b (the four lanes of a row transpose their 4 x 4 dwords).
+__device__ __forceinline__ v4u transpose_lanes(v4u v) {
+    const auto a = __builtin_amdgcn_permlane32_swap(v.x, v.z, false, false);  // groups 2, 3 of x with 0, 1 of z
+    const auto b = __builtin_amdgcn_permlane32_swap(v.y, v.w, false, false);
+    const auto c = __builtin_amdgcn_permlane16_swap(a[0], b[0], false, false);  // groups 1, 3 of one with 0, 2 of the other
+    const auto d = __builtin_amdgcn_permlane16_swap(a[1], b[1], false, false);
+    return v4u{c[0], c[1], d[0], d[1]};
+}
+// Lane group g's value g of its column, in every lane: o[b] is lane group b's v.
+__device__ __forceinline__ void spread_lanes(uint32_t v, uint32_t (&o)[4]) {
+    const auto h = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    const auto a = __builtin_amdgcn_permlane16_swap(h[0], h[0], false, false);
+    const auto b = __builtin_amdgcn_permlane16_swap(h[1], h[1], false, false);
+    o[0] = a[0];
+    o[1] = a[1];
+    o[2] = b[0];
+    o[3] = b[1];
+}
+
+template <int G, bool PACK, int P, int RW, int W>
+__global__ __launch_bounds__(64 * W) void batch_gemm_kernel(BatchGemm a, uint32_t S, uint32_t groups, uint32_t tgroups, uint32_t fuse) {
+    constexpr int KW = W / RW, kTokens = PACK ? 8 : 16 * G;
+    constexpr int NF = PACK ? 1 : 2 * G;        // 1 KB operands per block: [token group][hi, lo], or one packed
+    constexpr uint32_t TR = 16 * G;             // operand rows (tokens; PACK: hi, then lo of eight tokens)
+    constexpr uint32_t NR = 64 * RW;            // rows of the workgroup
+    static_assert(W <= kTokens, "a wave per token in the input stage, or several tokens");
+    constexpr int TW = kTokens / W;             // tokens per wave there
+    constexpr int NO = kGemmLds / (4096 * NF) / 4;  // octet rounds of 64 lanes per token
+    constexpr int kAhead = W == 16 ? 1 : 2;     // super-tiles requested ahead (16 waves have 128 registers each)
+    //                   // super-tiles requested ahead of the one being multiplied
+    extern __shared__ __align__(16) v4u smem[]; // input halves [block][NF][64 lanes], later sums [KW][TR][NR] f32
+    __shared__ float inv[32];                   // the tokens' scales 2^(e - 14)
+    __shared__ bool last;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = wave_id(), r = lane & 15, q = lane >> 4;
+    const uint32_t rw = wave % RW, kw = wave / RW;
+    // item (row group, split), split fastest, in contiguous shares per XCD (workgroup b runs on XCD
+    // b % 8): the splits of a row group mostly share an XCD
+    const uint32_t item = blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8;
+    if (item >= groups * S) return;
+    // (row group, token group): with two of the latter, tokens 16 tg .. + 15 are this workgroup's
+    const uint32_t gi = item / S, split = item % S, rg = gi / tgroups, tg = gi % tgroups;
+    const uint32_t Tp = (PACK ? 8 : TR) * tgroups;  // tokens per plane
+    if (tgroups > 1) {
+        a.x += (size_t)tg * TR * a.x_stride;
+        a.y += (size_t)tg * TR * a.y_stride;
+        a.T = min(a.T - tg * TR, TR);
+    }
+    const uint32_t nst = a.w.nst, nb = a.w.blocks, tiles = (a.w.rows + 15) / 16;
+    const uint32_t s0 = range_begin(nst, S, split), s1 = range_begin(nst, S, split + 1);
+
+    // ---- weights: the wave's row tiles 4 rw .. + 3 of the workgroup (a gate/up pair alternates the
+    // matrices), super-tiles s0 + kw, + KW, ...
+    // (through a buffer of no bytes past the range: the same two loads, without a memory access, so that
+    // every wait is an exact count)
+    const uint8_t* cp[4];
+    const uint16_t* dp[4];
 #pragma unroll
-    for (int r = 0; r < R; ++r)
+    for (int i = 0; i < 4; ++i) {
+        const uint32_t v = 4 * (rg * RW + rw) + i, tile = min(P == 2 ? v / 2 : v, tiles - 1);
+        const Q4View& w = P == 2 && (i & 1) ? a.w2 : a.w;
+        cp[i] = w.codes + (size_t)tile * nst * 1024;
+        dp[i] = w.scales + (size_t)tile * nst * 64;
+    }
+    v4u wc[kAhead][4];
+    uint32_t wd[kAhead][4];
+    auto request = [&](int u, uint32_t st) {
+        const bool in = st < s1;
+        const size_t at = in ? st : 0;
 #pragma unroll
-        for (int q = 0; q < P; ++q)
+        for (int i = 0; i < 4; ++i) {
+            const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(cp[i]) + at * 1024, 0, in ? 1024 : 0, 0x00020000);
+            const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(dp[i]) + at * 64, 0, in ? 128 : 0, 0x00020000);
+            wc[u][i] = __builtin_amdgcn_raw_buffer_load_b128(rc, lane * 16, 0, 2);
+            wd[u][i] = __builtin_amdgcn_raw_buffer_load_b16(rd, lane * 2, 0, 2);
+        }
+    };
+
+    // ---- inputs: token t = wave + 8 k, octet o = (block o / 4, part o % 4) of the range
+    const uint32_t no = (s1 - s0) * 16;  // octets of the range, those past the last block zero
+    v4f x[TW][NO][2];
 #pragma unroll
-            for (int g = 0; g < G; ++g)
+    for (int k = 0; k < TW; ++k) {
+        const uint32_t t = wave + W * k;
+        const float4* xp = reinterpret_cast<const float4*>(a.x + (size_t)min(t, a.T - 1) * a.x_stride);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) acc[r][q][g][e] = 0.0f;
-    // weights kCodeAhead blocks ahead in a register ring, inputs one block ahead (ping-pong)
-    constexpr int kCodeAhead = code_ahead<P, R>();
-    WOps<P, R> wr[kCodeAhead];
-    InOps<G> xi[2];
-    const uint32_t last_b = nb - 1;
-#pragma unroll
-    for (int u = 0; u < kCodeAhead; ++u) load_w(wr[u], a, min(b0 + u, last_b), rt0, tiles - 1, lane);
-    if (b0 < b1) load_in(xi[0], a, b0, lane);
-    for (uint32_t b = b0; b < b1; b += kCodeAhead) {
-#pragma unroll
-        for (int u = 0; u < kCodeAhead; ++u) {
-            const uint32_t bb = b + u;
-            if (bb >= b1) break;
-            if (bb + 1 < b1) load_in(xi[(u + 1) & 1], a, bb + 1, lane);
-            mfma_block(xi[u & 1], wr[u], kq, acc);
-            load_w(wr[u], a, min(bb + kCodeAhead, last_b), rt0, tiles - 1, lane);
+        for (int j = 0; j < NO; ++j) {
+            // (past the range too: a load under a branch would be waited for at the branch's end)
+            const uint32_t o = 64 * j + lane, b = min(s0 * 4 + (o >> 2), nb - 1), i0 = 8 * b + (o & 3);
+            x[k][j][0] = *gp(reinterpret_cast<const v4f*>(xp + i0));
+            x[k][j][1] = *gp(reinterpret_cast<const v4f*>(xp + i0 + 4));
         }
     }
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int r = 0; r < R; ++r)
+    for (int u = 0; u < kAhead; ++u) request(u, s0 + kw + KW * u);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-        for (int q = 0; q < P; ++q)
+    for (int k = 0; k < TW; ++k) {
+        const uint32_t t = wave + W * k;
+        if (t >= a.T) continue;  // (its operand rows are not stored)
+        float m = 0.0f;
 #pragma unroll
-            for (int g = 0; g < G; ++g)
+        for (int j = 0; j < NO; ++j) {
+            if ((uint32_t)(64 * j) >= no) break;
+            const uint32_t o = 64 * j + lane;
+            const bool in = o < no && s0 * 4 + (o >> 2) < nb;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) red[wave][r][q][16 * g + 4 * kq + e][lane & 15] = acc[r][q][g][e];
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    x[k][j][h][e] = in ? x[k][j][h][e] : 0.0f;
+                    m = fmaxf(m, fabsf(x[k][j][h][e]));
+                }
+        }
+        m = wave_max(m);
+        const int e = m > 0.0f ? ilogbf(m) : 0;
+        if (lane == 0) inv[t] = m > 0.0f ? ldexpf(1.0f, e - 14) : 0.0f;
+#pragma unroll
+        for (int j = 0; j < NO; ++j) {
+            const uint32_t o = 64 * j + lane;
+            if (o < no) {
+                // lane 16 p + row of the operand, its rows permuted by the block and part so that the
+                // stores of a token's octets spread over the banks
+                const uint32_t b = o >> 2, p = o & 3, s = (b & 3) * 4 + p;
+                float v[8];
+#pragma unroll
+                for (int h = 0; h < 8; ++h) v[h] = x[k][j][h / 4][h % 4];
+                v4u hi, lo;
+                octet_halves(v, 14 - e, hi, lo);
+                v4u* at = smem + (size_t)b * NF * 64 + 16 * p;
+                if constexpr (PACK) {
+                    at[t ^ s] = hi;
+                    at[(t + 8) ^ s] = lo;
+                } else {
+                    at[(t / 16) * 128 + (t % 16 ^ s)] = hi;
+                    at[(t / 16) * 128 + 64 + (t % 16 ^ s)] = lo;
+                }
+            }
+        }
+    }
     __syncthreads();
-    const size_t prow = (size_t)tiles * 16;
-    for (uint32_t i = tid; i < R * Tp * 16; i += kGemmThreads) {
-        const uint32_t r = i / (Tp * 16), t = (i / 16) % Tp, n = i & 15;
-        const uint32_t tile = rt0 + r, row = tile * 16 + n;
-        if (tile >= tiles || t >= a.T) continue;
-        float v[P];
+
+    // ---- products
+    float acc[4][G][4];
 #pragma unroll
-        for (int q = 0; q < P; ++q) v[q] = ((red[0][r][q][t][n] + red[1][r][q][t][n]) + red[2][r][q][t][n]) + red[3][r][q][t][n];
-        if (S > 1) {
+    for (int i = 0; i < 4; ++i)
 #pragma unroll
-            for (int q = 0; q < P; ++q) a.part[((size_t)(split * P + q) * Tp + t) * prow + row] = v[q];
-        } else if (row < a.w.rows) {
-            gemm_epilogue<P>(a, t, row, v);
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[i][g][e] = 0.0f;
+    const v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
+    for (uint32_t st0 = s0 + kw; st0 < s1; st0 += KW * kAhead) {
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            const uint32_t st = st0 + KW * u;
+            if (st >= s1) break;
+            v4u c[4];
+            uint32_t d[4][4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                c[i] = transpose_lanes(wc[u][i]);
+                spread_lanes(wd[u][i], d[i]);
+            }
+            request(u, st + KW * kAhead);
+#pragma unroll
+            for (int b = 0; b < 4; ++b) {
+                const v4u* at = smem + (size_t)((st - s0) * 4 + b) * NF * 64 + 16 * q + (r ^ (b * 4 + q));
+                v8h x16[NF];
+#pragma unroll
+                for (int f = 0; f < NF; ++f) x16[f] = __builtin_bit_cast(v8h, at[64 * f]);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const v8h w = __builtin_bit_cast(v8h, unpack_dword(c[i][b]));
+                    const float ds = h2f((uint16_t)d[i][b]);
+#pragma unroll
+                    for (int g = 0; g < G; ++g) {
+                        v4f D = __builtin_amdgcn_mfma_f32_16x16x32_f16(x16[PACK ? 0 : 2 * g], w, zero, 0, 0, 0);
+                        if constexpr (!PACK) D = __builtin_amdgcn_mfma_f32_16x16x32_f16(x16[2 * g + 1], w, D, 0, 0, 0);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) acc[i][g][e] = fmaf(ds, D[e], acc[i][g][e]);
+                    }
+                }
+            }
+        }
+    }
+    __syncthreads();  // every wave has read its operands
+
+    // ---- the waves' sums: [kw][operand row][row]
+    float* red = reinterpret_cast<float*>(smem);
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+                red[(kw * TR + 16 * g + 4 * q + e) * NR + 64 * rw + 16 * i + r] = acc[i][g][e];
+    __syncthreads();
+    // thread: row n of the workgroup (P == 2: the gate's row, tiles 2 j and 2 j + 1 paired), tokens t0, + TS, ...
+    constexpr uint32_t NY = NR / P, TS = 64 * W / NY, NT = kTokens / TS > 0 ? kTokens / TS : 1;
+    const uint32_t n = tid % NY, t0 = tid / NY;
+    const uint32_t row = rg * NY + n, prow = tiles * 16;
+    const uint32_t col = P == 2 ? n / 16 * 32 + n % 16 : n;
+    float v[NT][P];
+#pragma unroll
+    for (uint32_t j = 0; j < NT; ++j) {
+        const uint32_t t = t0 + TS * j;
+#pragma unroll
+        for (int p = 0; p < P; ++p) {
+            float s = 0.0f;
+            if (t < a.T) {
+#pragma unroll
+                for (int k = 0; k < KW; ++k) {
+                    const float* at = red + (size_t)k * TR * NR + t * NR + col + 16 * p;
+                    const float u = PACK ? at[0] + at[8 * NR] : at[0];
+                    s = k ? s + u : u;
+                }
+                s *= inv[t];
+            }
+            v[j][p] = s;
+        }
+    }
+    auto put = [&](uint32_t t, const float (&s)[P]) {
+        float* y = a.y + (size_t)t * a.y_stride + row;
+        if constexpr (P == 2) *y = gelu_mul(s[0], s[1]);
+        else *y = s[0];
+    };
+    if (S == 1) {
+#pragma unroll
+        for (uint32_t j = 0; j < NT; ++j)
+            if (t0 + TS * j < a.T && row < a.w.rows) put(t0 + TS * j, v[j]);
+        return;
+    }
+    // planes [split][P][Tp][prow]
+    auto plane = [&](uint32_t k, int p, uint32_t t) { return ((size_t)(k * P + p) * Tp + tg * TR + t) * prow + row; };
+    const __amdgpu_buffer_rsrc_t prs = __builtin_amdgcn_make_buffer_rsrc(a.part, 0, 0x7FFFFFFF, 0x00020000);
+#pragma unroll
+    for (uint32_t j = 0; j < NT; ++j) {
+        const uint32_t t = t0 + TS * j;
+        if (t < a.T && row < prow)
+#pragma unroll
+            for (int p = 0; p < P; ++p) {
+                if (fuse) __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v[j][p]), prs, (uint32_t)plane(split, p, t) * 4, 0, kThrough);
+                else a.part[plane(split, p, t)] = v[j][p];
+            }
+    }
+    if (!fuse) return;
+    // the last workgroup of the row group adds the planes: stored through to the memory side and
+    // waited for before the ticket, read from there (the XCDs' L2s are not coherent with each other)
+    __builtin_amdgcn_s_waitcnt(kWaitVm0);
+    __syncthreads();
+    if (tid == 0) {
+        const uint32_t ticket = __hip_atomic_fetch_add(a.counters + gi, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        last = ticket == S - 1;
+        if (last) __hip_atomic_store(a.counters + gi, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __syncthreads();
+    if (!last) return;
+    // every load of a few tokens at once, unconditional (past the planes or rows: out of the buffer, zeros)
+    constexpr uint32_t FS = G == 2 ? kFuseSplits : kDeferParts, JB = NT < 4 ? NT : 4;
+#pragma unroll
+    for (uint32_t j0 = 0; j0 < NT; j0 += JB) {
+        float u[JB][P][FS];
+#pragma unroll
+        for (uint32_t j = 0; j < JB; ++j)
+#pragma unroll
+            for (int p = 0; p < P; ++p)
+#pragma unroll
+                for (uint32_t k = 0; k < FS; ++k) {
+                    const uint32_t t = t0 + TS * (j0 + j);
+                    const uint32_t off = k < S && t < a.T && row < prow ? (uint32_t)plane(k, p, t) * 4 : 0x80000000u;
+                    u[j][p][k] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(prs, off, 0, kThrough));
+                }
+#pragma unroll
+        for (uint32_t j = 0; j < JB; ++j) {
+            const uint32_t t = t0 + TS * (j0 + j);
+            float s[P];
+#pragma unroll
+            for (int p = 0; p < P; ++p) {
+                s[p] = u[j][p][0];
+#pragma unroll
+                for (uint32_t k = 1; k < FS; ++k) s[p] += u[j][p][k];
+            }
+            if (t < a.T && row < a.w.rows) put(t, s);
         }
     }
 }
 
-// y from the S split-K partials of batch_gemm_kernel, summed in split order; one thread per (t, row).
+// y from S split-K partial planes, summed in split order; one thread per (t, row).
 template <int P>
 __global__ __launch_bounds__(256) void batch_reduce_kernel(BatchGemm a, uint32_t S, uint32_t Tp) {
     const uint32_t rows = a.w.rows, i = blockIdx.x * 256 + threadIdx.x;
@@ -515,7 +608,9 @@ __global__ __launch_bounds__(256) void batch_reduce_kernel(BatchGemm a, uint32_t
         for (uint32_t k = 1; k < S; ++k) s += a.part[((size_t)(k * P + q) * Tp + t) * prow + row];
         v[q] = s;
     }
-    gemm_epilogue<P>(a, t, row, v);
+    float* y = a.y + (size_t)t * a.y_stride + row;
+    if constexpr (P == 2) *y = gelu_mul(v[0], v[1]);
+    else *y = v[0];
 }
 
 // ---- Q4_0 GEMM over a wide pass -------------------------------------------------------------------
@@ -535,21 +630,6 @@ __global__ __launch_bounds__(256) void batch_reduce_kernel(BatchGemm a, uint32_t
 // shares (workgroup b runs on XCD b % 8), so that the workgroups that unpack the same weights share
 // an L2.
 constexpr uint32_t kWideChain = 8;
-
-// One lane's eight fp16 weights n - 8 of a block from the dword of its code bytes 4 q .. 4 q + 3: the
-// nibbles' bits in the mantissa of 1024 + n (or 1024 + 16 n), then 1032 subtracted (or scaled by 1/16
-// and 72 subtracted), exactly.  Weights 4 q + {0, 2}, 16 + 4 q + {0, 2}, 4 q + {1, 3}, 16 + 4 q + {1, 3}.
-__device__ __forceinline__ v4u unpack_dword(uint32_t c) {
-    const v2h bias = {(_Float16)1032.0f, (_Float16)1032.0f}, hb = {(_Float16)-72.0f, (_Float16)-72.0f},
-              sixteenth = {(_Float16)0.0625f, (_Float16)0.0625f};
-    const uint32_t c8 = c >> 8;
-    const v2h a = __builtin_bit_cast(v2h, (c & 0x000F000Fu) | 0x64006400u) - bias;
-    const v2h b = __builtin_elementwise_fma(__builtin_bit_cast(v2h, (c & 0x00F000F0u) | 0x64006400u), sixteenth, hb);
-    const v2h e = __builtin_bit_cast(v2h, (c8 & 0x000F000Fu) | 0x64006400u) - bias;
-    const v2h f = __builtin_elementwise_fma(__builtin_bit_cast(v2h, (c8 & 0x00F000F0u) | 0x64006400u), sixteenth, hb);
-    return v4u{__builtin_bit_cast(uint32_t, a), __builtin_bit_cast(uint32_t, b), __builtin_bit_cast(uint32_t, e),
-               __builtin_bit_cast(uint32_t, f)};
-}
 
 template <int WM, int P>
 __global__ __launch_bounds__(256, 2) void wide_gemm_kernel(BatchGemm a, uint32_t S, uint32_t mtiles, uint32_t ngroups) {
@@ -618,7 +698,10 @@ __global__ __launch_bounds__(256, 2) void wide_gemm_kernel(BatchGemm a, uint32_t
         const int buf = (b - b0) & 1;
         float d[4];
 #pragma unroll
-        for (int n = 0; n < 4; ++n) d[n] = h2f(dn[n]);
+        for (int n = 0; n < 4; ++n) {
+            d[n] = h2f(dn[n]);
+            asm("" : "+v"(d[n]));  // (converted once: as a mixed-precision operand of 64 FMAs it takes 1.5 % longer)
+        }
         v8h ah[4], al[4], bw[4];
 #pragma unroll
         for (int m = 0; m < 4; ++m) {
@@ -1154,22 +1237,26 @@ static uint32_t wide_splits(uint32_t rows, uint32_t blocks, uint32_t tokens, boo
 }
 
 size_t batch_image_bytes(uint32_t blocks, uint32_t tokens) {
-    if (tokens > kBatchMax)  // (every narrower pass's image fits too)
-        return std::max(batch_image_bytes(blocks, kBatchMax),
-                        ((size_t)blocks * 2048 + 64) * ((tokens + 127) / 128 * 8));
-    return (size_t)blocks * padded_tokens(tokens) * (128 + 4);
+    const size_t floats = (size_t)blocks * 128 * std::min(tokens, kBatchMax);
+    return tokens > kBatchMax ? std::max(floats, ((size_t)blocks * 2048 + 64) * ((tokens + 127) / 128 * 8)) : floats;
 }
 
 size_t batch_gemm_part_bytes(uint32_t rows, uint32_t blocks, uint32_t tokens, bool gelu_pair) {
-    size_t wide = 0;  // the largest over the wide passes up to `tokens`
-    for (uint32_t t = 64; t < tokens + 64; t += 64) {
-        const uint32_t T = std::min(t, tokens), S = T > kBatchMax ? wide_splits(rows, blocks, T, gelu_pair) : 1;
-        if (S > 1) wide = std::max(wide, (size_t)S * 16 * wide_groups(T) * ((rows + 15) / 16 * 16) * 4);
+    size_t most = 0;  // the largest over the passes of up to `tokens` tokens
+    const size_t prow = (rows + 15) / 16 * 16;
+    for (uint32_t t : {8u, 16u, 32u}) {
+        const uint32_t T = std::min(t, tokens), S = gemm_plan(rows, blocks, T, gelu_pair).S;
+        if (S > 1) most = std::max(most, (size_t)S * (gelu_pair ? 2 : 1) * padded_tokens(T) * prow * 4);
     }
-    if (tokens > kBatchMax) return std::max(wide, batch_gemm_part_bytes(rows, blocks, kBatchMax, gelu_pair));
-    const GemmPlan p = gemm_plan(rows, blocks, gelu_pair);
-    if (p.S == 1) return 0;
-    return (size_t)p.S * (gelu_pair ? 2 : 1) * padded_tokens(tokens) * ((rows + 15) / 16 * 16) * 4;
+    for (uint32_t t = 64; t < tokens + 64 && tokens > kBatchMax; t += 64) {
+        const uint32_t T = std::min(t, tokens), S = wide_splits(rows, blocks, T, gelu_pair);
+        if (S > 1) most = std::max(most, (size_t)S * 16 * wide_groups(T) * prow * 4);
+    }
+    return most;
+}
+
+size_t batch_gemm_counters(uint32_t rows, bool gelu_pair) {
+    return 2 * gemm_plan(rows, 1, 1, gelu_pair).groups;  // (the fewest rows per group, two token groups)
 }
 
 // The wide GEMM's input image: one workgroup per token, in every mode.
@@ -1198,25 +1285,14 @@ static hipError_t launch_wide_input(const BatchIn& in, hipStream_t s) {
 hipError_t launch_batch_input(const BatchIn& in, hipStream_t s) {
     if (in.T == 0 || in.T > kPassMax || in.K == 0 || in.K > 16384 || in.K % 32) return hipErrorInvalidValue;
     if (in.T > kBatchMax) return launch_wide_input(in, s);
-    if (in.mode == BI_PLAIN && !in.w_n) {
-        if (in.stride % 4 || reinterpret_cast<uintptr_t>(in.x) % 16) return hipErrorInvalidValue;
-        const uint32_t octets = in.K / 8;
-        const dim3 g(padded_tokens(in.T), (octets + 255) / 256);
-        if (in.parts) {
-            if (in.parts > kDeferPairParts || reinterpret_cast<uintptr_t>(in.part) % 16 || in.part_row % 4 ||
-                in.part_row < in.K)
-                return hipErrorInvalidValue;
-            hipLaunchKernelGGL(batch_plain_input_kernel<true>, g, dim3(256), 0, s, in);
-        } else {
-            hipLaunchKernelGGL(batch_plain_input_kernel<false>, g, dim3(256), 0, s, in);
-        }
-    } else {
+    if (in.mode == BI_PLAIN) return hipErrorInvalidValue;  // (the GEMM reads x itself)
+    {
         // float4 access to x, res, x_out and the norm weights
         const auto a16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
         if (in.stride % 4 || !a16(in.x) || !a16(in.res) || !a16(in.x_out) || !a16(in.w_a) || !a16(in.w_n))
             return hipErrorInvalidValue;
         const uint32_t octets = in.K / 8;
-        const dim3 g(padded_tokens(in.T));
+        const dim3 g(in.T);
         const size_t lds = in.mode == BI_EMBED ? (size_t)in.K * 4 : 0;
         if (in.parts) {
             if (in.mode != BI_RESID || octets > 512 || in.parts > kDeferParts || !a16(in.part) || in.part_row % 4 ||
@@ -1234,28 +1310,34 @@ hipError_t launch_batch_input(const BatchIn& in, hipStream_t s) {
     return hipGetLastError();
 }
 
-template <int P, int G>
+template <int P, int G, bool PACK>
 static hipError_t gemm_launch(const BatchGemm& a, hipStream_t s, uint32_t* parts) {
-    const GemmPlan p = gemm_plan(a.w.rows, a.w.blocks, P == 2);
-    const uint32_t tiles = (a.w.rows + 15) / 16;
-    const dim3 grid((tiles + p.R - 1) / p.R, p.S);
+    const GemmPlan p = gemm_plan(a.w.rows, a.w.blocks, a.T, P == 2);
+    constexpr uint32_t TR = 16 * G;
+    const uint32_t Tp = (PACK ? 8 : TR) * p.tg;
+    const bool defer = a.defer && P == 1 && p.S > 1;
+    const uint64_t planes = (uint64_t)p.S * P * Tp * ((a.w.rows + 15) / 16 * 16) * 4;
+    const bool fuse = p.S > 1 && !defer && a.counters && p.S <= (G == 2 ? kFuseSplits : kDeferParts) && planes < 0x7FFFFFFFu;
     if (p.S > 1 && !a.part) return hipErrorInvalidValue;
-    switch (p.R) {
-        case 1: hipLaunchKernelGGL((batch_gemm_kernel<P, G, 1>), grid, dim3(kGemmThreads), 0, s, a); break;
-        case 2: hipLaunchKernelGGL((batch_gemm_kernel<P, G, 2>), grid, dim3(kGemmThreads), 0, s, a); break;
-        case 4: hipLaunchKernelGGL((batch_gemm_kernel<P, G, 4>), grid, dim3(kGemmThreads), 0, s, a); break;
-        default:
-            if constexpr (P == 1) hipLaunchKernelGGL((batch_gemm_kernel<P, G, 8>), grid, dim3(kGemmThreads), 0, s, a);
-            break;
+    const uint32_t range = (a.w.nst + p.S - 1) / p.S;  // super-tiles, at most
+    const size_t lds = std::max<size_t>((size_t)range * 4096 * (PACK ? 1 : 2 * G), 256 * p.waves * TR);  // (operands, later the waves' sums)
+    const dim3 grid((p.groups * p.S + 7) / 8 * 8);
+    if constexpr (G == 1) {
+        if (p.waves == 8)
+            hipLaunchKernelGGL((batch_gemm_kernel<1, PACK, P, 1, 8>), grid, dim3(512), lds, s, a, p.S, p.groups, p.tg, fuse ? 1u : 0u);
+    }
+    if constexpr (!PACK) {
+        if (p.waves == 16)
+            hipLaunchKernelGGL((batch_gemm_kernel<G, false, P, 2 * G, 16>), grid, dim3(1024), lds, s, a, p.S, p.groups, p.tg, fuse ? 1u : 0u);
     }
     hipError_t e = hipGetLastError();
-    if (e != hipSuccess || p.S == 1) return e;
-    if (a.defer && !a.add && p.S <= (P == 2 ? kDeferPairParts : kDeferParts)) {
+    if (e != hipSuccess || p.S == 1 || fuse) return e;
+    if (defer) {
         if (parts) *parts = p.S;
         return hipSuccess;
     }
     const uint32_t n = a.T * a.w.rows;
-    hipLaunchKernelGGL((batch_reduce_kernel<P>), dim3((n + 255) / 256), dim3(256), 0, s, a, p.S, 16u * G);
+    hipLaunchKernelGGL((batch_reduce_kernel<P>), dim3((n + 255) / 256), dim3(256), 0, s, a, p.S, Tp);
     return hipGetLastError();
 }
 
@@ -1264,7 +1346,7 @@ static hipError_t wide_launch(const BatchGemm& a, hipStream_t s, uint32_t* parts
     const uint32_t m = wide_tokens(a.T), rows_wg = 16384 / m / P;  // (rows of each matrix)
     const uint32_t mtiles = (a.T + m - 1) / m, ngroups = (a.w.rows + rows_wg - 1) / rows_wg;
     const uint32_t S = wide_splits(a.w.rows, a.w.blocks, a.T, P == 2);
-    if (a.add || (S > 1 && !a.part)) return hipErrorInvalidValue;
+    if (S > 1 && !a.part) return hipErrorInvalidValue;
     const dim3 grid((mtiles * ngroups * S + 7) / 8 * 8);
     if (m == 128) hipLaunchKernelGGL((wide_gemm_kernel<2, P>), grid, dim3(256), 0, s, a, S, mtiles, ngroups);
     else hipLaunchKernelGGL((wide_gemm_kernel<1, P>), grid, dim3(256), 0, s, a, S, mtiles, ngroups);
@@ -1286,9 +1368,12 @@ hipError_t launch_batch_gemm(const BatchGemm& a, bool gelu_pair, hipStream_t s, 
         return gelu_pair ? wide_launch<2>(a, s, parts) : wide_launch<1>(a, s, parts);
     if (a.T == 0 || a.T > kBatchMax || a.w.rows == 0 || a.w.blocks == 0) return hipErrorInvalidValue;
     if (gelu_pair && (a.w2.rows != a.w.rows || a.w2.blocks != a.w.blocks)) return hipErrorInvalidValue;
-    const bool two = a.T > 16;
-    if (gelu_pair) return two ? gemm_launch<2, 2>(a, s, parts) : gemm_launch<2, 1>(a, s, parts);
-    return two ? gemm_launch<1, 2>(a, s, parts) : gemm_launch<1, 1>(a, s, parts);
+    // float4 loads of the inputs
+    if (!a.x || a.x_stride % 4 || reinterpret_cast<uintptr_t>(a.x) % 16) return hipErrorInvalidValue;
+    if (a.T <= 8) return gelu_pair ? gemm_launch<2, 1, true>(a, s, parts) : gemm_launch<1, 1, true>(a, s, parts);
+    if (a.T <= 16 || gemm_plan(a.w.rows, a.w.blocks, a.T, gelu_pair).tg == 2)
+        return gelu_pair ? gemm_launch<2, 1, false>(a, s, parts) : gemm_launch<1, 1, false>(a, s, parts);
+    return gelu_pair ? gemm_launch<2, 2, false>(a, s, parts) : gemm_launch<1, 2, false>(a, s, parts);
 }
 
 }  // namespace af

@@ -1,0 +1,72 @@
+"""The forms of the batched Q4_0 GEMV (af_q4_gemm): packed halves up to 8 tokens, one or two token groups,
+8- or 16-wave workgroups, K in one range, in ranges the last workgroup adds and in ranges a reduce launch
+adds, at the edges of row tiles, super-tiles and token groups."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import oracle
+from adaforge_amd import _native as N, hip, synth
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("columns,rows,tokens", [
+    (32, 1, 1), (128, 64, 8), (160, 65, 8),        # packed: one block, whole tiles, one past each
+    (4128, 63, 8), (16384, 130, 2),                # packed: several ranges of K, added by the last workgroup
+    (32, 16, 9), (2080, 1000, 16), (16384, 70, 9), # one group of 16 tokens
+    (32, 17, 17), (1056, 999, 17), (4096, 3840, 32),  # two groups
+    (3840, 15360, 16), (15360, 3856, 13),          # 16 waves, 2 row waves
+    (3840, 15361, 17), (3872, 15360, 32),          # 16 waves, 4 row waves, the last workgroup adds
+    (15360, 3844, 31),                             # and with a reduce launch
+])
+def test_forms_match_oracle(columns, rows, tokens):
+    w = synth.q4(f"forms{columns}x{rows}", columns, rows, signed=True)
+    rng = np.random.default_rng(columns * 7 + rows + tokens)
+    xs = rng.standard_normal((tokens, columns)).astype(np.float32)
+    xs[tokens // 2] *= np.float32(2.0 ** 40)  # scales are per token
+    h = N.P()
+    N.check(N.lib().af_q4_upload(w.ctypes.data_as(N.u8p), w.size, columns, rows, ctypes.byref(h)))
+    try:
+        xb, yb = hip.Buffer.from_numpy(xs), hip.Buffer(tokens * rows)
+        got = []
+        for _ in range(3):  # the tickets start every call at zero
+            yb.upload(np.full(tokens * rows, np.nan, np.float32))
+            N.check(N.lib().af_q4_gemm(h, xb.ptr, tokens, yb.ptr, None))
+            hip.synchronize()
+            got.append(yb.numpy().reshape(tokens, rows))
+    finally:
+        N.lib().af_q4_free(h)
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])
+    for t in {0, tokens // 2, tokens - 1}:
+        ref = oracle.q4_matvec(w, columns, rows, xs[t])
+        # inputs to 22 bits and fp32 sums in any order: the 2-norm of the error is far below 2^-20 of
+        # the 2-norm of the products it sums
+        scale = np.sqrt(columns) * np.abs(xs[t]).max() * 0.02 * 8
+        assert np.abs(got[0][t] - ref).max() <= 2.0 ** -20 * scale
+        if t != tokens // 2:
+            oracle.compare(ref, got[0][t])
+
+
+def test_non_finite_inputs_stay_in_their_token():
+    """An infinity or NaN makes its own token's outputs non-finite and no other's."""
+    columns, rows = 256, 48
+    w = synth.q4("forms-nan", columns, rows, signed=True)
+    h = N.P()
+    N.check(N.lib().af_q4_upload(w.ctypes.data_as(N.u8p), w.size, columns, rows, ctypes.byref(h)))
+    try:
+        for tokens in (5, 12, 30):
+            xs = np.random.default_rng(tokens).standard_normal((tokens, columns)).astype(np.float32)
+            xs[1, 7], xs[3, 200] = np.inf, np.nan
+            xb, yb = hip.Buffer.from_numpy(xs), hip.Buffer(tokens * rows)
+            N.check(N.lib().af_q4_gemm(h, xb.ptr, tokens, yb.ptr, None))
+            hip.synchronize()
+            y = yb.numpy().reshape(tokens, rows)
+            for t in range(tokens):
+                if t in (1, 3):
+                    assert not np.isfinite(y[t]).any()
+                else:
+                    oracle.compare(oracle.q4_matvec(w, columns, rows, xs[t]), y[t])
+    finally:
+        N.lib().af_q4_free(h)
