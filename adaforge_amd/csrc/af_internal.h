@@ -289,6 +289,14 @@ hipError_t launch_head_batch(const HeadArgs& a, uint32_t nv, uint32_t vstride, u
 hipError_t launch_attention(const AttnArgs& a, uint32_t group, uint32_t head_width, hipStream_t s,
                             uint32_t tokens = 1);
 uint32_t attention_block_heads(uint32_t group, uint32_t head_width);
+// Decode attention of 512-wide heads on the matrix cores (attention_mfma_kernel), with kAttnMfmaGroup or more
+// query heads per KV head and more than kAttnMfmaSpan visible positions: its two launches take 15-17 us up to
+// 4,096 positions, attention_kernel 9-15 us up to 1,024 and 20-24 from 1,100 on (4 to 16 query heads).
+// a.cmax from attention_mfma_chunks, a.part of kv_heads cmax group rows (attn_part_row).
+constexpr uint32_t kAttnMfmaGroup = 4, kAttnMfmaSpan = 1024, kAttnMfmaChunks = 256;
+bool attention_mfma(uint32_t group, uint32_t head_width, uint32_t span);
+uint32_t attention_mfma_chunks(uint32_t kv_heads, uint32_t span);
+hipError_t launch_attention_mfma(const AttnArgs& a, uint32_t group, hipStream_t s);
 hipError_t launch_rmsnorm(const float* x, const float* w, float* y, uint32_t width, uint32_t vectors, float eps,
                           hipStream_t s);
 hipError_t launch_resid(const InputStage& in, uint32_t width, float* y, hipStream_t s);

@@ -791,7 +791,8 @@ int af_attention_decode(const af_attention_args* p, void* stream) {
     if ((rc = ensure_device())) return rc;
     const uint32_t group = p->config.q_heads / p->config.kv_heads, D = p->config.width;
     if (nvis > kAttnMaxChunks * kAttnMaxChunkLen) return fail(AF_ERR_INVALID, "visible range above 131072 tokens");
-    const uint32_t cmax = kAttnMaxChunks;
+    const bool mfma = attention_mfma(group, D, nvis);
+    const uint32_t cmax = mfma ? attention_mfma_chunks(p->config.kv_heads, nvis) : kAttnMaxChunks;
     const bool xl = attn_xcd_local();
     std::lock_guard<std::mutex> lock(g_scratch.mu);
     if ((rc = grow(g_scratch.attn_part, (size_t)p->config.kv_heads * cmax * group * attn_part_row(D) * 4, false, "attention scratch")))
@@ -829,12 +830,14 @@ int af_attention_decode(const af_attention_args* p, void* stream) {
     a.out = p->out;
     a.part = g_scratch.attn_part.as<float>();
     a.counters = g_scratch.attn_counters.as<uint32_t>();
-    a.cmax = attn_chunks(nvis, cmax, kAttnMinChunk);  // the position is known: a block per chunk
+    a.cmax = mfma ? cmax : attn_chunks(nvis, cmax, kAttnMinChunk);  // the position is known: a block per chunk
     a.min_chunk = kAttnMinChunk;
     a.kv_heads = p->config.kv_heads;
     a.group = group;
     a.xcd_local = xl ? 1u : 0u;
-    HIP_OK(launch_attention(a, group, D, (hipStream_t)stream), "attention launch");
+    HIP_OK(mfma ? launch_attention_mfma(a, group, (hipStream_t)stream)
+                : launch_attention(a, group, D, (hipStream_t)stream),
+           "attention launch");
     return AF_OK;
 }
 
@@ -850,6 +853,7 @@ struct LayerDev {
     float input_eps = 0, q_eps = 0, k_eps = 0, post_attn_eps = 0, ffn_eps = 0, post_ffn_eps = 0;
     float layer_scale = 1, scale = 1;
     uint32_t q_heads = 0, kv_heads = 0, width = 0, window = 0, ring = 0, qn = 0, kn = 0;
+    uint32_t mfma_chunks = 0;  // most chunks of attention_mfma_kernel (0: it never runs)
     bool shared_v = false, v_norm = false;
 };
 
@@ -1004,7 +1008,7 @@ struct af_session {
         return e;
     }
     static double q4_bytes(const Q4Dev& m) { return (double)m.rows * (m.columns / 32) * 18.0; }
-    uint32_t host_pos = 0;  // position being consumed (profiling: attention bytes)
+    uint32_t host_pos = 0;  // position being queued, as far as the host knows (attention kernel choice, profiling)
 
     ~af_session() {
         if (stream) (void)hipStreamSynchronize(stream);
@@ -1079,8 +1083,14 @@ struct af_session {
         aa.xcd_local = attn_xl ? 1u : 0u;
         const double nvis = L.window ? std::min<double>(host_pos + 1, L.window) : host_pos + 1.0;
         const double attn_bytes = nvis * 2.0 * L.kn * 2.0 + 4.0 * (2.0 * L.qn + 2.0 * L.kn) + 4.0 * L.kn;
-        if ((e = timed(K_ATTN, attn_bytes, [&] { return launch_attention(aa, L.q_heads / L.kv_heads, L.width, stream); })) !=
-            hipSuccess)
+        // by the position the host last set or queued (either kernel is right at any position; a captured
+        // step keeps attention_kernel)
+        const bool mfma = L.mfma_chunks && attention_mfma(aa.group, L.width, (uint32_t)nvis);
+        if (mfma) aa.cmax = L.mfma_chunks;
+        if ((e = timed(K_ATTN, attn_bytes, [&] {
+                 return mfma ? launch_attention_mfma(aa, aa.group, stream)
+                             : launch_attention(aa, aa.group, L.width, stream);
+             })) != hipSuccess)
             return e;
 
         Q4Args oa{};
@@ -1270,6 +1280,7 @@ struct af_session {
     // The staging words are only rewritten after the stream has drained (every caller
     // synchronises before returning), so the async copy never reads a changed value.
     int set_state(uint32_t pos, uint32_t nstop) {
+        host_pos = pos;
         state_host[ST_POS] = pos;
         state_host[ST_BAD] = 0u;
         state_host[ST_STOP] = 0u;
@@ -1762,6 +1773,7 @@ int open_session(const af_layer_weights* layers, uint32_t n_layers, const af_out
     HIP_OK(hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking), "session stream");
 
     uint32_t max_kv = 0, max_q = 0, max_group = 1, max_qh_part = 0, max_qh = 0;
+    size_t max_part = 0;  // floats of attention_mfma_kernel's chunk partials
     s->layers.resize(n_layers);
     for (uint32_t i = 0; i < n_layers; ++i) {
         const af_layer_weights& w = layers[i];
@@ -1806,6 +1818,10 @@ int open_session(const af_layer_weights* layers, uint32_t n_layers, const af_out
         if ((rc = dev_alloc(L.vcache, kv, "V cache"))) return rc;
         HIP_OK(hipMemset(L.kcache.p, 0, kv), "K cache clear");
         HIP_OK(hipMemset(L.vcache.p, 0, kv), "V cache clear");
+        const uint32_t span = L.window ? std::min(L.window, capacity) : capacity;
+        if (attention_mfma(L.q_heads / L.kv_heads, L.width, span))
+            L.mfma_chunks = attention_mfma_chunks(L.kv_heads, span);
+        max_part = std::max(max_part, (size_t)L.mfma_chunks * L.q_heads * attn_part_row(L.width));
         max_kv = std::max(max_kv, L.kv_heads);
         max_q = std::max(max_q, L.qn);
         max_group = std::max(max_group, L.q_heads / L.kv_heads);
@@ -1840,7 +1856,7 @@ int open_session(const af_layer_weights* layers, uint32_t n_layers, const af_out
         {&s->PROJT, (size_t)hidden * 8, true},
         {&s->DT, (size_t)hidden * 8, true},
         {&s->LOGITS, (size_t)hm.rows * 4, false},
-        {&s->PART, (size_t)s->cmax * std::max<uint32_t>(max_qh_part, max_kv * step_part_stride(max_group)) * 4, false},
+        {&s->PART, std::max((size_t)s->cmax * std::max<uint32_t>(max_qh_part, max_kv * step_part_stride(max_group)), max_part) * 4, false},
         {&s->COUNTERS, (size_t)std::max<uint32_t>(max_qh, 64) * 4, true},
         {&s->HPART, (size_t)s->head_blocks * 16 * kHeadBatchMax, false},  // (the verification head's per vector)
         {&s->HCOUNT, 256, true},

@@ -1387,6 +1387,321 @@ __global__ __launch_bounds__(D) void attention_kernel(AttnArgs a) {
     if (tid == 0) __hip_atomic_store(a.counters + slot, 0u, __ATOMIC_RELAXED, kScope);
 }
 
+// ---- decode attention of wide heads on the matrix cores -------------------------------------------
+//
+// One token, 512-wide heads, 4 to 16 query heads per KV head (kAttnMfmaGroup on), on the fp16 MFMAs:
+// attention_kernel takes two query heads per block there, so that a KV head's cache is read 8 times and
+// every cached value is unpacked and multiplied 16 times on the VALU.  Here the KV head's query
+// heads are the 16 columns of S^T = K Q^T and O^T = V^T P^T (fewer heads: zero queries), with the fp32
+// queries and probabilities as scaled fp16 pairs hi + lo (about 22 bits, products exact in fp32), as in
+// the batched attention.
+//
+// A workgroup of four waves takes one chunk of the visible keys, 64 at a time:
+// - scores: wave w's 16 keys; a lane's operand is 16 bytes of its key's row, loaded straight from the
+//   cache (key lane % 16, channels 32 s + 8 (lane / 16) of step s);
+// - the waves exchange their maxima and then their probabilities through LDS (two barriers);
+// - values: wave w's 128 channels of all 64 keys with the 16-key MFMA: lane (m, q) loads channels 128 w
+//   + 8 m .. + 7 of keys 4 q + i and takes channel e of four keys as the operand of tile e: the channels
+//   a tile holds are every eighth one, which only orders the output.  No transpose.
+// K and V of the next 64 keys are requested as soon as this one's registers are free, the first ones
+// before the prologue.  The chunks' partials go to scratch and attention_mfma_merge_kernel adds them, one
+// workgroup per query head and 128 channels: 64 chunks of 16 heads are 2 MB, which one last
+// workgroup would read for longer than another launch takes.
+//
+// 16 query heads on one KV head: 16.7 us against 31.1 at 4,096 positions, 28.4 against 87.4 at 32,768 (of
+// them 4.8 us the merge, 3 us the loop at 4,096, the rest the launch and the prologue's chain).  Error
+// against 64 bits 2.1e-7 at 4,096 (attention_kernel: 2.2e-7).
+// Keys per chunk (a multiple of 64) and chunks of n visible keys in at most cmax chunks.
+__host__ __device__ inline uint32_t attn_mfma_span(uint32_t n, uint32_t cmax) {
+    const uint32_t tiles = (n + 63) / 64;
+    return (tiles + cmax - 1) / cmax * 64;
+}
+
+typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+typedef _Float16 h4 __attribute__((ext_vector_type(4)));
+
+__global__ __launch_bounds__(256) void attention_mfma_kernel(AttnArgs a) {
+    constexpr int D = 512, QP = D + 8;  // query row stride (halves)
+    __shared__ __align__(16) _Float16 qh[16 * QP], ql[16 * QP];
+    __shared__ __align__(16) double rsin[D / 2], rcos[D / 2];  // of the position's angles
+    __shared__ __align__(16) uint16_t knew[D], vnew[D];
+    __shared__ __align__(16) _Float16 ph[4][16][16], pl[4][16][16];  // [16-key group][query][key]
+    __shared__ float qscale[16], wmax[4][16], wsum[4][16];
+
+    if (a.state && a.state[ST_STOP]) return;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = wave_id(), m = lane & 15, q = lane >> 4;
+    const uint32_t c = blockIdx.x, h = blockIdx.y, group = a.group;
+    const uint32_t pos = a.state ? a.state[ST_POS] : a.position;
+    const uint32_t nvis = a.window ? min(pos + 1, a.window) : pos + 1, start = pos + 1 - nvis;
+    const uint32_t span = attn_mfma_span(nvis, a.cmax);
+    if (c * span >= nvis) return;
+    const uint32_t k_begin = start + c * span, k_end = min(k_begin + span, pos + 1);
+    const bool has_new = k_end == pos + 1;
+
+    const uint16_t* kh = a.kcache + (size_t)h * a.ring * D;
+    const uint16_t* vh = a.vcache + (size_t)h * a.ring * D;
+    v4u kr[16], vr[4][4];
+    // rows past the chunk's last key repeat it (their scores are masked, their values cleared)
+    auto load_k = [&](uint32_t k0) {
+        const uint16_t* p = kh + (size_t)(min(k0 + 16 * wave + m, k_end - 1) % a.ring) * D + 8 * q;
+#pragma unroll
+        for (int s = 0; s < 16; ++s) kr[s] = *gp(reinterpret_cast<const v4u*>(p + 32 * s));
+    };
+    auto load_v = [&](uint32_t k0) {
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                vr[g][i] = *gp(reinterpret_cast<const v4u*>(vh + (size_t)(min(k0 + 16 * g + 4 * q + i, k_end - 1) % a.ring) * D + 128 * wave + 8 * m));
+    };
+
+    // ---- prologue: wave w normalises and rotates query heads w, w + 4, ...; lane: channel pairs
+    // (4 lane + k, 4 lane + k + 256), channel 4 lane + k at k and its partner at k + 4
+    constexpr int NH = 4;
+    float x[NH][8], kx[8], vx[8], qw[8], kw[8];
+    auto row8 = [&](const float* p, float (&o)[8]) {
+        const v4f lo = *gp(reinterpret_cast<const v4f*>(p + 4 * lane)), hi = *gp(reinterpret_cast<const v4f*>(p + 256 + 4 * lane));
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            o[k] = lo[k];
+            o[k + 4] = hi[k];
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < NH; ++i) row8(a.q_raw + ((size_t)h * group + min(wave + 4 * i, group - 1)) * D, x[i]);
+    row8(a.q_norm, qw);
+    row8(a.k_norm, kw);
+    row8(a.k_raw + (size_t)h * D, kx);
+    row8(a.v_raw + (size_t)h * D, vx);
+    const double ifreq = a.inv_freq[tid];
+    __builtin_amdgcn_sched_barrier(0);
+    load_k(k_begin);
+    load_v(k_begin);
+    __builtin_amdgcn_sched_barrier(0);
+    double sn, cs;
+    sincos((double)pos * ifreq, &sn, &cs);
+    rsin[tid] = sn;
+    rcos[tid] = cs;
+    double ss[NH], kss = 0.0;
+#pragma unroll
+    for (int i = 0; i < NH; ++i) {
+        double v = 0.0;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) v += (double)x[i][k] * (double)x[i][k];
+        ss[i] = wave_sum(v);
+    }
+    const bool k_wave = has_new && wave == 0, v_wave = has_new && wave == 1;
+    if (k_wave || v_wave) {
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            const double u = k_wave ? kx[k] : vx[k];
+            kss += u * u;
+        }
+        kss = wave_sum(kss);
+    }
+    __syncthreads();  // rsin, rcos
+    auto rotate = [&](const float (&v)[8], double r, const float (&w)[8], float (&o)[8]) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const double sn = rsin[4 * lane + k], cs = rcos[4 * lane + k];
+            const double u0 = (double)norm_apply(v[k], r, w[k]), u1 = (double)norm_apply(v[k + 4], r, w[k + 4]);
+            o[k] = (float)__dsub_rn(__dmul_rn(u0, cs), __dmul_rn(u1, sn));
+            o[k + 4] = (float)__dadd_rn(__dmul_rn(u0, sn), __dmul_rn(u1, cs));
+        }
+    };
+#pragma unroll
+    for (int i = 0; i < NH; ++i) {
+        const uint32_t hq = wave + 4 * i;
+        float o[8];
+        rotate(x[i], inv_rms_fast(ss[i], D, a.q_eps), qw, o);
+        float mx = 0.0f;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) {
+            if (hq >= group) o[k] = 0.0f;
+            mx = fmaxf(mx, fabsf(o[k]));
+        }
+        mx = wave_max(mx);
+        const float s = mx > 0.0f ? ldexpf(1.0f, 4 - ilogbf(mx)) : 1.0f;  // |q s| < 32
+#pragma unroll
+        for (int k = 0; k < 8; k += 4) {
+            h4 hi, lo;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const float u = o[k + j] * s;
+                hi[j] = (_Float16)u;
+                lo[j] = (_Float16)(u - (float)hi[j]);
+            }
+            *reinterpret_cast<h4*>(qh + hq * QP + 64 * k + 4 * lane) = hi;
+            *reinterpret_cast<h4*>(ql + hq * QP + 64 * k + 4 * lane) = lo;
+        }
+        if (lane == 0) qscale[hq] = a.scale / s;  // (s is a power of two)
+    }
+    if (k_wave) {
+        float o[8];
+        rotate(kx, inv_rms_fast(kss, D, a.k_eps), kw, o);
+#pragma unroll
+        for (int k = 0; k < 8; ++k) knew[4 * lane + k % 4 + 256 * (k / 4)] = f2h(o[k]);
+    }
+    if (v_wave) {
+        const double r = inv_rms_fast(kss, D, a.v_eps);
+#pragma unroll
+        for (int k = 0; k < 8; ++k)
+            vnew[4 * lane + k % 4 + 256 * (k / 4)] = f2h(a.v_norm ? (float)__dmul_rn((double)vx[k], r) : vx[k]);
+    }
+    __syncthreads();
+    if (has_new) {  // append
+        const size_t at = ((size_t)h * a.ring + pos % a.ring) * D;
+        reinterpret_cast<uint32_t*>(a.kcache + at)[tid] = reinterpret_cast<const uint32_t*>(knew)[tid];
+        reinterpret_cast<uint32_t*>(a.vcache + at)[tid] = reinterpret_cast<const uint32_t*>(vnew)[tid];
+    }
+
+    v4f acc[8], accl[8];  // sums of the hi and of the lo products
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] = accl[e] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    float mrun = -INFINITY, lrun = 0.0f;  // of query m
+    const float qs = qscale[m];
+    for (uint32_t k0 = k_begin; k0 < k_end; k0 += 64) {
+        // scores of keys k0 + 16 w + 4 q + e, query m; the new key's row is in LDS (its cache slot may be
+        // written meanwhile)
+        if (k0 + 16 * wave + m == pos) {
+#pragma unroll
+            for (int s = 0; s < 16; ++s) kr[s] = *reinterpret_cast<const v4u*>(knew + 32 * s + 8 * q);
+        }
+        // (eight sums of the hi products and one of the lo products: a chain of 32 additions at the score's
+        // size would double the error against 64 bits)
+        v4f sh[8], sv = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) sh[i] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int s = 0; s < 16; ++s) {
+            const h8 A = __builtin_bit_cast(h8, kr[s]);
+            sh[s % 8] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, *reinterpret_cast<const h8*>(qh + m * QP + 32 * s + 8 * q), sh[s % 8], 0, 0, 0);
+            sv = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, *reinterpret_cast<const h8*>(ql + m * QP + 32 * s + 8 * q), sv, 0, 0, 0);
+        }
+        sv = (((sh[0] + sh[1]) + (sh[2] + sh[3])) + ((sh[4] + sh[5]) + (sh[6] + sh[7]))) + sv;
+        if (k0 + 64 < k_end) load_k(k0 + 64);
+        float mx = -INFINITY;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            sv[e] = k0 + 16 * wave + 4 * q + e < k_end ? sv[e] * qs : -INFINITY;
+            mx = fmaxf(mx, sv[e]);
+        }
+        mx = positions_max<16>(mx);
+        if (q == 0) wmax[wave][m] = mx;
+        __syncthreads();
+        const float mn = fmaxf(fmaxf(mrun, fmaxf(wmax[0][m], wmax[1][m])), fmaxf(wmax[2][m], wmax[3][m]));
+        const float al = expf(mrun - mn);  // (key k0 is visible: mn is finite)
+        float sum = 0.0f;
+        h4 hi, lo;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float p = sv[e] == -INFINITY ? 0.0f : expf(sv[e] - mn);
+            sum += p;
+            const float u = p * 16384.0f;
+            hi[e] = (_Float16)u;
+            lo[e] = (_Float16)(u - (float)hi[e]);
+        }
+        *reinterpret_cast<h4*>(&ph[wave][m][4 * q]) = hi;
+        *reinterpret_cast<h4*>(&pl[wave][m][4 * q]) = lo;
+        sum = row_total(sum);
+        if (q == 0) wsum[wave][m] = sum;
+        __syncthreads();
+        mrun = mn;
+        lrun = fmaf(lrun, al, (wsum[0][m] + wsum[1][m]) + (wsum[2][m] + wsum[3][m]));
+        // values of channels 128 w + 8 (4 q + i) + e, query m
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+            acc[e] *= al;
+            accl[e] *= al;
+        }
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint32_t key = k0 + 16 * g + 4 * q + i;
+                if (key >= k_end) vr[g][i] = v4u{0u, 0u, 0u, 0u};  // (what a probability of zero multiplies must be finite)
+                else if (key == pos) vr[g][i] = *reinterpret_cast<const v4u*>(vnew + 128 * wave + 8 * m);
+            }
+            const h4 bh = *reinterpret_cast<const h4*>(&ph[g][m][4 * q]), bl = *reinterpret_cast<const h4*>(&pl[g][m][4 * q]);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const uint32_t sel = e & 1 ? 0x07060302u : 0x05040100u;
+                const v2u w = {__builtin_amdgcn_perm(vr[g][1][e / 2], vr[g][0][e / 2], sel),
+                               __builtin_amdgcn_perm(vr[g][3][e / 2], vr[g][2][e / 2], sel)};
+                const h4 A = __builtin_bit_cast(h4, w);
+                acc[e] = __builtin_amdgcn_mfma_f32_16x16x16f16(A, bh, acc[e], 0, 0, 0);
+                accl[e] = __builtin_amdgcn_mfma_f32_16x16x16f16(A, bl, accl[e], 0, 0, 0);
+            }
+        }
+        if (k0 + 64 < k_end) load_v(k0 + 64);
+    }
+    if (m >= group) return;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] += accl[e];
+    constexpr uint32_t R = attn_part_row(D);
+    float* pr = a.part + (((size_t)h * a.cmax + c) * group + m) * R;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int e = 0; e < 8; e += 4)
+            *reinterpret_cast<float4*>(pr + 128 * wave + 8 * (4 * q + i) + e) =
+                make_float4(acc[e][i] * (1.0f / 16384.0f), acc[e + 1][i] * (1.0f / 16384.0f),
+                            acc[e + 2][i] * (1.0f / 16384.0f), acc[e + 3][i] * (1.0f / 16384.0f));
+    if (wave == 0 && q == 0) *reinterpret_cast<float2*>(pr + D) = make_float2(mrun, lrun);
+}
+
+// out = sum_c w_c o_c / sum_c w_c l_c, w_c = exp(m_c - max m), over the chunks of one query head; block
+// (128 channels, query head), 16 phases of 32 threads (four channels each) over the chunks.
+__global__ __launch_bounds__(512) void attention_mfma_merge_kernel(AttnArgs a) {
+    constexpr int D = 512, PH = 16;
+    constexpr uint32_t R = attn_part_row(D);
+    __shared__ float w[kAttnMfmaChunks], red[8];
+    __shared__ __align__(16) float4 acc[PH][32];
+    if (a.state && a.state[ST_STOP]) return;
+    const uint32_t tid = threadIdx.x, h = blockIdx.y / a.group, g = blockIdx.y % a.group;
+    const uint32_t pos = a.state ? a.state[ST_POS] : a.position;
+    const uint32_t nvis = a.window ? min(pos + 1, a.window) : pos + 1;
+    const uint32_t span = attn_mfma_span(nvis, a.cmax), chunks = (nvis + span - 1) / span;
+    const float* base = a.part + ((size_t)h * a.cmax * a.group + g) * R;
+    const size_t step = (size_t)a.group * R;
+    const uint32_t f = tid % 32, phase = tid / 32, ch = blockIdx.x * 128 + 4 * f;
+    // this thread's first pieces are requested before the weights are known
+    constexpr int U = 4;
+    float4 v[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) v[u] = *reinterpret_cast<const float4*>(base + min(phase + PH * u, chunks - 1) * step + ch);
+    const float2 ml = tid < chunks ? *reinterpret_cast<const float2*>(base + tid * step + D) : make_float2(-INFINITY, 0.0f);
+    const float M = block_max_f(ml.x, red);
+    const float wc = ml.x == -INFINITY ? 0.0f : expf(ml.x - M);
+    if (tid < kAttnMfmaChunks) w[tid] = wc;
+    const float L = block_sum_f(wc * ml.y, red);  // (its barriers publish w)
+    float4 s = make_float4(0.f, 0.f, 0.f, 0.f);
+    for (uint32_t k0 = phase; k0 < chunks; k0 += PH * U) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const uint32_t k = k0 + PH * u;
+            const float wk = k < chunks ? w[k] : 0.0f;
+            if (k0 != phase) v[u] = *reinterpret_cast<const float4*>(base + min(k, chunks - 1) * step + ch);
+            s.x = fmaf(wk, v[u].x, s.x);
+            s.y = fmaf(wk, v[u].y, s.y);
+            s.z = fmaf(wk, v[u].z, s.z);
+            s.w = fmaf(wk, v[u].w, s.w);
+        }
+    }
+    acc[phase][f] = s;
+    __syncthreads();
+    if (tid >= 32) return;
+    float4 t = acc[0][tid];
+#pragma unroll
+    for (int p = 1; p < PH; ++p) {
+        t.x += acc[p][tid].x;
+        t.y += acc[p][tid].y;
+        t.z += acc[p][tid].z;
+        t.w += acc[p][tid].w;
+    }
+    *reinterpret_cast<float4*>(a.out + (size_t)(h * a.group + g) * D + ch) = make_float4(t.x / L, t.y / L, t.z / L, t.w / L);
+}
+
 // Query heads per attention block: all of a KV head's at width 256 (1, 2 or 4), two at width 512
 // (one for a single query head per KV head), so the block's LDS stays within bounds.
 uint32_t attention_block_heads(uint32_t group, uint32_t head_width) {
@@ -1436,6 +1751,28 @@ hipError_t launch_attention(const AttnArgs& args, uint32_t group, uint32_t head_
     } else {
         return hipErrorInvalidValue;
     }
+    return hipGetLastError();
+}
+
+// Whether a decode step's attention over at most `span` positions takes attention_mfma_kernel.
+bool attention_mfma(uint32_t group, uint32_t head_width, uint32_t span) {
+    return head_width == 512 && group >= kAttnMfmaGroup && span > kAttnMfmaSpan;
+}
+
+// Chunks of attention_mfma_kernel: one per 64 keys, at most kAttnMfmaChunks per KV head and one per CU
+// in all.
+uint32_t attention_mfma_chunks(uint32_t kv_heads, uint32_t span) {
+    return std::max(1u, std::min({(span + 63) / 64, kAttnMfmaChunks, 256 / std::min(kv_heads, 256u)}));
+}
+
+hipError_t launch_attention_mfma(const AttnArgs& a, uint32_t group, hipStream_t s) {
+    if (a.group != group || group > 16 || a.kv_heads == 0 || a.cmax == 0 || a.cmax > kAttnMfmaChunks ||
+        a.mode != ATT_DECODE || a.raw_parts)
+        return hipErrorInvalidValue;
+    hipLaunchKernelGGL(attention_mfma_kernel, dim3(a.cmax, a.kv_heads), dim3(256), 0, s, a);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) return e;
+    hipLaunchKernelGGL(attention_mfma_merge_kernel, dim3(4, a.kv_heads * group), dim3(512), 0, s, a);
     return hipGetLastError();
 }
 

@@ -1,0 +1,87 @@
+"""Decode attention of 512-wide heads with 4 to 16 query heads per KV head (attention_mfma_kernel and its
+merge) through af_attention_decode, against the oracle, at chunk and key-group boundaries."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import oracle
+from adaforge_amd import _native as N, hip, synth
+
+pytestmark = pytest.mark.gpu
+W = 512
+
+
+def rope(x, heads, factors, pos):
+    return oracle.rope(W, 1e6, factors, 131072, x, pos).astype(np.float32)
+
+
+def normed(w, x):
+    return oracle.rmsnorm(w, 1e-6, x).astype(np.float32)
+
+
+@pytest.mark.parametrize("context,window,q_heads,kv_heads,scale", [
+    (1025, None, 16, 1, 1.0),     # one key into a seventeenth 64-key chunk
+    (1088, None, 8, 1, 0.05),     # whole chunks; half the query columns empty
+    (1500, 1100, 4, 1, 0.05),     # a window that starts inside the cache and ends off a 16-key group
+    (1041, None, 32, 2, 0.05),    # two KV heads
+    (1300, 1030, 16, 4, 1.0),     # a wrapped ring
+    (16449, None, 16, 1, 0.05),   # more keys than 64 per chunk
+])
+def test_wide_heads_match_oracle(context, window, q_heads, kv_heads, scale):
+    pos, v_norm = context - 1, 1
+    ring = context if window is None else window + 17
+    rng = np.random.default_rng(context + q_heads)
+    q, k, v = (rng.standard_normal(h * W).astype(np.float32) for h in (q_heads, kv_heads, kv_heads))
+    qn, kn = (1 + 0.1 * rng.standard_normal((2, W))).astype(np.float32)
+    if scale == 1.0:
+        qn *= np.float32(W ** -0.5)
+    keys = rng.standard_normal((context, kv_heads, W)).astype(np.float16)
+    values = (rng.standard_normal((context, kv_heads, W)) * np.exp2(rng.integers(-20, 1, (1, kv_heads, W)))).astype(np.float16)
+    factors = synth.gemma4_rope_factors(W)
+    first = 0 if window is None else max(0, context - window)
+    kc = np.full((kv_heads, ring, W), np.nan, np.float16)  # every slot that is not visible is a NaN
+    vc = kc.copy()
+    for t in range(first, pos):
+        kc[:, t % ring], vc[:, t % ring] = keys[t], values[t]
+    bufs = [hip.Buffer.from_numpy(a) for a in (q, k, v, qn, kn, kc.view(np.uint16), vc.view(np.uint16))]
+    out = hip.Buffer(q_heads * W)
+    args = N.AttentionArgs(*(b.ptr for b in bufs[:5]), 1e-6, 1e-6, 1e-6, v_norm,
+                           N.RopeDesc(W, 1e6, factors.ctypes.data_as(N.f32p), 131072),
+                           N.AttentionConfigDesc(q_heads, kv_heads, W, window or 0, scale),
+                           bufs[5].ptr, bufs[6].ptr, ring, pos, out.ptr)
+    N.check(N.lib().af_attention_decode(ctypes.byref(args), None))
+    hip.synchronize()
+    got = out.numpy()
+    k_new = rope(np.concatenate([normed(kn, k[i * W:(i + 1) * W]) for i in range(kv_heads)]), kv_heads, factors, pos)
+    v_new = np.concatenate([normed(np.ones(W, np.float32), v[i * W:(i + 1) * W]) for i in range(kv_heads)])
+    slot = bufs[5].numpy().view(np.float16)[:, pos % ring].astype(np.float32).ravel()
+    vslot = bufs[6].numpy().view(np.float16)[:, pos % ring].astype(np.float32).ravel()
+    assert np.abs(slot - k_new).max() <= 2.0 ** -10 * np.abs(k_new).max()
+    assert np.abs(vslot - v_new).max() <= 2.0 ** -10 * np.abs(v_new).max()
+    keys[pos], values[pos] = slot.reshape(kv_heads, W), vslot.reshape(kv_heads, W)
+    q_rot = rope(np.concatenate([normed(qn, q[i * W:(i + 1) * W]) for i in range(q_heads)]), q_heads, factors, pos)
+    ref = oracle.attention(q_heads, kv_heads, W, window, scale, q_rot, keys.astype(np.float32).ravel(),
+                           values.astype(np.float32).ravel(), context, pos)
+    oracle.compare(ref, got)
+    # and per channel's own scale (values down to 2^-20 of the largest, below fp16's normal range):
+    # 32-bit sums of at most `context` terms at 22-bit probabilities
+    size = np.abs(values[first:context].astype(np.float32)).max(0)  # [kv_heads][W]
+    size = np.repeat(size, q_heads // kv_heads, 0).ravel()
+    assert (np.abs(got - ref) <= 2.0 ** -17 * size + 1e-12).all()
+
+
+def test_session_past_the_threshold_matches_the_batched_layers():
+    """A Gemma-4-shaped session past 1,024 positions: logits after 24 tokens consumed one at a time (the
+    step's matrix-core attention) against the same tokens through the batched layers."""
+    from tests.test_gpu_batch import open_with_env
+    model = synth.gemma4_model(name="gemma4-past", layers=2, hidden=1024, intermediate=2048, local_q=(16, 8, 256),
+                               global_q=(16, 1, 512), vocabulary=2048, window=16, global_every=2)
+    ids = [int(i) for i in synth.prompt_ids(1064, model.vocabulary, name="gemma4-past.ids")]
+    got = []
+    for batch in (0, 32):
+        with open_with_env(model, 1100, AF_TRACE_BATCH=batch) as s:
+            s.generate(ids[:1040], [2047], 1)   # (its id is part of both conversations)
+            got.append(s.trace(ids[1040:], layer_outputs=False)[2])
+    assert np.abs(got[0] - got[1]).max() <= 1e-3 * np.abs(got[1]).max()
+    assert int(np.argmax(got[0])) == int(np.argmax(got[1]))
