@@ -1,7 +1,6 @@
 // Host side of the C ABI (include/af.h): validation, weight repacking and
-// upload, standalone operators, and the generation session that captures the
-// whole decode step (the persistent launch of every layer, then the head with greedy
-// selection) as one HIP graph replayed per token.
+// upload, standalone operators, and the generation session, whose decode step is the
+// persistent launch of every layer, then the head with greedy selection.
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -973,7 +972,8 @@ struct af_session {
     std::vector<uint32_t> cached;  // tokens of the conversation (GenerationSession prefix)
     uint32_t consumed = 0;         // positions with K/V in the caches
     bool poisoned = false;
-    bool use_graphs = true;
+    bool use_graphs = true;             // replay captured steps (per-operation sessions)
+    bool graphs_after_fall_back = false;
     KernelTimer* timer = nullptr;  // set during af_session_profile
     // Batched prefill (batch.hip): prompt positions run through the layers up to kPassMax at a time,
     // every weight read once per pass.  prefill_batch: positions per pass for generation
@@ -1269,8 +1269,8 @@ struct af_session {
         return AF_OK;
     }
 
-    // One decode (with_head) or prefill step: a replay of the graph captured at open, or direct
-    // launches (AF_DISABLE_GRAPHS).  Every argument of a step's launches is fixed for the session
+    // One decode (with_head) or prefill step: direct launches, or a replay of the graph captured at open
+    // (per-operation sessions without AF_DISABLE_GRAPHS).  Every argument of a step's launches is fixed for the session
     // (the position, ids and stop state live in device memory), so one graph serves every token.
     hipError_t run_step(bool with_head) {
         if (use_graphs) return hipGraphLaunch(with_head ? decode_exec : prefill_exec, stream);
@@ -1309,6 +1309,7 @@ struct af_session {
     // an interrupted merge left are cleared; the graphs are recaptured for the new path.
     int fall_back() {
         use_step = false;
+        use_graphs = graphs_after_fall_back;
         HIP_OK(hipMemsetAsync(COUNTERS.p, 0, COUNTERS.bytes, stream), "attention counters clear");
         HIP_OK(hipStreamSynchronize(stream), "fall-back");
         if (use_graphs) {
@@ -1879,15 +1880,20 @@ int open_session(const af_layer_weights* layers, uint32_t n_layers, const af_out
     HIP_OK(hipEventCreate(&s->ev_start), "event");
     s->attn_xl = attn_xcd_local();
     if ((rc = setup_step(*s))) return rc;
-    // A model whose step mixes step-kernel runs with per-operation layers is launched directly:
-    // replays of its captured step faulted on the host inside hipGraphLaunch under a rocprofv3
-    // kernel trace (cause not established), and without a profiler it decodes at the same rate
-    // either way (at most kDecodeAhead steps are queued ahead, so launch costs are hidden).
-    if (s->use_step && s->segmented()) s->use_graphs = false;
+    // Steps of the step kernel are launched directly, two launches per token: between tokens a graph
+    // replay leaves 13.4 us from the head's end to the next launch, direct launches 5.7 (64 tokens of
+    // six layers: 19.82 against 19.41 ms; 48 layers decode 0.4 % faster), and at most kDecodeAhead
+    // steps are queued ahead, so the launches' host time is hidden.  A step whose layers all run per
+    // operation is five launches per layer and replayed as a graph, also after a fall-back.  A step that
+    // mixes both is never captured: its replays faulted on the host inside hipGraphLaunch under a
+    // rocprofv3 kernel trace (cause not established), at the same rate as direct launches.
+    if (s->use_step) {
+        s->graphs_after_fall_back = s->use_graphs && !s->segmented();
+        s->use_graphs = false;
+    }
     HIP_OK(hipDeviceSynchronize(), "session upload");
     if (s->use_graphs) {
-        // the step kernel and the head (decode), or the step kernel alone (prefill); on the
-        // per-operation path every layer's kernels.  No timeline memset is recorded: the timer
+        // every layer's kernels, with the head (decode) or without (prefill).  No timeline memset is recorded: the timer
         // that adds it is only set around direct launches (af_session_profile).
         if ((rc = s->capture(true, s->decode_graph, s->decode_exec))) return rc;
         if ((rc = s->capture(false, s->prefill_graph, s->prefill_exec))) return rc;

@@ -233,13 +233,12 @@ typedef void (*af_token_fn)(void* user, uint32_t id);
 typedef struct af_session af_session;
 
 /* open_session: uploads every layer and the head, allocates KV caches for `capacity`
- * tokens (1..AF_MAX_CONTEXT) and captures the decode step (one launch for every layer, then the
- * head with greedy selection) and the prefill step (the layers alone) as HIP graphs, replayed
- * once per token (crates/cuda-backend/src/stack.rs:1100-1145 captures its layers the same way).
- * Layers outside the persistent step kernel's limits (Gemma 4's 512-wide global layers) run on
- * the per-operation kernels, between one step-kernel launch per run of the other layers; such a
- * session launches its steps directly (no graph: the same rate, measured).  A model with no layer
- * the step kernel takes runs on the per-operation kernels alone, captured as graphs.  With
+ * tokens (1..AF_MAX_CONTEXT).  A decode step is one launch for every layer, then the head with greedy
+ * selection; a prefill step the layers alone.  Layers outside the persistent step kernel's limits
+ * (Gemma 4's 512-wide global layers) run on the per-operation kernels, between one step-kernel launch
+ * per run of the other layers.  A model with no layer the step kernel takes runs on the per-operation
+ * kernels alone, its steps captured as HIP graphs and replayed once per token
+ * (crates/cuda-backend/src/stack.rs:1100-1145 captures its layers the same way).  With
  * AF_DISABLE_GRAPHS set in the environment every session launches its steps directly. */
 int af_session_open(const af_layer_weights* layers, uint32_t n_layers, const af_output_head* head,
                     uint32_t capacity, af_session** out);
