@@ -198,8 +198,9 @@ constexpr uint32_t kBatchMax = 32;   // tokens per batch (crates/cuda-backend/sr
 // where lane 16 q + t % 16 holds elements 4 q + {0, 2}, 16 + 4 q + {0, 2}, 4 q + {1, 3}, 16 + 4 q +
 // {1, 3} of token t's block: the order in which a dword of four code bytes unpacks.
 constexpr uint32_t kPassMax = 512;
-// Tokens of a wide GEMM workgroup's tile: 128, or 64 when a tile of 128 would be half padding.
-__host__ __device__ inline uint32_t wide_tokens(uint32_t T) { return T % 128 == 0 || T % 128 > 64 ? 128u : 64u; }
+// Tokens of a wide GEMM workgroup's tile: 64 for a pass of at most 64 tokens (a tile of 128 would be half
+// padding), else 128 (three tiles of 64 took as long as two of 128).
+__host__ __device__ inline uint32_t wide_tokens(uint32_t T) { return T > 64 ? 128u : 64u; }
 __host__ __device__ inline uint32_t wide_groups(uint32_t T) {
     const uint32_t m = wide_tokens(T);
     return (T + m - 1) / m * (m / 16);

@@ -615,12 +615,12 @@ __global__ __launch_bounds__(256) void batch_reduce_kernel(BatchGemm a, uint32_t
 
 // ---- Q4_0 GEMM over a wide pass -------------------------------------------------------------------
 //
-// y[t][r] = sum_b d_rb sum_j (n_rbj - 8) x_tbj for more than kBatchMax tokens.  A workgroup of four
-// waves takes M = 64 WM tokens x 64 WN rows (WM WN = 4; a wave 64 x 64: 4 x 4 MFMA tiles) over K range
-// `split`, one 32-weight block (one MFMA depth) per step: the tokens' halves are copied from the
-// image, which is laid out as the MFMAs read it, and the weights unpacked once per workgroup, both
-// into LDS, double buffered; step s + 1's are written while step s is multiplied, and step s + 2's
-// loads are in flight.  The block's d_rb differs from the next one's, so each block's 16 x 16
+// y[t][r] = sum_b d_rb sum_j (n_rbj - 8) x_tbj for more than kBatchMax tokens.  A workgroup takes M = 64 WM
+// tokens x 64 WN rows over K range `split`, WM x WN waves of 64 x 64 (4 x 4 MFMA tiles) for each of WK
+// 32-weight blocks (one MFMA depth) per step: the tokens' halves are copied from the image, which
+// is laid out as the MFMAs read it, and the weights unpacked once per workgroup, both into LDS,
+// double buffered; step s + 1's are written while step s is multiplied, and step s + 2's loads are
+// in flight.  The WK waves of a tile add their sums in LDS at the end.  The block's d_rb differs from the next one's, so each block's 16 x 16
 // products are folded into fp32 sums on their own (one FMA per product and lane: half as many VALU
 // cycles as the two MFMAs take; the token's scale waits for the epilogue, so that the fold has no other
 // factor).  Sums run over kWideChain blocks, then join a total, so that no chain of fp32 additions is
@@ -631,33 +631,37 @@ __global__ __launch_bounds__(256) void batch_reduce_kernel(BatchGemm a, uint32_t
 // an L2.
 constexpr uint32_t kWideChain = 8;
 
-template <int WM, int P>
-__global__ __launch_bounds__(256, 2) void wide_gemm_kernel(BatchGemm a, uint32_t S, uint32_t mtiles, uint32_t ngroups) {
-    constexpr int WN = 4 / WM, MG = 4 * WM, NT = 4 * WN;  // 16-token groups and 16-row tiles of the workgroup
-    __shared__ v4u As[2][MG * 128];  // [token group][hi, lo][64 lanes]
-    __shared__ v4u Bs[2][NT * 64];   // [row tile][64 lanes]
+template <int WM, int WN, int WK, int P>
+__global__ __launch_bounds__(64 * WM * WN * WK, 2 / WK ? 2 / WK : 1) void wide_gemm_kernel(BatchGemm a, uint32_t S, uint32_t mtiles, uint32_t ngroups) {
+    constexpr int MG = 4 * WM, NT = 4 * WN;       // 16-token groups and 16-row tiles of the workgroup
+    constexpr int W = WM * WN * WK, TH = 64 * W;  // waves, threads
+    constexpr int SA = 8 / WN, SB = 4 / WM;       // 16-byte pieces of the image and code dwords per thread and step
+    constexpr int kA = MG * 128 * WK, kB = NT * 64 * WK;  // v4u per stage
+    __shared__ v4u smem[WK > 1 && W * 1024 > 2 * (kA + kB) ? W * 1024 : 2 * (kA + kB)];
+    // stage buf: [block of the step][token group][hi, lo][64 lanes], then [block][row tile][64 lanes]
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = wave_id(), r = lane & 15, q = lane >> 4;
-    const uint32_t wm = wave / WN, wn = wave % WN;
+    const uint32_t wk = wave / (WM * WN), wm = wave / WN % WM, wn = wave % WN;
     const uint32_t total = mtiles * ngroups * S, per = gridDim.x / 8;
     const uint32_t item = blockIdx.x % 8 * per + blockIdx.x / 8;
     if (item >= total) return;
     const uint32_t mt0 = item % mtiles, ng = item / mtiles % ngroups, split = item / mtiles / ngroups;
     const uint32_t nb = a.w.blocks, G = mtiles * MG, tiles = (a.w.rows + 15) / 16;
-    const uint32_t b0 = nb * split / S, b1 = nb * (split + 1) / S;
+    const uint32_t b0 = nb * split / S, b1 = nb * (split + 1) / S, last = b1 - 1;
     // row tile i of the workgroup (of wave i / 4): a gate/up pair's waves hold two tiles of each matrix,
     // alternating, so that a lane holds both products of a row
     auto tile_of = [&](uint32_t i) { return P == 2 ? ng * (NT / 2) + i / 4 * 2 + (i % 4) / 2 : ng * NT + i; };
     auto mat_of = [&](uint32_t i) -> const Q4View& { return P == 2 && (i & 1) ? a.w2 : a.w; };
 
-    const v4u* img = reinterpret_cast<const v4u*>(a.img) + (size_t)mt0 * MG * 128 + tid;
-    v4u sa[MG / 2];    // step s + 1's halves on their way to LDS
-    uint32_t sc[WN];   // and code dwords of the row tiles this wave unpacks (wave WN .. + WN - 1)
-    uint16_t dn[4];    // the next step's scales of the lane's rows
-    const uint8_t* cp[WN];
+    // this thread's share of a step: image pieces tid + TH i of its WK blocks (kA / WK per block), and the code
+    // dwords of row tiles wave SB + i (of block (wave SB + i) / NT)
+    v4u sa[SA];
+    uint32_t sc[SB];
+    uint16_t dn[4];  // the next step's scales of the lane's rows
+    const uint8_t* cp[SB];
     const uint16_t* dp[4];
 #pragma unroll
-    for (int i = 0; i < WN; ++i) {
-        const uint32_t k = wave * WN + i;
+    for (int i = 0; i < SB; ++i) {
+        const uint32_t k = (wave * SB + i) % NT;
         cp[i] = mat_of(k).codes + (size_t)min(tile_of(k), tiles - 1) * a.w.nst * 1024 + r * 16 + q * 4;
     }
 #pragma unroll
@@ -665,21 +669,27 @@ __global__ __launch_bounds__(256, 2) void wide_gemm_kernel(BatchGemm a, uint32_t
         const uint32_t k = wn * 4 + i;
         dp[i] = mat_of(k).scales + (size_t)min(tile_of(k), tiles - 1) * a.w.nst * 64 + r;
     }
-    auto load = [&](uint32_t b) {
+    const v4u* img = reinterpret_cast<const v4u*>(a.img) + (size_t)mt0 * MG * 128;
+    auto load = [&](uint32_t b) {  // (blocks past the range repeat its last one; their scales are zeroed)
 #pragma unroll
-        for (int i = 0; i < MG / 2; ++i) sa[i] = *gp(img + (size_t)b * G * 128 + 256 * i);
+        for (int i = 0; i < SA; ++i) {
+            const uint32_t e = tid + TH * i;
+            sa[i] = *gp(img + (size_t)min(b + e / (MG * 128), last) * G * 128 + e % (MG * 128));
+        }
 #pragma unroll
-        for (int i = 0; i < WN; ++i) sc[i] = *gp(reinterpret_cast<const uint32_t*>(cp[i] + (size_t)b * 256));
+        for (int i = 0; i < SB; ++i)
+            sc[i] = *gp(reinterpret_cast<const uint32_t*>(cp[i] + (size_t)min(b + (wave * SB + i) / NT, last) * 256));
     };
     auto load_d = [&](uint32_t b) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) dn[i] = gp(dp[i])[(size_t)b * 16];
+        for (int i = 0; i < 4; ++i) dn[i] = gp(dp[i])[(size_t)min(b + wk, last) * 16];
     };
     auto stage = [&](int buf) {
+        v4u* A = smem + buf * (kA + kB);
 #pragma unroll
-        for (int i = 0; i < MG / 2; ++i) As[buf][tid + 256 * i] = sa[i];
+        for (int i = 0; i < SA; ++i) A[tid + TH * i] = sa[i];
 #pragma unroll
-        for (int i = 0; i < WN; ++i) Bs[buf][(wave * WN + i) * 64 + lane] = unpack_dword(sc[i]);
+        for (int i = 0; i < SB; ++i) A[kA + (wave * SB + i) * 64 + lane] = unpack_dword(sc[i]);
     };
     v4f acc[4][4], tot[4][4];
     const v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -688,31 +698,33 @@ __global__ __launch_bounds__(256, 2) void wide_gemm_kernel(BatchGemm a, uint32_t
 #pragma unroll
         for (int n = 0; n < 4; ++n) acc[m][n] = tot[m][n] = zero;
 
-    const uint32_t last = b1 - 1;
     load(b0);
     load_d(b0);
     stage(0);
-    load(min(b0 + 1, last));
+    load(b0 + WK);
     __syncthreads();
-    for (uint32_t b = b0; b < b1; ++b) {
-        const int buf = (b - b0) & 1;
+    uint32_t step = 0;
+    for (uint32_t b = b0; b < b1; b += WK, ++step) {
+        const v4u* A = smem + (step & 1) * (kA + kB);
+        const v4u* B = A + kA + wk * NT * 64;
+        A += wk * MG * 128;
         float d[4];
 #pragma unroll
         for (int n = 0; n < 4; ++n) {
-            d[n] = h2f(dn[n]);
+            d[n] = WK == 1 || b + wk < b1 ? h2f(dn[n]) : 0.0f;
             asm("" : "+v"(d[n]));  // (converted once: as a mixed-precision operand of 64 FMAs it takes 1.5 % longer)
         }
         v8h ah[4], al[4], bw[4];
 #pragma unroll
         for (int m = 0; m < 4; ++m) {
-            ah[m] = __builtin_bit_cast(v8h, As[buf][(wm * 4 + m) * 128 + lane]);
-            al[m] = __builtin_bit_cast(v8h, As[buf][(wm * 4 + m) * 128 + 64 + lane]);
+            ah[m] = __builtin_bit_cast(v8h, A[(wm * 4 + m) * 128 + lane]);
+            al[m] = __builtin_bit_cast(v8h, A[(wm * 4 + m) * 128 + 64 + lane]);
         }
 #pragma unroll
-        for (int n = 0; n < 4; ++n) bw[n] = __builtin_bit_cast(v8h, Bs[buf][(wn * 4 + n) * 64 + lane]);
-        stage(buf ^ 1);
-        load(min(b + 2, last));
-        load_d(min(b + 1, last));
+        for (int n = 0; n < 4; ++n) bw[n] = __builtin_bit_cast(v8h, B[(wn * 4 + n) * 64 + lane]);
+        stage((step & 1) ^ 1);
+        load(b + 2 * WK);
+        load_d(b + WK);
 #pragma unroll
         for (int n = 0; n < 4; ++n) {
             v4f D[4];
@@ -725,7 +737,7 @@ __global__ __launch_bounds__(256, 2) void wide_gemm_kernel(BatchGemm a, uint32_t
 #pragma unroll
                 for (int e = 0; e < 4; ++e) acc[m][n][e] = fmaf(d[n], D[m][e], acc[m][n][e]);
         }
-        if (((b - b0) & (kWideChain - 1)) == kWideChain - 1) {
+        if ((step & (kWideChain - 1)) == kWideChain - 1) {
 #pragma unroll
             for (int m = 0; m < 4; ++m)
 #pragma unroll
@@ -736,11 +748,37 @@ __global__ __launch_bounds__(256, 2) void wide_gemm_kernel(BatchGemm a, uint32_t
         }
         __syncthreads();
     }
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+        for (int n = 0; n < 4; ++n) tot[m][n] += acc[m][n];
 
-    // lane: rows r of its tiles, tokens 4 q + e of its groups
+    // lane: rows r of its tiles, tokens 4 q + e of its groups.  The WK waves of a tile exchange their sums
+    // through LDS, each adding and writing 4 / WK of the token groups.
+    if constexpr (WK > 1) {
+        v4f* X = reinterpret_cast<v4f*>(smem);
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+#pragma unroll
+            for (int n = 0; n < 4; ++n) X[(wave * 16 + m * 4 + n) * 64 + lane] = tot[m][n];
+        __syncthreads();
+    }
     const float* inv = reinterpret_cast<const float*>(a.img + (size_t)nb * G * 2048);
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
+    for (int mi = 0; mi < 4 / WK; ++mi) {
+        const uint32_t m = wk * (4 / WK) + mi;
+        v4f t4[4];
+#pragma unroll
+        for (int n = 0; n < 4; ++n) {
+            if constexpr (WK == 1) {
+                t4[n] = tot[mi][n];
+            } else {
+                const v4f* X = reinterpret_cast<const v4f*>(smem);
+                t4[n] = X[((wave % (WM * WN)) * 16 + m * 4 + n) * 64 + lane];
+#pragma unroll
+                for (int k = 1; k < WK; ++k) t4[n] += X[((wave % (WM * WN) + k * WM * WN) * 16 + m * 4 + n) * 64 + lane];
+            }
+        }
         const uint32_t t0 = (mt0 * MG + wm * 4 + m) * 16 + 4 * q;
         const v4f s = *gp(reinterpret_cast<const v4f*>(inv + t0));
 #pragma unroll
@@ -750,10 +788,9 @@ __global__ __launch_bounds__(256, 2) void wide_gemm_kernel(BatchGemm a, uint32_t
             for (int e = 0; e < 4; ++e) {
                 const uint32_t t = t0 + e;
                 if (t >= a.T || row >= a.w.rows) continue;
-                const float v = (tot[m][n][e] + acc[m][n][e]) * s[e];
+                const float v = t4[n][e] * s[e];
                 if constexpr (P == 2) {
-                    const float u = (tot[m][n + 1][e] + acc[m][n + 1][e]) * s[e];
-                    a.y[(size_t)t * a.y_stride + row] = gelu_mul(v, u);
+                    a.y[(size_t)t * a.y_stride + row] = gelu_mul(v, t4[n + 1][e] * s[e]);
                 } else if (S > 1) {
                     a.part[((size_t)split * G * 16 + t) * (tiles * 16) + row] = v;
                 } else {
@@ -1228,12 +1265,36 @@ uint32_t batch_padded(uint32_t tokens) {
     return tokens > kBatchMax ? 16 * wide_groups(tokens) : padded_tokens(tokens);
 }
 
-// K splits of a wide GEMM: about 512 workgroups (two per CU), each with at least kWideChain blocks;
-// a gate/up pair is not split (its epilogue needs whole sums; its grid is large anyway).
-static uint32_t wide_splits(uint32_t rows, uint32_t blocks, uint32_t tokens, bool pair) {
-    if (pair) return 1;
-    const uint32_t m = wide_tokens(tokens), items = (rows + 16383 / m) / (16384 / m) * ((tokens + m - 1) / m);
-    return std::max<uint32_t>(1, std::min({(512 + items / 2) / items, kDeferParts, blocks / kWideChain}));
+// Work split of a wide GEMM: 64 or 128 tokens x 128 rows per workgroup, wk waves sharing K inside it, S
+// splits of K over workgroups (their sums added by the next kernel), S rounded down so that one round of
+// workgroups holds them all (270 workgroups on 256 places took 82 us, 240 took 47).
+// - 64 tokens: eight waves, four along K: a CU's 240 places hold a 15360-row gate/up pair once, and four waves
+//   in one place leave it waiting (3840 -> 2 x 15360: 50 us against 113 with four waves of 64 x 256).
+// - 128 tokens: eight waves, two along K, one workgroup per CU; or four waves, none along K, two workgroups
+//   per CU, which hide each other's barriers but need twice the splits.  The latter for grids of several
+//   rounds (512 tokens, the pair: 286 us against 323) and where they fill the places better; equal, the
+//   former, whose splits are fewer or none (128 tokens, 4096 -> 3840: 21.6 us against 25.5; 512 tokens, qkv:
+//   no partial sums), but for two or three splits (512 tokens, 15360 -> 3840: 145 us against 155).
+// A gate/up pair is not split (its epilogue needs whole sums).
+struct WidePlan {
+    uint32_t wk, mtiles, groups, S;
+};
+static WidePlan wide_plan(uint32_t rows, uint32_t blocks, uint32_t tokens, bool pair) {
+    constexpr uint32_t kCus = 256, kRounds = 384;
+    const uint32_t m = wide_tokens(tokens), mtiles = (tokens + m - 1) / m, vrows = pair ? (rows + 31) / 32 * 64 : rows;
+    const uint32_t groups = (vrows + 127) / 128, items = mtiles * groups;
+    const auto splits = [&](uint32_t wk, uint32_t places) {
+        return pair ? 1u : std::max<uint32_t>(1, std::min({places / items, kDeferParts, blocks / (kWideChain * wk)}));
+    };
+    const auto used = [&](uint32_t S, uint32_t places) {  // share of the places of the rounds it takes
+        const uint32_t n = items * S;
+        return (double)n / ((n + places - 1) / places * places);
+    };
+    if (m == 64) return WidePlan{4, mtiles, groups, splits(4, kCus)};
+    const uint32_t S1 = splits(1, 2 * kCus), S2 = splits(2, kCus);
+    const double u1 = used(S1, 2 * kCus), u2 = used(S2, kCus);
+    const bool two = items < kRounds && (u2 > u1 + 0.02 || (u2 > u1 - 0.02 && S2 != 2 && S2 != 3));
+    return WidePlan{two ? 2u : 1u, mtiles, groups, two ? S2 : S1};
 }
 
 size_t batch_image_bytes(uint32_t blocks, uint32_t tokens) {
@@ -1249,7 +1310,7 @@ size_t batch_gemm_part_bytes(uint32_t rows, uint32_t blocks, uint32_t tokens, bo
         if (S > 1) most = std::max(most, (size_t)S * (gelu_pair ? 2 : 1) * padded_tokens(T) * prow * 4);
     }
     for (uint32_t t = 64; t < tokens + 64 && tokens > kBatchMax; t += 64) {
-        const uint32_t T = std::min(t, tokens), S = wide_splits(rows, blocks, T, gelu_pair);
+        const uint32_t T = std::min(t, tokens), S = wide_plan(rows, blocks, T, gelu_pair).S;
         if (S > 1) most = std::max(most, (size_t)S * 16 * wide_groups(T) * prow * 4);
     }
     return most;
@@ -1343,13 +1404,13 @@ static hipError_t gemm_launch(const BatchGemm& a, hipStream_t s, uint32_t* parts
 
 template <int P>
 static hipError_t wide_launch(const BatchGemm& a, hipStream_t s, uint32_t* parts) {
-    const uint32_t m = wide_tokens(a.T), rows_wg = 16384 / m / P;  // (rows of each matrix)
-    const uint32_t mtiles = (a.T + m - 1) / m, ngroups = (a.w.rows + rows_wg - 1) / rows_wg;
-    const uint32_t S = wide_splits(a.w.rows, a.w.blocks, a.T, P == 2);
+    const WidePlan p = wide_plan(a.w.rows, a.w.blocks, a.T, P == 2);
+    const uint32_t S = p.S;
     if (S > 1 && !a.part) return hipErrorInvalidValue;
-    const dim3 grid((mtiles * ngroups * S + 7) / 8 * 8);
-    if (m == 128) hipLaunchKernelGGL((wide_gemm_kernel<2, P>), grid, dim3(256), 0, s, a, S, mtiles, ngroups);
-    else hipLaunchKernelGGL((wide_gemm_kernel<1, P>), grid, dim3(256), 0, s, a, S, mtiles, ngroups);
+    const dim3 grid((p.mtiles * p.groups * S + 7) / 8 * 8);
+    if (p.wk == 4) hipLaunchKernelGGL((wide_gemm_kernel<1, 2, 4, P>), grid, dim3(512), 0, s, a, S, p.mtiles, p.groups);
+    else if (p.wk == 2) hipLaunchKernelGGL((wide_gemm_kernel<2, 2, 2, P>), grid, dim3(512), 0, s, a, S, p.mtiles, p.groups);
+    else hipLaunchKernelGGL((wide_gemm_kernel<2, 2, 1, P>), grid, dim3(256), 0, s, a, S, p.mtiles, p.groups);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess || S == 1) return e;
     if (a.defer) {

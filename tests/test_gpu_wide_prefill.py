@@ -15,9 +15,9 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("q_heads,kv_heads,window,intermediate,n,batch", [
     (16, 8, 16, 2048, 33, 33),     # one 64-token tile, nearly half padding
     (16, 8, 100, 2080, 64, 64),    # a full 64-token tile; FFN rows and columns off every tile
-    (8, 8, 24, 1056, 150, 65),     # a 128-token tile, then one that ends a pass of 65 + 65 + 20
+    (8, 8, 24, 1056, 150, 65),     # 128-token tiles, nearly half padding; passes of 65 + 65 + 20
     (16, 4, 64, 2048, 280, 128),   # full 128-token tiles; two passes and a narrow remainder
-    (16, 8, 40, 2080, 330, 161),   # three 64-token tiles; the window's ring wraps inside the pass
+    (16, 8, 40, 2080, 330, 161),   # two 128-token tiles, the second mostly padding; the ring wraps inside the pass
     (16, 8, 1024, 2048, 530, 512), # the largest pass, then a narrow one
 ])
 def test_wide_trace_teacher_forced(q_heads, kv_heads, window, intermediate, n, batch):
