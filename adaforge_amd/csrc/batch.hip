@@ -618,9 +618,8 @@ __global__ __launch_bounds__(256) void batch_reduce_kernel(BatchGemm a, uint32_t
 // y[t][r] = sum_b d_rb sum_j (n_rbj - 8) x_tbj for more than kBatchMax tokens.  A workgroup takes M = 64 WM
 // tokens x 64 WN rows over K range `split`, WM x WN waves of 64 x 64 (4 x 4 MFMA tiles) for each of WK
 // 32-weight blocks (one MFMA depth) per step: the tokens' halves are copied from the image, which
-// is laid out as the MFMAs read it, and the weights unpacked once per workgroup, both into LDS,
-// double buffered; step s + 1's are written while step s is multiplied, and step s + 2's loads are
-// in flight.  The WK waves of a tile add their sums in LDS at the end.  The block's d_rb differs from the next one's, so each block's 16 x 16
+// is laid out as the MFMAs read it, by LDS DMA two steps ahead, and the weights unpacked once per
+// workgroup into LDS while the step before is multiplied.  The WK waves of a tile add their sums in LDS at the end.  The block's d_rb differs from the next one's, so each block's 16 x 16
 // products are folded into fp32 sums on their own (one FMA per product and lane: half as many VALU
 // cycles as the two MFMAs take; the token's scale waits for the epilogue, so that the fold has no other
 // factor).  Sums run over kWideChain blocks, then join a total, so that no chain of fp32 additions is
@@ -630,6 +629,7 @@ __global__ __launch_bounds__(256) void batch_reduce_kernel(BatchGemm a, uint32_t
 // shares (workgroup b runs on XCD b % 8), so that the workgroups that unpack the same weights share
 // an L2.
 constexpr uint32_t kWideChain = 8;
+typedef __attribute__((address_space(3))) void* lds_ptr;
 
 template <int WM, int WN, int WK, int P>
 __global__ __launch_bounds__(64 * WM * WN * WK, 2 / WK ? 2 / WK : 1) void wide_gemm_kernel(BatchGemm a, uint32_t S, uint32_t mtiles, uint32_t ngroups) {
@@ -637,8 +637,12 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2 / WK ? 2 / WK : 1) void wide_g
     constexpr int W = WM * WN * WK, TH = 64 * W;  // waves, threads
     constexpr int SA = 8 / WN, SB = 4 / WM;       // 16-byte pieces of the image and code dwords per thread and step
     constexpr int kA = MG * 128 * WK, kB = NT * 64 * WK;  // v4u per stage
-    __shared__ v4u smem[WK > 1 && W * 1024 > 2 * (kA + kB) ? W * 1024 : 2 * (kA + kB)];
-    // stage buf: [block of the step][token group][hi, lo][64 lanes], then [block][row tile][64 lanes]
+    constexpr int NA = WK == 4 ? 2 : 3;           // image stages (three of the 64-token form would fill the LDS)
+    constexpr int kAll = NA * kA + 2 * kB;
+    static_assert(WK == 1 || W * 1024 <= kAll, "the waves' sums fit the stages");
+    // NA image stages [block of the step][token group][hi, lo][64 lanes], two weight stages [block][row
+    // tile][64 lanes]
+    __shared__ v4u smem[kAll];
     const uint32_t tid = threadIdx.x, lane = tid & 63, wave = wave_id(), r = lane & 15, q = lane >> 4;
     const uint32_t wk = wave / (WM * WN), wm = wave / WN % WM, wn = wave % WN;
     const uint32_t total = mtiles * ngroups * S, per = gridDim.x / 8;
@@ -654,7 +658,6 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2 / WK ? 2 / WK : 1) void wide_g
 
     // this thread's share of a step: image pieces tid + TH i of its WK blocks (kA / WK per block), and the code
     // dwords of row tiles wave SB + i (of block (wave SB + i) / NT)
-    v4u sa[SA];
     uint32_t sc[SB];
     uint16_t dn[4];  // the next step's scales of the lane's rows
     const uint8_t* cp[SB];
@@ -670,12 +673,16 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2 / WK ? 2 / WK : 1) void wide_g
         dp[i] = mat_of(k).scales + (size_t)min(tile_of(k), tiles - 1) * a.w.nst * 64 + r;
     }
     const v4u* img = reinterpret_cast<const v4u*>(a.img) + (size_t)mt0 * MG * 128;
-    auto load = [&](uint32_t b) {  // (blocks past the range repeat its last one; their scales are zeroed)
+    // (blocks past the range repeat its last one; their scales are zeroed)
+    auto copy = [&](uint32_t b, int st) {  // the image's pieces straight into stage st
 #pragma unroll
         for (int i = 0; i < SA; ++i) {
             const uint32_t e = tid + TH * i;
-            sa[i] = *gp(img + (size_t)min(b + e / (MG * 128), last) * G * 128 + e % (MG * 128));
+            __builtin_amdgcn_global_load_lds(img + (size_t)min(b + e / (MG * 128), last) * G * 128 + e % (MG * 128),
+                                             (lds_ptr)(smem + st * kA + wave * 64 + TH * i), 16, 0, 0);
         }
+    };
+    auto load = [&](uint32_t b) {
 #pragma unroll
         for (int i = 0; i < SB; ++i)
             sc[i] = *gp(reinterpret_cast<const uint32_t*>(cp[i] + (size_t)min(b + (wave * SB + i) / NT, last) * 256));
@@ -684,12 +691,11 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2 / WK ? 2 / WK : 1) void wide_g
 #pragma unroll
         for (int i = 0; i < 4; ++i) dn[i] = gp(dp[i])[(size_t)min(b + wk, last) * 16];
     };
-    auto stage = [&](int buf) {
-        v4u* A = smem + buf * (kA + kB);
+    const uint32_t lds = (uint32_t)(uintptr_t)(lds_ptr)smem;
+    auto unpack = [&](int st) {  // (a store that the compiler sees would also wait for every copy in flight)
+        const uint32_t at = lds + 16 * (NA * kA + st * kB + wave * SB * 64 + lane);
 #pragma unroll
-        for (int i = 0; i < SA; ++i) A[tid + TH * i] = sa[i];
-#pragma unroll
-        for (int i = 0; i < SB; ++i) A[kA + (wave * SB + i) * 64 + lane] = unpack_dword(sc[i]);
+        for (int i = 0; i < SB; ++i) asm volatile("ds_write_b128 %0, %1 offset:%2" ::"v"(at), "v"(unpack_dword(sc[i])), "n"(1024 * i) : "memory");
     };
     v4f acc[4][4], tot[4][4];
     const v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
@@ -700,31 +706,62 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2 / WK ? 2 / WK : 1) void wide_g
 
     load(b0);
     load_d(b0);
-    stage(0);
+    unpack(0);
     load(b0 + WK);
-    __syncthreads();
-    uint32_t step = 0;
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int st = 0; st < NA - 1; ++st) copy(b0 + st * WK, st);
+    __builtin_amdgcn_sched_barrier(0);
+    uint32_t step = 0, sa = 0;  // step % NA
     for (uint32_t b = b0; b < b1; b += WK, ++step) {
-        const v4u* A = smem + (step & 1) * (kA + kB);
-        const v4u* B = A + kA + wk * NT * 64;
-        A += wk * MG * 128;
+        // This step's copies are in (with three stages, all but the SA newest requests: the copies for the
+        // next step are the last ones of an iteration) and its weights written, in every wave; every wave
+        // has read the stages that are written below.
+        if constexpr (NA == 3) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(SA) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        // The operands are read and waited for in one block: the compiler would wait for every copy in
+        // flight before an LDS read that it sees.
+        v4u ahu[4], alu[4], bwu[4];
+        const uint32_t pa = lds + 16 * (sa * kA + wk * MG * 128 + wm * 512 + lane),
+                       pb = lds + 16 * (NA * kA + (step & 1) * kB + wk * NT * 64 + wn * 256 + lane);
+        asm volatile(
+            "ds_read_b128 %8, %13\n\t"
+            "ds_read_b128 %0, %12\n\t"
+            "ds_read_b128 %1, %12 offset:2048\n\t"
+            "ds_read_b128 %2, %12 offset:4096\n\t"
+            "ds_read_b128 %3, %12 offset:6144\n\t"
+            "ds_read_b128 %4, %12 offset:1024\n\t"
+            "ds_read_b128 %5, %12 offset:3072\n\t"
+            "ds_read_b128 %6, %12 offset:5120\n\t"
+            "ds_read_b128 %7, %12 offset:7168\n\t"
+            "ds_read_b128 %9, %13 offset:1024\n\t"
+            "ds_read_b128 %10, %13 offset:2048\n\t"
+            "ds_read_b128 %11, %13 offset:3072\n\t"
+            "s_waitcnt lgkmcnt(0)"
+            : "=&v"(ahu[0]), "=&v"(ahu[1]), "=&v"(ahu[2]), "=&v"(ahu[3]), "=&v"(alu[0]), "=&v"(alu[1]), "=&v"(alu[2]),
+              "=&v"(alu[3]), "=&v"(bwu[0]), "=&v"(bwu[1]), "=&v"(bwu[2]), "=&v"(bwu[3])
+            : "v"(pa), "v"(pb)
+            : "memory");
+        v8h ah[4], al[4], bw[4];
+#pragma unroll
+        for (int m = 0; m < 4; ++m) {
+            ah[m] = __builtin_bit_cast(v8h, ahu[m]);
+            al[m] = __builtin_bit_cast(v8h, alu[m]);
+            bw[m] = __builtin_bit_cast(v8h, bwu[m]);
+        }
         float d[4];
 #pragma unroll
         for (int n = 0; n < 4; ++n) {
             d[n] = WK == 1 || b + wk < b1 ? h2f(dn[n]) : 0.0f;
             asm("" : "+v"(d[n]));  // (converted once: as a mixed-precision operand of 64 FMAs it takes 1.5 % longer)
         }
-        v8h ah[4], al[4], bw[4];
-#pragma unroll
-        for (int m = 0; m < 4; ++m) {
-            ah[m] = __builtin_bit_cast(v8h, A[(wm * 4 + m) * 128 + lane]);
-            al[m] = __builtin_bit_cast(v8h, A[(wm * 4 + m) * 128 + 64 + lane]);
-        }
-#pragma unroll
-        for (int n = 0; n < 4; ++n) bw[n] = __builtin_bit_cast(v8h, B[(wn * 4 + n) * 64 + lane]);
-        stage((step & 1) ^ 1);
+        unpack((step & 1) ^ 1);
         load(b + 2 * WK);
         load_d(b + WK);
+        __builtin_amdgcn_sched_barrier(0);
+        copy(b + (NA - 1) * WK, sa ? sa - 1 : NA - 1);
+        __builtin_amdgcn_sched_barrier(0);
+        sa = sa == NA - 1 ? 0 : sa + 1;
 #pragma unroll
         for (int n = 0; n < 4; ++n) {
             v4f D[4];
@@ -746,8 +783,8 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2 / WK ? 2 / WK : 1) void wide_g
                     acc[m][n] = zero;
                 }
         }
-        __syncthreads();
     }
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // no copy outlives its LDS
 #pragma unroll
     for (int m = 0; m < 4; ++m)
 #pragma unroll
@@ -756,6 +793,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2 / WK ? 2 / WK : 1) void wide_g
     // lane: rows r of its tiles, tokens 4 q + e of its groups.  The WK waves of a tile exchange their sums
     // through LDS, each adding and writing 4 / WK of the token groups.
     if constexpr (WK > 1) {
+        __syncthreads();  // (every wave's last operands are read and its copies in)
         v4f* X = reinterpret_cast<v4f*>(smem);
 #pragma unroll
         for (int m = 0; m < 4; ++m)
