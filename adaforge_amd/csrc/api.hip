@@ -794,7 +794,10 @@ int af_attention_decode(const af_attention_args* p, void* stream) {
     const uint32_t cmax = mfma ? attention_mfma_chunks(p->config.kv_heads, nvis) : kAttnMaxChunks;
     const bool xl = attn_xcd_local();
     std::lock_guard<std::mutex> lock(g_scratch.mu);
-    if ((rc = grow(g_scratch.attn_part, (size_t)p->config.kv_heads * cmax * group * attn_part_row(D) * 4, false, "attention scratch")))
+    // (for the heads' longest range, whatever this call's: a call at a later position allocates nothing)
+    constexpr uint32_t kSpan = kAttnMaxChunks * kAttnMaxChunkLen;
+    const uint32_t most = std::max(kAttnMaxChunks, attention_mfma(group, D, kSpan) ? attention_mfma_chunks(p->config.kv_heads, kSpan) : 0u);
+    if ((rc = grow(g_scratch.attn_part, (size_t)p->config.kv_heads * most * group * attn_part_row(D) * 4, false, "attention scratch")))
         return rc;
     if ((rc = grow(g_scratch.attn_counters, (size_t)std::max<uint32_t>(64, p->config.q_heads) * 4, true,
                    "attention counters")))

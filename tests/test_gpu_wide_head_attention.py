@@ -4,6 +4,7 @@ import ctypes
 
 import numpy as np
 import pytest
+import torch
 
 import oracle
 from adaforge_amd import _native as N, hip, synth
@@ -18,6 +19,24 @@ def rope(x, heads, factors, pos):
 
 def normed(w, x):
     return oracle.rmsnorm(w, 1e-6, x).astype(np.float32)
+
+
+def test_late_call_allocates_nothing():
+    """The scratch of a shape's first call serves every later position, also past the switch of kernels."""
+    q_heads, ring = 16, 16384
+    factors = synth.gemma4_rope_factors(W)
+    bufs = [hip.Buffer.from_numpy(np.ones(n * W, np.float32)) for n in (q_heads, 1, 1, 1, 1)]
+    cache = [hip.Buffer.from_numpy(np.zeros((ring, W), np.uint16)) for _ in range(2)]
+    out = hip.Buffer(q_heads * W)
+    free = []
+    for pos in (8, 16383):
+        args = N.AttentionArgs(*(b.ptr for b in bufs), 1e-6, 1e-6, 1e-6, 1,
+                               N.RopeDesc(W, 1e6, factors.ctypes.data_as(N.f32p), 131072),
+                               N.AttentionConfigDesc(q_heads, 1, W, 0, 1.0), cache[0].ptr, cache[1].ptr, ring, pos, out.ptr)
+        N.check(N.lib().af_attention_decode(ctypes.byref(args), None))
+        hip.synchronize()
+        free.append(torch.cuda.mem_get_info()[0])
+    assert free[0] == free[1]
 
 
 @pytest.mark.parametrize("context,window,q_heads,kv_heads,scale", [
