@@ -660,36 +660,42 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2 / WK ? 2 / WK : 1) void wide_g
     // dwords of row tiles wave SB + i (of block (wave SB + i) / NT)
     uint32_t sc[SB];
     uint16_t dn[4];  // the next step's scales of the lane's rows
-    const uint8_t* cp[SB];
-    const uint16_t* dp[4];
+    // (every request is a buffer's base, the thread's constant offset and the block's scalar one: 64-bit
+    // addresses per request took a third of the loop's VALU cycles)
+    __amdgpu_buffer_rsrc_t rc[SB], rd[4];
 #pragma unroll
     for (int i = 0; i < SB; ++i) {
         const uint32_t k = (wave * SB + i) % NT;
-        cp[i] = mat_of(k).codes + (size_t)min(tile_of(k), tiles - 1) * a.w.nst * 1024 + r * 16 + q * 4;
+        const uint8_t* p = mat_of(k).codes + (size_t)min(tile_of(k), tiles - 1) * a.w.nst * 1024;
+        rc[i] = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(p), 0, a.w.nst * 1024, 0x00020000);
     }
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const uint32_t k = wn * 4 + i;
-        dp[i] = mat_of(k).scales + (size_t)min(tile_of(k), tiles - 1) * a.w.nst * 64 + r;
+        const uint16_t* p = mat_of(k).scales + (size_t)min(tile_of(k), tiles - 1) * a.w.nst * 64;
+        rd[i] = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p), 0, a.w.nst * 128, 0x00020000);
     }
-    const v4u* img = reinterpret_cast<const v4u*>(a.img) + (size_t)mt0 * MG * 128;
+    const __amdgpu_buffer_rsrc_t ri =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<int8_t*>(reinterpret_cast<const int8_t*>(a.img)), 0, nb * G * 2048, 0x00020000);
     // (blocks past the range repeat its last one; their scales are zeroed)
     auto copy = [&](uint32_t b, int st) {  // the image's pieces straight into stage st
 #pragma unroll
         for (int i = 0; i < SA; ++i) {
-            const uint32_t e = tid + TH * i;
-            __builtin_amdgcn_global_load_lds(img + (size_t)min(b + e / (MG * 128), last) * G * 128 + e % (MG * 128),
-                                             (lds_ptr)(smem + st * kA + wave * 64 + TH * i), 16, 0, 0);
+            // (piece tid + TH i lies in block TH i / (MG 128) for every thread)
+            static_assert((MG * 128) % TH == 0, "a block is whole rounds of the threads");
+            const uint32_t blk = min(b + TH * i / (MG * 128), last);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(ri, (lds_ptr)(smem + st * kA + wave * 64 + TH * i), 16, tid * 16,
+                                                     (blk * G + mt0 * MG) * 2048 + TH * i % (MG * 128) * 16, 0, 0);
         }
     };
     auto load = [&](uint32_t b) {
 #pragma unroll
         for (int i = 0; i < SB; ++i)
-            sc[i] = *gp(reinterpret_cast<const uint32_t*>(cp[i] + (size_t)min(b + (wave * SB + i) / NT, last) * 256));
+            sc[i] = __builtin_amdgcn_raw_buffer_load_b32(rc[i], r * 16 + q * 4, min(b + (wave * SB + i) / NT, last) * 256, 0);
     };
     auto load_d = [&](uint32_t b) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) dn[i] = gp(dp[i])[(size_t)min(b + wk, last) * 16];
+        for (int i = 0; i < 4; ++i) dn[i] = __builtin_amdgcn_raw_buffer_load_b16(rd[i], r * 2, min(b + wk, last) * 32, 0);
     };
     const uint32_t lds = (uint32_t)(uintptr_t)(lds_ptr)smem;
     auto unpack = [&](int st) {  // (a store that the compiler sees would also wait for every copy in flight)
