@@ -7,7 +7,7 @@
 // wide_attention_kernel, after a pass that appends every token's K and V).  Above kBatchMax tokens a
 // pass is bound by its products, which the wide kernels share out like any large matrix product; up to
 // it by the weight stream.  512 tokens through six layers of the 12B shape: 14.3 ms in 16 passes of 32,
-// 5.3 ms in one.
+// 4.86 ms in one.
 //
 // Up to kBatchMax tokens each token's GEMM input is written as two fp16 halves per 32-element block: with u the block
 // scaled by 2^(14 - e) (e = ilogb of the block's max |x|, so that |u| < 2^15), hi = fp16(u) and
