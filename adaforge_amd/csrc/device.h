@@ -140,6 +140,49 @@ __device__ __forceinline__ float row_total(float v) {
     return __uint_as_float(q[0]) + __uint_as_float(q[1]);
 }
 
+// Softmax attention of one query over keys [lo, hi) by one wave, key by key in fp32: what an attention on the
+// matrix cores falls back to when a sum of its own is not finite.  There an infinite cached value (an
+// overflow of fp16) meets halves that are zero or of the other sign, also of keys that the query does not see;
+// here a key of score -inf has weight 0 and an infinite value stays in its channel.  Lane: channels 256 g +
+// 4 lane + k at 4 g + k; krow(key), vrow(key): the key's rows.  A NaN sum ends the loop (every output is one).
+template <int D, class K, class V>
+__device__ __forceinline__ void plain_attention(const float (&q)[D / 64], float scale, uint32_t lo, uint32_t hi, K krow,
+                                                V vrow, float (&acc)[D / 64], float& m, float& l) {
+    const uint32_t lane = threadIdx.x & 63;
+    auto row = [&](const uint16_t* p, float (&o)[D / 64]) {
+#pragma unroll
+        for (int g = 0; g < D / 256; ++g) {
+            const uint2 w = *reinterpret_cast<const uint2*>(p + 256 * g + 4 * lane);
+            o[4 * g] = h2f((uint16_t)w.x);
+            o[4 * g + 1] = h2f((uint16_t)(w.x >> 16));
+            o[4 * g + 2] = h2f((uint16_t)w.y);
+            o[4 * g + 3] = h2f((uint16_t)(w.y >> 16));
+        }
+    };
+#pragma unroll
+    for (int e = 0; e < D / 64; ++e) acc[e] = 0.0f;
+    m = -INFINITY;
+    l = 0.0f;
+#pragma unroll 1
+    for (uint32_t key = lo; key < hi; ++key) {
+        float v[D / 64], d = 0.0f;
+        row(krow(key), v);
+#pragma unroll
+        for (int e = 0; e < D / 64; ++e) d = fmaf(q[e], v[e], d);
+        const float s = wave_sum(d) * scale, mn = fmaxf(m, s);
+        const float p = s == -INFINITY ? 0.0f : expf(s - mn), al = mn == -INFINITY ? 1.0f : expf(m - mn);
+        l = fmaf(l, al, p);
+        row(vrow(key), v);
+#pragma unroll
+        for (int e = 0; e < D / 64; ++e) acc[e] = fmaf(p, v[e], acc[e] * al);
+        m = mn;
+        if (l != l) {
+            m = 0.0f;  // (a maximum of -inf would drop the sums where partials are merged)
+            break;
+        }
+    }
+}
+
 // f32(x * r * w) with the products in double, as the FP64 RMSNorm oracle rounds its output.
 __device__ __forceinline__ float norm_apply(float x, double r, float w) {
     return (float)__dmul_rn(__dmul_rn((double)x, r), (double)w);

@@ -1408,7 +1408,11 @@ __global__ __launch_bounds__(D) void attention_kernel(AttnArgs a) {
 // workgroup per query head and 128 channels: 64 chunks of 16 heads are 2 MB, which one last
 // workgroup would read for longer than another launch takes.
 //
-// 16 query heads on one KV head: 16.7 us against 31.1 at 4,096 positions, 28.4 against 87.4 at 32,768 (of
+// Infinities (fp16 overflows of cached rows) meet low halves of zero or of the other sign, so a wave whose sums
+// are not finite takes its channels again key by key in fp32 (plain_attention), as attention_kernel computes
+// them; the check is 33 FMAs and a ballot per wave (16.7 -> 16.9 us at 4,096 positions, a barrier more 17.3).
+//
+// 16 query heads on one KV head: 16.9 us against 31.1 at 4,096 positions, 28.4 against 87.4 at 32,768 (of
 // them 4.8 us the merge, 3 us the loop at 4,096, the rest the launch and the prologue's chain).  Error
 // against 64 bits 2.1e-7 at 4,096 (attention_kernel: 2.2e-7).
 // Keys per chunk (a multiple of 64) and chunks of n visible keys in at most cmax chunks.
@@ -1590,7 +1594,7 @@ __global__ __launch_bounds__(256) void attention_mfma_kernel(AttnArgs a) {
         if (q == 0) wmax[wave][m] = mx;
         __syncthreads();
         const float mn = fmaxf(fmaxf(mrun, fmaxf(wmax[0][m], wmax[1][m])), fmaxf(wmax[2][m], wmax[3][m]));
-        const float al = expf(mrun - mn);  // (key k0 is visible: mn is finite)
+        const float al = expf(mrun - mn);  // (key k0 is visible: mn is finite, or the sums end as NaN)
         float sum = 0.0f;
         h4 hi, lo;
 #pragma unroll
@@ -1635,11 +1639,50 @@ __global__ __launch_bounds__(256) void attention_mfma_kernel(AttnArgs a) {
         }
         if (k0 + 64 < k_end) load_v(k0 + 64);
     }
-    if (m >= group) return;
+    float odd = lrun * 0.0f;  // NaN if a sum is not finite
 #pragma unroll
-    for (int e = 0; e < 8; ++e) acc[e] += accl[e];
+    for (int e = 0; e < 8; ++e) {
+        acc[e] += accl[e];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) odd = fmaf(acc[e][i], 0.0f, odd);
+    }
     constexpr uint32_t R = attn_part_row(D);
-    float* pr = a.part + (((size_t)h * a.cmax + c) * group + m) * R;
+    float* part = a.part + ((size_t)h * a.cmax + c) * group * R;
+    if (__any(odd != 0.0f)) {
+        // an infinity or NaN among the chunk's rows: this wave's channels again in fp32, relative to the
+        // other waves' maximum and sum unless those are not finite either (then in no wave)
+#pragma unroll 1
+        for (uint32_t hq = 0; hq < group; ++hq) {
+            float u[8], w[8], qf[8], o[8], mf, lf;
+            row8(a.q_raw + ((size_t)h * group + hq) * D, u);
+            row8(a.q_norm, w);
+            double v = 0.0;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) v += (double)u[k] * (double)u[k];
+            rotate(u, inv_rms_fast(wave_sum(v), D, a.q_eps), w, qf);
+            plain_attention<D>(
+                qf, a.scale, k_begin, k_end,
+                [&](uint32_t key) { return key == pos ? knew : kh + (size_t)(key % a.ring) * D; },
+                [&](uint32_t key) { return key == pos ? vnew : vh + (size_t)(key % a.ring) * D; }, o, mf, lf);
+            const float ms = __shfl(mrun, hq), ls = __shfl(lrun, hq);
+            if (ls * 0.0f == 0.0f) {
+#pragma unroll
+                for (int k = 0; k < 8; ++k) o[k] *= expf(mf - ms);
+                mf = ms;
+                lf = ls;
+            }
+            float* pr = part + hq * R;
+            if (lane / 32 == wave % 2) {
+                const int g = 4 * (wave / 2);
+                *reinterpret_cast<float4*>(pr + 64 * g + 4 * lane) =
+                    g ? make_float4(o[4], o[5], o[6], o[7]) : make_float4(o[0], o[1], o[2], o[3]);
+            }
+            if (wave == 0 && lane == 0) *reinterpret_cast<float2*>(pr + D) = make_float2(mf, lf);
+        }
+        return;
+    }
+    if (m >= group) return;
+    float* pr = part + m * R;
 #pragma unroll
     for (int i = 0; i < 4; ++i)
 #pragma unroll
@@ -1680,8 +1723,9 @@ __global__ __launch_bounds__(512) void attention_mfma_merge_kernel(AttnArgs a) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const uint32_t k = k0 + PH * u;
-            const float wk = k < chunks ? w[k] : 0.0f;
             if (k0 != phase) v[u] = *reinterpret_cast<const float4*>(base + min(k, chunks - 1) * step + ch);
+            if (k >= chunks) continue;  // (the last piece again, which may be infinite: not added with a weight of 0)
+            const float wk = w[k];
             s.x = fmaf(wk, v[u].x, s.x);
             s.y = fmaf(wk, v[u].y, s.y);
             s.z = fmaf(wk, v[u].z, s.z);

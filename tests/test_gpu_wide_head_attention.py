@@ -104,3 +104,56 @@ def test_session_past_the_threshold_matches_the_batched_layers():
             got.append(s.trace(ids[1040:], layer_outputs=False)[2])
     assert np.abs(got[0] - got[1]).max() <= 1e-3 * np.abs(got[1]).max()
     assert int(np.argmax(got[0])) == int(np.argmax(got[1]))
+
+
+def plain(q, k, v, scale):
+    """Softmax attention of one query in 64 bits; a key whose score is -inf has weight 0."""
+    with np.errstate(all="ignore"):
+        sc = (k.astype(np.float64) @ q.astype(np.float64)) * scale
+        p = np.exp(sc - sc.max())
+        p[sc == -np.inf] = 0.0
+        return p @ v.astype(np.float64) / p.sum()
+
+
+@pytest.mark.parametrize("context,q_heads,kv_heads", [(700, 8, 1), (1500, 4, 1), (1500, 16, 1), (2100, 16, 2)])
+@pytest.mark.parametrize("kind", ["key", "value", "new key"])
+def test_infinite_rows(kind, context, q_heads, kv_heads):
+    """The same meaning below and above the switch of kernels (1,024 positions): an infinite cached key
+    element gives its key weight 0 where the score is -inf (and NaN where it is +inf), an infinite cached value an
+    infinite output in its own channel alone."""
+    pos, group = context - 1, q_heads // kv_heads
+    rng = np.random.default_rng(context + q_heads)
+    q, k, v = (rng.standard_normal(h * W).astype(np.float32) for h in (q_heads, kv_heads, kv_heads))
+    qn, kn = (1 + 0.1 * rng.standard_normal((2, W))).astype(np.float32)
+    scale = 0.05
+    keys, values = rng.standard_normal((2, kv_heads, context, W)).astype(np.float16)
+    if kind == "key":
+        keys[0, [333, context - 70], 100] = np.inf
+        keys[-1, 334, 100] = -np.inf if kv_heads > 1 else np.inf
+    elif kind == "value":
+        values[:, 333, 3], values[:, context - 2, 200] = np.inf, -np.inf
+    else:
+        kn[120] = 1e7
+    factors = synth.gemma4_rope_factors(W)
+    bufs = [hip.Buffer.from_numpy(a) for a in (q, k, v, qn, kn, keys.view(np.uint16), values.view(np.uint16))]
+    out = hip.Buffer(q_heads * W)
+    args = N.AttentionArgs(*(b.ptr for b in bufs[:5]), 1e-6, 1e-6, 1e-6, 0,
+                           N.RopeDesc(W, 1e6, factors.ctypes.data_as(N.f32p), 131072),
+                           N.AttentionConfigDesc(q_heads, kv_heads, W, 0, scale), bufs[5].ptr, bufs[6].ptr, context, pos,
+                           out.ptr)
+    N.check(N.lib().af_attention_decode(ctypes.byref(args), None))
+    hip.synchronize()
+    got = out.numpy().reshape(q_heads, W)
+    keys, values = bufs[5].numpy().view(np.float16), bufs[6].numpy().view(np.float16)
+    if kind == "new key":
+        assert np.isinf(keys[:, pos]).any()
+    finite = 0
+    for h in range(q_heads):
+        qh = rope(normed(qn, q[h * W:(h + 1) * W]), 1, factors, pos)
+        ref = plain(qh, keys[h // group], values[h // group], scale)
+        assert np.array_equal(np.isnan(got[h]), np.isnan(ref)), (kind, h)
+        assert np.array_equal(np.isposinf(got[h]), np.isposinf(ref)) and np.array_equal(np.isneginf(got[h]), np.isneginf(ref))
+        ok = np.isfinite(ref)
+        finite += ok.sum()
+        oracle.compare(ref[ok], got[h][ok])
+    assert finite >= 16  # (by the seeds: in every case some heads, or channels, stay finite)
