@@ -917,7 +917,7 @@ __global__ __launch_bounds__(256) void batch_attention_kernel(BatchAttn a) {
             mx = fmaxf(mx, fabsf(v[j]));
         }
         mx = wave_max(mx);
-        const float s = mx > 0.0f ? ldexpf(1.0f, 4 - ilogbf(mx)) : 1.0f;  // |q s| < 32
+        const float s = query_scale(mx);  // |q s| < 32
 #pragma unroll
         for (int j = 0; j < D / 64; ++j) split_f16(v[j] * s, qh[r * KP + lane + 64 * j], ql[r * KP + lane + 64 * j]);
         if (lane == 0) qscale[r] = 1.0f / s;
@@ -1151,7 +1151,7 @@ __global__ __launch_bounds__(256, D == 256 ? 2 : 1) void wide_attention_kernel(B
                 for (int e = 0; e < 4; ++e) mx = fmaxf(mx, fabsf(v[s][k][e]));
             }
         mx = lanes4_max(mx);
-        const float s = mx > 0.0f ? ldexpf(1.0f, 4 - ilogbf(mx)) : 1.0f;  // |q s| < 32
+        const float s = query_scale(mx);  // |q s| < 32
 #pragma unroll
         for (int i = 0; i < DS; ++i)
 #pragma unroll

@@ -140,6 +140,12 @@ __device__ __forceinline__ float row_total(float v) {
     return __uint_as_float(q[0]) + __uint_as_float(q[1]);
 }
 
+// The power of two that brings a query whose largest element is mx below 32 (its fp16 halves' scale); at
+// most 2^126, so that it and its reciprocal are finite: a query below 2^-122 keeps smaller halves.
+__device__ __forceinline__ float query_scale(float mx) {
+    return mx > 0.0f ? ldexpf(1.0f, min(4 - ilogbf(mx), 126)) : 1.0f;
+}
+
 // Softmax attention of one query over keys [lo, hi) by one wave, key by key in fp32: what an attention on the
 // matrix cores falls back to when a sum of its own is not finite.  There an infinite cached value (an
 // overflow of fp16) meets halves that are zero or of the other sign, also of keys that the query does not see;

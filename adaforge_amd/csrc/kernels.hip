@@ -1525,7 +1525,7 @@ __global__ __launch_bounds__(256) void attention_mfma_kernel(AttnArgs a) {
             mx = fmaxf(mx, fabsf(o[k]));
         }
         mx = wave_max(mx);
-        const float s = mx > 0.0f ? ldexpf(1.0f, 4 - ilogbf(mx)) : 1.0f;  // |q s| < 32
+        const float s = query_scale(mx);  // |q s| < 32
 #pragma unroll
         for (int k = 0; k < 8; k += 4) {
             h4 hi, lo;

@@ -116,11 +116,11 @@ def plain(q, k, v, scale):
 
 
 @pytest.mark.parametrize("context,q_heads,kv_heads", [(700, 8, 1), (1500, 4, 1), (1500, 16, 1), (2100, 16, 2)])
-@pytest.mark.parametrize("kind", ["key", "value", "new key"])
-def test_infinite_rows(kind, context, q_heads, kv_heads):
+@pytest.mark.parametrize("kind", ["key", "value", "new key", "tiny query", "huge query"])
+def test_infinite_rows_and_extreme_queries(kind, context, q_heads, kv_heads):
     """The same meaning below and above the switch of kernels (1,024 positions): an infinite cached key
     element gives its key weight 0 where the score is -inf (and NaN where it is +inf), an infinite cached value an
-    infinite output in its own channel alone."""
+    infinite output in its own channel alone, and queries at either end of the range of floats scores."""
     pos, group = context - 1, q_heads // kv_heads
     rng = np.random.default_rng(context + q_heads)
     q, k, v = (rng.standard_normal(h * W).astype(np.float32) for h in (q_heads, kv_heads, kv_heads))
@@ -132,8 +132,13 @@ def test_infinite_rows(kind, context, q_heads, kv_heads):
         keys[-1, 334, 100] = -np.inf if kv_heads > 1 else np.inf
     elif kind == "value":
         values[:, 333, 3], values[:, context - 2, 200] = np.inf, -np.inf
-    else:
+    elif kind == "new key":
         kn[120] = 1e7
+    elif kind == "tiny query":
+        qn *= np.float32(2.0 ** -130)
+    else:
+        qn *= np.float32(2.0 ** 90)
+        scale *= 2.0 ** -90
     factors = synth.gemma4_rope_factors(W)
     bufs = [hip.Buffer.from_numpy(a) for a in (q, k, v, qn, kn, keys.view(np.uint16), values.view(np.uint16))]
     out = hip.Buffer(q_heads * W)

@@ -52,6 +52,19 @@ def test_wide_trace_gemma4_width_512_shared_v():
     print(f"gemma4 wide: layer ratio {ratio:.3f}, K/V ratio {ulps:.3f}, {differ} fp16 values differ", flush=True)
 
 
+@pytest.mark.parametrize("batch", [32, 100])
+def test_batched_trace_of_tiny_queries(batch):
+    """Queries of about 2^-130 (a subnormal query norm): every key weighs the same, in narrow and wide passes."""
+    model = synth.model(name="tinyq", layers=1, hidden=1024, intermediate=2048, q_heads=16, kv_heads=8, head_width=256,
+                        vocabulary=2048, window=64, global_every=2)
+    model.layers[0].q_norm *= np.float32(2.0 ** -130)
+    n = 100
+    ids = [int(i) for i in synth.prompt_ids(n, model.vocabulary, name="tinyq.ids")]
+    with open_with_env(model, n + 8, AF_TRACE_BATCH=batch) as s:
+        outputs, kv, _, _ = s.trace(ids, kv_rows=8 * 256, logits=False, hidden=False)
+    oracle.check_layer_stack(model, ids, outputs, kv, threads=THREADS, positions=[0, 1, 31, 32, 63, 64, 99])
+
+
 def test_wide_prefill_ids_match_one_position_at_a_time():
     """Greedy ids after a 300-token prompt: one wide pass against one step-kernel launch per position, and
     again on a follow-up turn whose pass starts in the middle of the ring."""
