@@ -194,7 +194,8 @@ constexpr uint32_t kBatchMax = 32;   // tokens per batch (crates/cuda-backend/sr
 // Prompt positions per prefill pass.  A pass of more than kBatchMax positions takes the wide GEMM
 // (wide_gemm_kernel), whose input image is laid out as its MFMAs read it and holds one scale per
 // token: with G = ceil(T / M) M / 16 groups of 16 tokens (M = wide_tokens(T)),
-//   fp16 [nb][G][hi, lo][64 lanes][8], then the tokens' scales 2^(e - 14) as float [16 G]
+//   fp16 [nb][G][hi, lo][64 lanes][8], then the tokens' scales 2^(e - 14) as float [16 G], then block
+//   factors float [nb][16 G]
 // where lane 16 q + t % 16 holds elements 4 q + {0, 2}, 16 + 4 q + {0, 2}, 4 q + {1, 3}, 16 + 4 q +
 // {1, 3} of token t's block: the order in which a dword of four code bytes unpacks.
 constexpr uint32_t kPassMax = 512;

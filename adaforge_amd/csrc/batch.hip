@@ -56,6 +56,31 @@ __device__ __forceinline__ void octet_halves(const float (&v)[8], int sh, v4u& h
     lo = v4u{l0, l1, l2, l3};
 }
 
+// Exponent e of a token's scale 2^(14 - e): ilogb of its largest |x| (128 for an infinity, whose products are
+// not finite at any scale).
+__device__ __forceinline__ int token_exponent(float m) { return m > 0.0f ? min(ilogbf(m), 128) : 0; }
+
+// The halves hi + lo hold u to 2^-23 of itself, or to 2^-25.  So with one scale for a whole token (|u| < 2^15) a
+// block is held to 2^-23 of its own largest element as long as that is 2^-16 of the token's or more.  A block
+// below 2^-kBlockSpread (four bits earlier, for its smaller elements) has its own scale, e + spread instead
+// of e, and its products are multiplied by 2^spread: an outlier channel costs no other block its bits.
+// 512 positions through six layers of the 12B shape: 3.93 ms, 4.37 where every token has such blocks (3.92
+// without the rule).  Returns spread, 0 for every other block; at least -100 (below that a block no longer counts in fp32 sums).
+constexpr int kBlockSpread = 12;
+__device__ __forceinline__ int block_spread(float m, int e) {
+    const int d = m > 0.0f ? ilogbf(m) - e : 0;
+    return d < -kBlockSpread ? max(d, -100) : 0;
+}
+
+// Largest |v| of a block, in each of its four lanes (parts 0-3).
+__device__ __forceinline__ float block_max4(const float (&v)[8]) {
+    float m = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) m = fmaxf(m, fabsf(v[k]));
+    m = fmaxf(m, dpp<kDppXor1>(m));
+    return fmaxf(m, dpp<kDppXor2>(m));
+}
+
 // Part p of block b of token t into the wide GEMM's image of G 16-token groups.
 __device__ __forceinline__ void wide_halves(const float (&v)[8], int sh, uint32_t b, uint32_t p, uint32_t t, uint32_t G,
                                             v4u* img) {
@@ -74,14 +99,14 @@ __device__ __forceinline__ void wide_halves(const float (&v)[8], int sh, uint32_
 // float4), and every global load of the token (x, res and both norm weights) is issued before the
 // first reduction, so the kernel waits for memory once.
 // PS: x comes from in.parts split-K partial planes (NO == 1 only).
-// WIDE: the wide GEMM's image, one scale per token; no padding tokens are written (their rows of the
+// WIDE: the wide GEMM's image, one scale per token but for small blocks (block_spread); no padding tokens are written (their rows of the
 // product are never stored).  Workgroup b takes token (b % 8) ceil(T / 8) + b / 8, so that the 16
 // tokens whose halves share a 256-byte run of the image are mostly written through one XCD's L2.
 template <int NO, bool PS, bool WIDE>
 __global__ __launch_bounds__(512) void batch_input_kernel(BatchIn in) {
     extern __shared__ __align__(16) float xs[];  // [K], BI_EMBED only
     __shared__ double red[8];
-    __shared__ float redf[8];
+    __shared__ float redf[8], reds[8];
     const uint32_t tid = threadIdx.x, K = in.K, nb = K / 32, no = K / 8, WG = wide_groups(in.T);
     const uint32_t t = WIDE ? blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8 : blockIdx.x;
     if (t >= in.T) return;
@@ -193,7 +218,6 @@ __global__ __launch_bounds__(512) void batch_input_kernel(BatchIn in) {
     }
     // the GEMM's input
     float v[NO][8];
-    float m = 0.0f;
 #pragma unroll
     for (int j = 0; j < NO; ++j)
 #pragma unroll
@@ -203,22 +227,45 @@ __global__ __launch_bounds__(512) void batch_input_kernel(BatchIn in) {
             v[j][4 * h + 1] = u.y;
             v[j][4 * h + 2] = u.z;
             v[j][4 * h + 3] = u.w;
-#pragma unroll
-            for (int k = 0; k < 4; ++k) m = fmaxf(m, fabsf(v[j][4 * h + k]));
         }
     int e = 0;
+    float bm[NO];  // the octets' blocks' largest elements
+    float *inv = nullptr, *factor = nullptr;
     if constexpr (WIDE) {
-        m = block_max_f(m, redf);
-        e = m > 0.0f ? ilogbf(m) : 0;
-        float* inv = reinterpret_cast<float*>(in.img + (size_t)nb * WG * 2048);
-        if (tid == 0) inv[t] = m > 0.0f ? ldexpf(1.0f, e - 14) : 0.0f;
+        // the token's largest block and its smallest that is not zero, with the same barriers
+        float m = 0.0f, least = INFINITY;
+#pragma unroll
+        for (int j = 0; j < NO; ++j) {
+            bm[j] = block_max4(v[j]);
+            m = fmaxf(m, bm[j]);
+            if (bm[j] > 0.0f) least = fminf(least, bm[j]);
+        }
+        m = wave_max(m);
+        least = -wave_max(-least);
+        if ((tid & 63) == 0) {
+            redf[tid >> 6] = m;
+            reds[tid >> 6] = least;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < 8; ++w) {
+            m = fmaxf(m, redf[w]);
+            least = fminf(least, reds[w]);
+        }
+        e = token_exponent(m);
+        inv = reinterpret_cast<float*>(in.img + (size_t)nb * WG * 2048);
+        const bool spread = m > 0.0f && block_spread(least, e) != 0;
+        if (spread) factor = inv + 16 * WG + t;
+        if (tid == 0) inv[t] = m > 0.0f ? ldexpf(spread ? -1.0f : 1.0f, e - 14) : 0.0f;
     }
 #pragma unroll
     for (int j = 0; j < NO; ++j) {
         const uint32_t o = tid + 512 * j;
         if (o >= no) continue;
         if constexpr (WIDE) {
-            wide_halves(v[j], 14 - e, o >> 2, o & 3, t, WG, reinterpret_cast<v4u*>(in.img));
+            const int d = block_spread(bm[j], e);
+            if (factor && (o & 3) == 0) factor[(size_t)(o >> 2) * 16 * WG] = ldexpf(1.0f, d);
+            wide_halves(v[j], 14 - e - d, o >> 2, o & 3, t, WG, reinterpret_cast<v4u*>(in.img));
         } else {
             v4f* y = reinterpret_cast<v4f*>(reinterpret_cast<float*>(in.img) + (size_t)t * K) + 8 * (o >> 2) + (o & 3);
             y[0] = v4f{v[j][0], v[j][1], v[j][2], v[j][3]};
@@ -622,7 +669,8 @@ __global__ __launch_bounds__(256) void batch_reduce_kernel(BatchGemm a, uint32_t
 // workgroup into LDS while the step before is multiplied.  The WK waves of a tile add their sums in LDS at the end.  The block's d_rb differs from the next one's, so each block's 16 x 16
 // products are folded into fp32 sums on their own (one FMA per product and lane: half as many VALU
 // cycles as the two MFMAs take; the token's scale waits for the epilogue, so that the fold has no other
-// factor).  Sums run over kWideChain blocks, then join a total, so that no chain of fp32 additions is
+// factor, unless a token of the tile has small blocks with scales of their own: then a second form of the
+// loop multiplies by the blocks' factors).  Sums run over kWideChain blocks, then join a total, so that no chain of fp32 additions is
 // longer than K / 32 / kWideChain + kWideChain.
 //
 // Work items (split, row group, token tile), token tile fastest, go to the XCDs in contiguous
@@ -710,6 +758,10 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2 / WK ? 2 / WK : 1) void wide_g
 #pragma unroll
         for (int n = 0; n < 4; ++n) acc[m][n] = tot[m][n] = zero;
 
+    const float* inv = reinterpret_cast<const float*>(a.img + (size_t)nb * G * 2048);
+    float scales[MG / 4];  // of the tile's tokens, 64 at a time
+#pragma unroll
+    for (int i = 0; i < MG / 4; ++i) scales[i] = gp(inv)[mt0 * MG * 16 + 64 * i + lane];
     load(b0);
     load_d(b0);
     unpack(0);
@@ -718,78 +770,108 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2 / WK ? 2 / WK : 1) void wide_g
 #pragma unroll
     for (int st = 0; st < NA - 1; ++st) copy(b0 + st * WK, st);
     __builtin_amdgcn_sched_barrier(0);
-    uint32_t step = 0, sa = 0;  // step % NA
-    for (uint32_t b = b0; b < b1; b += WK, ++step) {
-        // This step's copies are in (with three stages, all but the SA newest requests: the copies for the
-        // next step are the last ones of an iteration) and its weights written, in every wave; every wave
-        // has read the stages that are written below.
-        if constexpr (NA == 3) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(SA) : "memory");
-        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
-        // The operands are read and waited for in one block: the compiler would wait for every copy in
-        // flight before an LDS read that it sees.
-        v4u ahu[4], alu[4], bwu[4];
-        const uint32_t pa = lds + 16 * (sa * kA + wk * MG * 128 + wm * 512 + lane),
-                       pb = lds + 16 * (NA * kA + (step & 1) * kB + wk * NT * 64 + wn * 256 + lane);
-        asm volatile(
-            "ds_read_b128 %8, %13\n\t"
-            "ds_read_b128 %0, %12\n\t"
-            "ds_read_b128 %1, %12 offset:2048\n\t"
-            "ds_read_b128 %2, %12 offset:4096\n\t"
-            "ds_read_b128 %3, %12 offset:6144\n\t"
-            "ds_read_b128 %4, %12 offset:1024\n\t"
-            "ds_read_b128 %5, %12 offset:3072\n\t"
-            "ds_read_b128 %6, %12 offset:5120\n\t"
-            "ds_read_b128 %7, %12 offset:7168\n\t"
-            "ds_read_b128 %9, %13 offset:1024\n\t"
-            "ds_read_b128 %10, %13 offset:2048\n\t"
-            "ds_read_b128 %11, %13 offset:3072\n\t"
-            "s_waitcnt lgkmcnt(0)"
-            : "=&v"(ahu[0]), "=&v"(ahu[1]), "=&v"(ahu[2]), "=&v"(ahu[3]), "=&v"(alu[0]), "=&v"(alu[1]), "=&v"(alu[2]),
-              "=&v"(alu[3]), "=&v"(bwu[0]), "=&v"(bwu[1]), "=&v"(bwu[2]), "=&v"(bwu[3])
-            : "v"(pa), "v"(pb)
-            : "memory");
-        v8h ah[4], al[4], bw[4];
+    bool small = false;
 #pragma unroll
-        for (int m = 0; m < 4; ++m) {
-            ah[m] = __builtin_bit_cast(v8h, ahu[m]);
-            al[m] = __builtin_bit_cast(v8h, alu[m]);
-            bw[m] = __builtin_bit_cast(v8h, bwu[m]);
+    for (int i = 0; i < MG / 4; ++i) small |= scales[i] < 0.0f && mt0 * MG * 16 + 64 * i + lane < a.T;
+    auto multiply = [&](auto spread) {
+        constexpr bool SPREAD = decltype(spread)::value;
+        // SPREAD: this lane's tokens with factors, bit 4 m + e
+        uint32_t own = 0;
+        const float* factor = inv + 16 * G + (mt0 * MG + wm * 4) * 16 + 4 * q;
+        if constexpr (SPREAD) {
+#pragma unroll
+            for (int m = 0; m < 4; ++m) {
+                const v4f s = *gp(reinterpret_cast<const v4f*>(inv + (mt0 * MG + wm * 4 + m) * 16 + 4 * q));
+#pragma unroll
+                for (int e = 0; e < 4; ++e) own |= s[e] < 0.0f ? 1u << (4 * m + e) : 0u;
+            }
         }
-        float d[4];
+        uint32_t step = 0, sa = 0;  // step % NA
+        for (uint32_t b = b0; b < b1; b += WK, ++step) {
+            // This step's copies are in (with three stages, all but the SA newest requests: the copies for the
+            // next step are the last ones of an iteration) and its weights written, in every wave; every wave
+            // has read the stages that are written below.
+            if constexpr (NA == 3) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(SA) : "memory");
+            else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+            // The operands are read and waited for in one block: the compiler would wait for every copy in
+            // flight before an LDS read that it sees.
+            v4u ahu[4], alu[4], bwu[4];
+            const uint32_t pa = lds + 16 * (sa * kA + wk * MG * 128 + wm * 512 + lane),
+                           pb = lds + 16 * (NA * kA + (step & 1) * kB + wk * NT * 64 + wn * 256 + lane);
+            asm volatile(
+                "ds_read_b128 %8, %13\n\t"
+                "ds_read_b128 %0, %12\n\t"
+                "ds_read_b128 %1, %12 offset:2048\n\t"
+                "ds_read_b128 %2, %12 offset:4096\n\t"
+                "ds_read_b128 %3, %12 offset:6144\n\t"
+                "ds_read_b128 %4, %12 offset:1024\n\t"
+                "ds_read_b128 %5, %12 offset:3072\n\t"
+                "ds_read_b128 %6, %12 offset:5120\n\t"
+                "ds_read_b128 %7, %12 offset:7168\n\t"
+                "ds_read_b128 %9, %13 offset:1024\n\t"
+                "ds_read_b128 %10, %13 offset:2048\n\t"
+                "ds_read_b128 %11, %13 offset:3072\n\t"
+                "s_waitcnt lgkmcnt(0)"
+                : "=&v"(ahu[0]), "=&v"(ahu[1]), "=&v"(ahu[2]), "=&v"(ahu[3]), "=&v"(alu[0]), "=&v"(alu[1]), "=&v"(alu[2]),
+                  "=&v"(alu[3]), "=&v"(bwu[0]), "=&v"(bwu[1]), "=&v"(bwu[2]), "=&v"(bwu[3])
+                : "v"(pa), "v"(pb)
+                : "memory");
+            v8h ah[4], al[4], bw[4];
 #pragma unroll
-        for (int n = 0; n < 4; ++n) {
-            d[n] = WK == 1 || b + wk < b1 ? h2f(dn[n]) : 0.0f;
-            asm("" : "+v"(d[n]));  // (converted once: as a mixed-precision operand of 64 FMAs it takes 1.5 % longer)
-        }
-        unpack((step & 1) ^ 1);
-        load(b + 2 * WK);
-        load_d(b + WK);
-        __builtin_amdgcn_sched_barrier(0);
-        copy(b + (NA - 1) * WK, sa ? sa - 1 : NA - 1);
-        __builtin_amdgcn_sched_barrier(0);
-        sa = sa == NA - 1 ? 0 : sa + 1;
+            for (int m = 0; m < 4; ++m) {
+                ah[m] = __builtin_bit_cast(v8h, ahu[m]);
+                al[m] = __builtin_bit_cast(v8h, alu[m]);
+                bw[m] = __builtin_bit_cast(v8h, bwu[m]);
+            }
+            float d[4];
 #pragma unroll
-        for (int n = 0; n < 4; ++n) {
-            v4f D[4];
+            for (int n = 0; n < 4; ++n) {
+                d[n] = WK == 1 || b + wk < b1 ? h2f(dn[n]) : 0.0f;
+                asm("" : "+v"(d[n]));  // (converted once: as a mixed-precision operand of 64 FMAs it takes 1.5 % longer)
+            }
+            v4f f[4];
+            if constexpr (SPREAD) {
 #pragma unroll
-            for (int m = 0; m < 4; ++m) D[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[m], bw[n], zero, 0, 0, 0);
+                for (int m = 0; m < 4; ++m) f[m] = *gp(reinterpret_cast<const v4f*>(factor + (size_t)min(b + wk, last) * 16 * G + 16 * m));
+            }
+            unpack((step & 1) ^ 1);
+            load(b + 2 * WK);
+            load_d(b + WK);
+            __builtin_amdgcn_sched_barrier(0);
+            copy(b + (NA - 1) * WK, sa ? sa - 1 : NA - 1);
+            __builtin_amdgcn_sched_barrier(0);
+            sa = sa == NA - 1 ? 0 : sa + 1;
 #pragma unroll
-            for (int m = 0; m < 4; ++m) D[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[m], bw[n], D[m], 0, 0, 0);
+            for (int n = 0; n < 4; ++n) {
+                v4f D[4];
 #pragma unroll
-            for (int m = 0; m < 4; ++m)
+                for (int m = 0; m < 4; ++m) D[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[m], bw[n], zero, 0, 0, 0);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) acc[m][n][e] = fmaf(d[n], D[m][e], acc[m][n][e]);
-        }
-        if ((step & (kWideChain - 1)) == kWideChain - 1) {
+                for (int m = 0; m < 4; ++m) D[m] = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[m], bw[n], D[m], 0, 0, 0);
+                if constexpr (SPREAD) {
 #pragma unroll
-            for (int m = 0; m < 4; ++m)
+                    for (int m = 0; m < 4; ++m)
 #pragma unroll
-                for (int n = 0; n < 4; ++n) {
-                    tot[m][n] += acc[m][n];
-                    acc[m][n] = zero;
+                        for (int e = 0; e < 4; ++e) D[m][e] *= own >> (4 * m + e) & 1 ? f[m][e] : 1.0f;
                 }
+#pragma unroll
+                for (int m = 0; m < 4; ++m)
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) acc[m][n][e] = fmaf(d[n], D[m][e], acc[m][n][e]);
+            }
+            if ((step & (kWideChain - 1)) == kWideChain - 1) {
+#pragma unroll
+                for (int m = 0; m < 4; ++m)
+#pragma unroll
+                    for (int n = 0; n < 4; ++n) {
+                        tot[m][n] += acc[m][n];
+                        acc[m][n] = zero;
+                    }
+            }
         }
-    }
+    };
+    if (__any(small)) multiply(std::true_type{});
+    else multiply(std::false_type{});
     asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // no copy outlives its LDS
 #pragma unroll
     for (int m = 0; m < 4; ++m)
@@ -807,7 +889,6 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2 / WK ? 2 / WK : 1) void wide_g
             for (int n = 0; n < 4; ++n) X[(wave * 16 + m * 4 + n) * 64 + lane] = tot[m][n];
         __syncthreads();
     }
-    const float* inv = reinterpret_cast<const float*>(a.img + (size_t)nb * G * 2048);
 #pragma unroll
     for (int mi = 0; mi < 4 / WK; ++mi) {
         const uint32_t m = wk * (4 / WK) + mi;
@@ -824,7 +905,9 @@ __global__ __launch_bounds__(64 * WM * WN * WK, 2 / WK ? 2 / WK : 1) void wide_g
             }
         }
         const uint32_t t0 = (mt0 * MG + wm * 4 + m) * 16 + 4 * q;
-        const v4f s = *gp(reinterpret_cast<const v4f*>(inv + t0));
+        v4f s = *gp(reinterpret_cast<const v4f*>(inv + t0));
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[e] = fabsf(s[e]);
 #pragma unroll
         for (int n = 0; n < 4; n += P) {
             const uint32_t row = tile_of(wn * 4 + n) * 16 + r;
@@ -1343,7 +1426,7 @@ static WidePlan wide_plan(uint32_t rows, uint32_t blocks, uint32_t tokens, bool 
 
 size_t batch_image_bytes(uint32_t blocks, uint32_t tokens) {
     const size_t floats = (size_t)blocks * 128 * std::min(tokens, kBatchMax);
-    return tokens > kBatchMax ? std::max(floats, ((size_t)blocks * 2048 + 64) * ((tokens + 127) / 128 * 8)) : floats;
+    return tokens > kBatchMax ? std::max(floats, ((size_t)blocks * (2048 + 64) + 64) * ((tokens + 127) / 128 * 8)) : floats;
 }
 
 size_t batch_gemm_part_bytes(uint32_t rows, uint32_t blocks, uint32_t tokens, bool gelu_pair) {

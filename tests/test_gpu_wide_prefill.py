@@ -52,6 +52,63 @@ def test_wide_trace_gemma4_width_512_shared_v():
     print(f"gemma4 wide: layer ratio {ratio:.3f}, K/V ratio {ulps:.3f}, {differ} fp16 values differ", flush=True)
 
 
+def one_channel_model(name, special, **kw):
+    """A one-layer model whose embeddings are zero in channel 5 for every id not in `special`, and large there."""
+    model = synth.model(name=name, layers=1, hidden=1024, q_heads=16, kv_heads=8, head_width=256, vocabulary=2048, **kw)
+    rows = model.table.reshape(model.vocabulary, model.hidden // 256, 210)  # Q6_K: ql[128], qh[64], scales, d
+    keep = np.isin(np.arange(model.vocabulary), special)
+    rows[~keep, 0, 5] &= 0xF0
+    rows[~keep, 0, 128 + 5] = rows[~keep, 0, 128 + 5] & 0xFC | 2  # code 32: weight 0
+    rows[keep, 0, 5] |= 0x0F
+    rows[keep, 0, 128 + 5] |= 3  # code 63: weight 31
+    rows[keep, 0, 192] = 127     # (the scale of channels 0-15)
+    return model
+
+
+def zero_block(matrix, columns):
+    """The Q4_0 matrix with the scales of its first 32 columns' blocks zero."""
+    blocks = matrix.reshape(-1, columns // 32, 18)
+    blocks[:, 0, :2] = 0
+    return matrix
+
+
+@pytest.mark.parametrize("n", [40, 100])
+def test_wide_trace_keeps_small_blocks_beside_an_outlier(n):
+    """A channel 2^30 above the others in some tokens' GEMM inputs, in a block whose weights are zero: the
+    products come from the small blocks alone and are as exact as without it (K/V within one fp16 ulp, layer
+    outputs within the oracle's tolerance)."""
+    ids = [int(i) for i in synth.prompt_ids(n, 2048, name=f"outlier{n}.ids")]
+    model = one_channel_model(f"outlier{n}", ids[3::2], intermediate=2048, window=0, global_every=1)
+    L = model.layers[0]
+    L.input_norm[5] = L.ffn_norm[5] = np.float32(2.0 ** 30)
+    for m in (L.q, L.k, L.v, L.gate, L.up):
+        zero_block(m, model.hidden)
+    with open_with_env(model, n + 8, AF_TRACE_BATCH=512) as s:
+        outputs, kv, _, _ = s.trace(ids, kv_rows=8 * 256, logits=False, hidden=False)
+    positions = [0, 1, 2, 3, 4, 15, 16, 31, 32, n - 2, n - 1]
+    ratio, ulps, differ = oracle.check_layer_stack(model, ids, outputs, kv, threads=THREADS, positions=positions)
+    print(f"outlier n={n}: layer ratio {ratio:.3f}, K/V ratio {ulps:.3f}, {differ} fp16 values differ", flush=True)
+
+
+@pytest.mark.parametrize("n", [40, 100])
+def test_wide_trace_non_finite_token(n):
+    """One token's GEMM input overflows fp32 (beside other tokens and the tile's padding): no position that does not see
+    it changes."""
+    at, window = 19, 8
+    ids = [int(i) for i in synth.prompt_ids(n, 2047, name=f"nonfinite{n}.ids")]
+    ids[at] = 2047
+    model = one_channel_model(f"nonfinite{n}", [2047], intermediate=2048, window=window, global_every=2)
+    model.layers[0].input_norm[5] = np.float32(3e38)
+    with open_with_env(model, n + 8, AF_TRACE_BATCH=512) as s:
+        outputs, kv, _, _ = s.trace(ids, kv_rows=8 * 256, logits=False, hidden=False)
+    assert not np.isfinite(kv[at]).any() and np.isfinite(np.delete(kv, at, 0)).all()
+    # (a batched attention multiplies a key that a query does not see by zero: positions of its tile of
+    # queries may be NaN too, so the ones checked are those of other tiles)
+    kv[at] = 0.0  # (seen by none of these; the oracle takes finite histories)
+    positions = [p for p in (32, 33, 39, 47, 48, 63, 64, 65, 99) if p < n]
+    oracle.check_layer_stack(model, ids, outputs, kv, threads=THREADS, positions=positions)
+
+
 @pytest.mark.parametrize("batch", [32, 100])
 def test_batched_trace_of_tiny_queries(batch):
     """Queries of about 2^-130 (a subnormal query norm): every key weighs the same, in narrow and wide passes."""
