@@ -70,3 +70,32 @@ def test_non_finite_inputs_stay_in_their_token():
                     oracle.compare(oracle.q4_matvec(w, columns, rows, xs[t]), y[t])
     finally:
         N.lib().af_q4_free(h)
+
+
+@pytest.mark.parametrize("columns,rows,tokens", [(160, 65, 8), (4128, 63, 5), (2080, 1000, 16), (1056, 999, 17),
+                                                 (3840, 15361, 16), (3872, 15360, 30), (16384, 130, 32)])
+def test_small_blocks_beside_an_outlier(columns, rows, tokens):
+    """Some tokens hold one element 2^30 above the rest, in a block whose weights are zero: their products come from
+    the small blocks alone, to the tolerance of the tokens without one."""
+    w = synth.q4(f"outlier{columns}x{rows}", columns, rows, signed=True)
+    w.reshape(rows, columns // 32, 18)[:, 2, :2] = 0
+    rng = np.random.default_rng(columns + rows + tokens)
+    xs = rng.standard_normal((tokens, columns)).astype(np.float32)
+    small = xs.copy()
+    small[:, 64:96] = 0.0
+    xs[1::2, 70] = np.float32(2.0 ** 30)
+    h = N.P()
+    N.check(N.lib().af_q4_upload(w.ctypes.data_as(N.u8p), w.size, columns, rows, ctypes.byref(h)))
+    try:
+        xb, yb = hip.Buffer.from_numpy(xs), hip.Buffer(tokens * rows)
+        N.check(N.lib().af_q4_gemm(h, xb.ptr, tokens, yb.ptr, None))
+        hip.synchronize()
+        y = yb.numpy().reshape(tokens, rows)
+    finally:
+        N.lib().af_q4_free(h)
+    for t in {0, 1, 2, tokens // 2, tokens - 1}:
+        ref = oracle.q4_matvec(w, columns, rows, small[t])
+        # inputs to 22 bits of their block's largest and fp32 sums, as in test_forms_match_oracle
+        scale = np.sqrt(columns) * np.abs(small[t]).max() * 0.02 * 8
+        assert np.abs(y[t] - ref).max() <= 2.0 ** -20 * scale
+        oracle.compare(ref, y[t])
