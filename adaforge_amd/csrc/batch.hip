@@ -1005,6 +1005,35 @@ __device__ __forceinline__ float lanes4_max(float v) {
 
 }  // namespace
 
+// Queries i0, i0 + step, ... (16 / step of them) of KV head h against the keys that each sees in [k_begin, k_end),
+// in fp32 (plain_attention): where a wave's sums are not finite, an infinite cached value of a key that one
+// query sees may have met the zero probability of another.
+template <int D>
+__device__ __forceinline__ void plain_queries(const BatchAttn& a, const uint16_t* kh, const uint16_t* vh, uint32_t h, uint32_t i0,
+                                              uint32_t step, uint32_t c, uint32_t k_begin, uint32_t k_end) {
+    const uint32_t lane = threadIdx.x & 63, q_heads = a.kv_heads * a.group;
+#pragma unroll 1
+    for (uint32_t qi = i0; qi < min(i0 + 16, a.T * a.group); qi += step) {
+        const uint32_t t = qi / a.group, qh = h * a.group + qi % a.group, end = a.pos0 + t + 1;
+        const float* src = a.q + ((size_t)t * q_heads + qh) * D + 4 * lane;
+        float x[D / 64], o[D / 64], m, l;
+#pragma unroll
+        for (int e = 0; e < D / 64; ++e) x[e] = src[e / 4 * 256 + e % 4];
+        const uint32_t lo = a.window && end > a.window ? end - a.window : 0u;
+        plain_attention<D>(
+            x, a.scale, max(lo, k_begin), min(end, k_end), [&](uint32_t key) { return kh + (size_t)(key % a.ring) * D; },
+            [&](uint32_t key) { return vh + (size_t)(key % a.ring) * D; }, o, m, l);
+        float* p = a.nchunks == 1 ? a.out + (size_t)t * a.out_stride + (size_t)qh * D
+                                  : a.part + (((size_t)t * q_heads + qh) * a.nchunks + c) * (D + 2);
+#pragma unroll
+        for (int e = 0; e < D / 64; ++e) p[4 * lane + e / 4 * 256 + e % 4] = a.nchunks == 1 ? o[e] / l : o[e];
+        if (a.nchunks > 1 && lane == 0) {
+            p[D] = m;
+            p[D + 1] = l;
+        }
+    }
+}
+
 template <int D, int KC>
 __global__ __launch_bounds__(256) void batch_attention_kernel(BatchAttn a) {
     constexpr int KP = D + 8;         // row stride of K and of the query planes (halves)
@@ -1145,7 +1174,16 @@ __global__ __launch_bounds__(256) void batch_attention_kernel(BatchAttn a) {
             }
         }
     }
-    __syncthreads();
+    float odd = 0.0f;  // NaN if a sum is not finite
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) odd = fmaf(acc[j][i], 0.0f, odd);
+    if (__syncthreads_or(odd != 0.0f)) {
+        plain_queries<D>(a, a.kcache + (size_t)h * a.ring * D, a.vcache + (size_t)h * a.ring * D, h, 16 * qt + wave, 4, c,
+                         k_begin, k_end);
+        return;
+    }
     if (a.nchunks == 1) {
 #pragma unroll
         for (int j = 0; j < NT; ++j)
@@ -1361,6 +1399,15 @@ __global__ __launch_bounds__(256, D == 256 ? 2 : 1) void wide_attention_kernel(B
             }
             acc[j] = o;
         }
+    }
+    float odd = lrun * 0.0f;  // NaN if a sum is not finite
+#pragma unroll
+    for (int j = 0; j < DT; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) odd = fmaf(acc[j][e], 0.0f, odd);
+    if (__any(odd != 0.0f)) {
+        plain_queries<D>(a, kh, vh, h, 64 * qt + 16 * wave, 1, c, k_begin, k_end);
+        return;
     }
     if (qi >= nq) return;
     if (a.nchunks == 1) {

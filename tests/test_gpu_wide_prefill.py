@@ -52,9 +52,10 @@ def test_wide_trace_gemma4_width_512_shared_v():
     print(f"gemma4 wide: layer ratio {ratio:.3f}, K/V ratio {ulps:.3f}, {differ} fp16 values differ", flush=True)
 
 
-def one_channel_model(name, special, **kw):
+def one_channel_model(name, special, q_heads=16, **kw):
     """A one-layer model whose embeddings are zero in channel 5 for every id not in `special`, and large there."""
-    model = synth.model(name=name, layers=1, hidden=1024, q_heads=16, kv_heads=8, head_width=256, vocabulary=2048, **kw)
+    model = synth.model(name=name, layers=1, hidden=1024, q_heads=q_heads, kv_heads=8, head_width=256,
+                        vocabulary=2048, **kw)
     rows = model.table.reshape(model.vocabulary, model.hidden // 256, 210)  # Q6_K: ql[128], qh[64], scales, d
     keep = np.isin(np.arange(model.vocabulary), special)
     rows[~keep, 0, 5] &= 0xF0
@@ -102,10 +103,36 @@ def test_wide_trace_non_finite_token(n):
     with open_with_env(model, n + 8, AF_TRACE_BATCH=512) as s:
         outputs, kv, _, _ = s.trace(ids, kv_rows=8 * 256, logits=False, hidden=False)
     assert not np.isfinite(kv[at]).any() and np.isfinite(np.delete(kv, at, 0)).all()
-    # (a batched attention multiplies a key that a query does not see by zero: positions of its tile of
-    # queries may be NaN too, so the ones checked are those of other tiles)
     kv[at] = 0.0  # (seen by none of these; the oracle takes finite histories)
-    positions = [p for p in (32, 33, 39, 47, 48, 63, 64, 65, 99) if p < n]
+    positions = [p for p in (0, 15, 16, 18, 27, 31, 32, 33, 39, 47, 48, 63, 64, 65, 99) if p < n]
+    oracle.check_layer_stack(model, ids, outputs, kv, threads=THREADS, positions=positions)
+
+
+@pytest.mark.parametrize("batch", [32, 512])
+@pytest.mark.parametrize("q_heads,window", [(8, 0), (16, 24), (32, 24)])
+def test_overflowed_value_reaches_only_the_positions_that_see_it(q_heads, window, batch):
+    """One position's V overflows fp16: positions before it, and those whose window it has left, are as
+    without it, also in its own tile of queries."""
+    n, at = 130, 45
+    ids = [int(i) for i in synth.prompt_ids(n, 2047, name="overflow.ids")]
+    ids[at] = 2047
+    model = one_channel_model("overflow", [2047], q_heads=q_heads, intermediate=2048, window=window,
+                              global_every=2 if window else 1)
+    L = model.layers[0]
+    first = L.v.reshape(8 * 256, model.hidden // 32, 18)[0, 0]  # row 0, columns 0-31: only channel 5 weighs
+    first[:2] = np.frombuffer(np.float16(60000.0).tobytes(), np.uint8)
+    first[2:] = 0x88
+    first[2 + 5] = 0x8F
+    with open_with_env(model, n + 8, AF_TRACE_BATCH=batch) as s:
+        outputs, kv, _, _ = s.trace(ids, kv_rows=8 * 256, logits=False, hidden=False)
+    assert np.isinf(kv[at, 0, 1, 0]) and np.isfinite(np.delete(kv, at, 0)).all()
+    sees = np.arange(n) >= at
+    if window:
+        sees &= np.arange(n) < at + window
+    bad = ~np.isfinite(outputs[:, 0]).all(axis=1)
+    assert np.array_equal(bad, sees), np.nonzero(bad != sees)[0]
+    kv[at] = 0.0  # (seen by none of these; the oracle takes finite histories)
+    positions = [p for p in (0, 15, 16, 31, 32, 40, 44, 63, 64, 69, 70, 95, 96, 129) if not sees[p]]
     oracle.check_layer_stack(model, ids, outputs, kv, threads=THREADS, positions=positions)
 
 
