@@ -398,6 +398,7 @@ struct Scratch {
     std::mutex mu;
     DevMem head_partial, head_counter, attn_part, attn_counters;
     DevMem batch_part, batch_counters;  // split-K partials and tickets of af_q4_gemm
+    DevMem batch_x;                     // and its vectors, where y overlaps them
     DevMem attn_freq;                   // the last RoPE inverse frequencies of af_attention_decode
     std::vector<double> attn_freq_host; // their host copy (re-uploaded only when they change)
 };
@@ -504,7 +505,16 @@ int af_q4_gemm(const af_q4* m, const float* x, uint32_t tokens, float* y, void* 
                    "batch partials")))
         return rc;
     if ((rc = grow(g_scratch.batch_counters, batch_gemm_counters(w.rows, false) * 4, true, "batch counters"))) return rc;
+    // (whatever this call's y: a later call in place, under graph capture for instance, allocates nothing)
+    if ((rc = grow(g_scratch.batch_x, (size_t)kBatchMax * w.blocks * 128, false, "batch vectors"))) return rc;
     const hipStream_t s = (hipStream_t)stream;
+    // Workgroups write y while others still read x: vectors that y overlaps are copied first.
+    const size_t xb = (size_t)tokens * w.blocks * 128, yb = (size_t)tokens * w.rows * 4;
+    const uintptr_t x0 = reinterpret_cast<uintptr_t>(x), y0 = reinterpret_cast<uintptr_t>(y);
+    if (x0 < y0 + yb && y0 < x0 + xb && x0 % 16 == 0) {  // (a misaligned x is refused by the launch)
+        HIP_OK(hipMemcpyAsync(g_scratch.batch_x.p, x, xb, hipMemcpyDeviceToDevice, s), "batched GEMV input copy");
+        x = g_scratch.batch_x.as<float>();
+    }
     BatchGemm g{};
     g.w = w;
     g.x = x;

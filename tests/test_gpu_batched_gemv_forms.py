@@ -99,3 +99,26 @@ def test_small_blocks_beside_an_outlier(columns, rows, tokens):
         scale = np.sqrt(columns) * np.abs(small[t]).max() * 0.02 * 8
         assert np.abs(y[t] - ref).max() <= 2.0 ** -20 * scale
         oracle.compare(ref, y[t])
+
+
+@pytest.mark.parametrize("n,tokens,offset", [(1024, 5, 0), (3840, 12, 0), (3840, 32, 0), (2080, 30, 2080 * 4), (2080, 8, -64)])
+def test_outputs_over_the_inputs(n, tokens, offset):
+    """y in place of x, or overlapping it by any number of elements: the vectors are read before any is written."""
+    w = synth.q4(f"inplace{n}", n, n, signed=True)
+    xs = np.random.default_rng(n + tokens).standard_normal((tokens, n)).astype(np.float32)
+    h = N.P()
+    N.check(N.lib().af_q4_upload(w.ctypes.data_as(N.u8p), w.size, n, n, ctypes.byref(h)))
+    try:
+        b = hip.Buffer(3 * tokens * n)
+        whole = np.zeros(3 * tokens * n, np.float32)
+        whole[tokens * n:2 * tokens * n] = xs.ravel()
+        for _ in range(3):
+            b.upload(whole)
+            at = b.ptr + tokens * n * 4
+            N.check(N.lib().af_q4_gemm(h, at, tokens, at + 4 * offset, None))
+            hip.synchronize()
+            y = b.numpy()[tokens * n + offset:][:tokens * n].reshape(tokens, n)
+            for t in {0, tokens // 2, tokens - 1}:
+                oracle.compare(oracle.q4_matvec(w, n, n, xs[t]), y[t])
+    finally:
+        N.lib().af_q4_free(h)
