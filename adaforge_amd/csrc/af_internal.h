@@ -246,10 +246,13 @@ struct BatchGemm {
     float* y;               // y[t * y_stride + r], r < w.rows (gate/up: f32(gelu(gate)) * up)
     size_t y_stride;
     float* part;            // split-K partials (batch_gemm_part_bytes)
-    uint32_t* counters;     // batch_gemm_counters words, zero between launches
+    uint64_t* counters;     // batch_gemm_counters tickets, zero between launches
+    uint64_t epoch;         // tickets count from here: kEpochStep more than the launch's before it, or 0 where
+                            // no two launches on these counters ever overlap
     bool defer;             // a single matrix split over K: leave the partials for the next kernel (no y)
 };
 constexpr uint32_t kDeferParts = 16;  // K splits at most
+constexpr uint64_t kEpochStep = 1ull << 20;
 
 // Attention of a batch over the KV cache after the append pass (batch_attention_kernel): the
 // tokens' queries q[t][q_heads][D], token t at position pos0 + t seeing keys [max(0, pos0 + t + 1 -

@@ -399,6 +399,7 @@ struct Scratch {
     DevMem head_partial, head_counter, attn_part, attn_counters;
     DevMem batch_part, batch_counters;  // split-K partials and tickets of af_q4_gemm
     DevMem batch_x;                     // and its vectors, where y overlaps them
+    uint64_t batch_epoch = 0;           // of its last call's tickets
     DevMem attn_freq;                   // the last RoPE inverse frequencies of af_attention_decode
     std::vector<double> attn_freq_host; // their host copy (re-uploaded only when they change)
 };
@@ -504,7 +505,13 @@ int af_q4_gemm(const af_q4* m, const float* x, uint32_t tokens, float* y, void* 
     if ((rc = grow(g_scratch.batch_part, batch_gemm_part_bytes(w.rows, w.blocks, kBatchMax, false) + 4, false,
                    "batch partials")))
         return rc;
-    if ((rc = grow(g_scratch.batch_counters, batch_gemm_counters(w.rows, false) * 4, true, "batch counters"))) return rc;
+    const size_t tickets = batch_gemm_counters(w.rows, false), had = g_scratch.batch_counters.bytes;
+    if ((rc = grow(g_scratch.batch_counters, tickets * 8, true, "batch counters"))) return rc;
+    if (const char* left = std::getenv("AF_GEMM_TICKETS_LEFT"); left && g_scratch.batch_counters.bytes != had) {
+        // (for tests: what calls that overlapped may leave)
+        const std::vector<uint64_t> v(tickets, std::strtoull(left, nullptr, 10));
+        HIP_OK(hipMemcpy(g_scratch.batch_counters.p, v.data(), tickets * 8, hipMemcpyHostToDevice), "batch counters");
+    }
     // (whatever this call's y: a later call in place, under graph capture for instance, allocates nothing)
     if ((rc = grow(g_scratch.batch_x, (size_t)kBatchMax * w.blocks * 128, false, "batch vectors"))) return rc;
     const hipStream_t s = (hipStream_t)stream;
@@ -523,7 +530,8 @@ int af_q4_gemm(const af_q4* m, const float* x, uint32_t tokens, float* y, void* 
     g.y = y;
     g.y_stride = w.rows;
     g.part = g_scratch.batch_part.as<float>();
-    g.counters = g_scratch.batch_counters.as<uint32_t>();
+    g.counters = g_scratch.batch_counters.as<uint64_t>();
+    g.epoch = g_scratch.batch_epoch += kEpochStep;
     HIP_OK(launch_batch_gemm(g, false, s), "batched GEMV launch");
     return AF_OK;
 }
@@ -1362,7 +1370,7 @@ struct af_session {
             {&ACTB, T * intermediate * 4},
             {&DB, T * hidden * 4},        {&BIMG, batch_image_bytes(blocks, (uint32_t)T)}, {&BGEMM, part},
             {&BPART, (size_t)kBatchMax * kBatchAttnChunks * max_qh_part * 4},
-            {&BCOUNT, T * std::max<uint32_t>(max_qh, 64) * 4}, {&BTICKETS, tickets * 4},
+            {&BCOUNT, T * std::max<uint32_t>(max_qh, 64) * 4}, {&BTICKETS, tickets * 8},
         };
         for (auto& b : bufs) {
             int rc = dev_alloc(*b.m, b.bytes, "batch buffer");
@@ -1406,7 +1414,7 @@ struct af_session {
         g.y = y;
         g.y_stride = y_stride;
         g.part = BGEMM.as<float>();
-        g.counters = BTICKETS.as<uint32_t>();
+        g.counters = BTICKETS.as<uint64_t>();
         g.defer = parts != nullptr;
         return launch_batch_gemm(g, m2 != nullptr, stream, parts);
     }

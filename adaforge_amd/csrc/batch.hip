@@ -649,13 +649,17 @@ __global__ __launch_bounds__(64 * W) void batch_gemm_kernel(BatchGemm a, uint32_
     }
     if (!fuse) return;
     // the last workgroup of the row group adds the planes: stored through to the memory side and
-    // waited for before the ticket, read from there (the XCDs' L2s are not coherent with each other)
+    // waited for before the ticket, read from there (the XCDs' L2s are not coherent with each other).
+    // Tickets count from the launch's epoch: two launches that overlap on the same counters (which
+    // callers are told not to make) spoil each other's sums and may leave a count behind, but a
+    // later launch's epoch is above it.
+    if (tid == 0) __hip_atomic_fetch_max(a.counters + gi, a.epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     __builtin_amdgcn_s_waitcnt(kWaitVm0);
     __syncthreads();
     if (tid == 0) {
-        const uint32_t ticket = __hip_atomic_fetch_add(a.counters + gi, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        last = ticket == S - 1;
-        if (last) __hip_atomic_store(a.counters + gi, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        const uint64_t ticket = __hip_atomic_fetch_add(a.counters + gi, (uint64_t)1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        last = ticket == a.epoch + S - 1;
+        if (last) __hip_atomic_store(a.counters + gi, (uint64_t)0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     }
     __syncthreads();
     if (!last) return;

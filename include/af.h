@@ -89,8 +89,10 @@ void af_q4_free(af_q4* m);
 int af_q4_gemv(const af_q4* m, const float* x, float* y, void* stream);
 /* y[t][rows] = W x[t][columns] for t < tokens, 1 <= tokens <= 32, with W read once for all
  * vectors (crates/cuda-backend/src/batch.rs:113-148 BatchKernels::matvec, MAX_BATCH = 32 at
- * batch.rs:10; kernels/ada/q4_batch.cu).  The vectors' digit image lives in library scratch shared by
- * all calls: calls that overlap on different streams race. */
+ * batch.rs:10; kernels/ada/q4_batch.cu).  y may overlap x.  Partial sums over ranges of the columns
+ * and their completion tickets live in library scratch shared by all calls: the outputs of calls that
+ * overlap on different streams are undefined.  Calls after them are not affected, but for a captured call,
+ * whose replays may be wrong until the next direct call on as many rows. */
 int af_q4_gemm(const af_q4* m, const float* x, uint32_t tokens, float* y, void* stream);
 
 /* Q6Matrix upload (crates/domain/src/q6.rs:8-20; crates/cuda-backend/src/logits.rs:292-316). */

@@ -2,6 +2,9 @@
 8- or 16-wave workgroups, K in one range, in ranges the last workgroup adds and in ranges a reduce launch
 adds, at the edges of row tiles, super-tiles and token groups."""
 import ctypes
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -122,3 +125,65 @@ def test_outputs_over_the_inputs(n, tokens, offset):
                 oracle.compare(oracle.q4_matvec(w, n, n, xs[t]), y[t])
     finally:
         N.lib().af_q4_free(h)
+
+
+def test_captured_calls_replay_among_direct_ones():
+    """A captured call's tickets serve every replay, with direct calls (whose tickets count from higher) in between."""
+    columns, rows, tokens = 15360, 3840, 5
+    w = synth.q4("replay", columns, rows, signed=True)
+    xs = np.random.default_rng(7).standard_normal((4, tokens, columns)).astype(np.float32)
+    h = N.P()
+    N.check(N.lib().af_q4_upload(w.ctypes.data_as(N.u8p), w.size, columns, rows, ctypes.byref(h)))
+    try:
+        xb, yb = hip.Buffer.from_numpy(xs[0]), hip.Buffer(tokens * rows)
+        s = hip.Stream()
+
+        def call():
+            N.check(N.lib().af_q4_gemm(h, xb.ptr, tokens, yb.ptr, s.handle))
+
+        call()
+        s.synchronize()
+        graph = hip.Graph(s, call)
+        for x in xs:
+            xb.upload(x)
+            got = []
+            for run in (call, lambda: graph.launch(s), lambda: graph.launch(s), call):
+                yb.upload(np.full(tokens * rows, np.nan, np.float32))
+                run()
+                s.synchronize()
+                got.append(yb.numpy())
+            assert all(np.array_equal(got[0], g) for g in got[1:])
+            oracle.compare(oracle.q4_matvec(w, columns, rows, x[0]), got[0][:rows])
+    finally:
+        N.lib().af_q4_free(h)
+
+
+LEFT = """
+import ctypes
+import numpy as np
+import oracle
+from adaforge_amd import _native as N, hip, synth
+for columns, rows, tokens in [(15360, 3840, 5), (4096, 3840, 32), (3840, 15361, 17)]:
+    w = synth.q4(f"left{columns}", columns, rows, signed=True)
+    xs = np.random.default_rng(rows).standard_normal((tokens, columns)).astype(np.float32)
+    h = N.P()
+    N.check(N.lib().af_q4_upload(w.ctypes.data_as(N.u8p), w.size, columns, rows, ctypes.byref(h)))
+    xb, yb = hip.Buffer.from_numpy(xs), hip.Buffer(tokens * rows)
+    for _ in range(2):
+        yb.upload(np.full(tokens * rows, np.nan, np.float32))
+        N.check(N.lib().af_q4_gemm(h, xb.ptr, tokens, yb.ptr, None))
+        hip.synchronize()
+        for t in (0, tokens - 1):
+            oracle.compare(oracle.q4_matvec(w, columns, rows, xs[t]), yb.numpy().reshape(tokens, rows)[t])
+print("sums complete")
+"""
+
+
+@pytest.mark.parametrize("left", [1, 3, 17])
+def test_tickets_left_by_overlapping_calls(left):
+    """Counts in the completion tickets, as two calls that overlapped on different streams may leave them (set from the
+    host where the tickets are allocated): the calls that follow are complete."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+    r = subprocess.run([sys.executable, "-c", LEFT], cwd=root, env=dict(os.environ, AF_GEMM_TICKETS_LEFT=str(left)),
+                       capture_output=True, text=True, timeout=100)
+    assert r.returncode == 0 and "sums complete" in r.stdout, r.stdout[-2000:] + r.stderr[-2000:]
