@@ -1393,8 +1393,10 @@ __global__ __launch_bounds__(D) void attention_kernel(AttnArgs a) {
 // attention_kernel takes two query heads per block there, so that a KV head's cache is read 8 times and
 // every cached value is unpacked and multiplied 16 times on the VALU.  Here the KV head's query
 // heads are the 16 columns of S^T = K Q^T and O^T = V^T P^T (fewer heads: zero queries), with the fp32
-// queries and probabilities as scaled fp16 pairs hi + lo (about 22 bits, products exact in fp32), as in
-// the batched attention.
+// queries and probabilities as the sum of three scaled fp16 pieces (all of an fp32's 24 bits, products exact
+// in fp32): with two pieces, as in the batched attention, the error against 64 bits was 2-3 % above
+// attention_kernel's from 1,025 to 1,500 visible positions (1.98 and 1.94e-7 over 24 seeds at 1,025), with
+// three it is at or below it in every case (1.93e-7; 2.01 and 2.22e-7 at 4,096) for 0.9 us more.
 //
 // A workgroup of four waves takes one chunk of the visible keys, 64 at a time:
 // - scores: wave w's 16 keys; a lane's operand is 16 bytes of its key's row, loaded straight from the
@@ -1408,11 +1410,11 @@ __global__ __launch_bounds__(D) void attention_kernel(AttnArgs a) {
 // workgroup per query head and 128 channels: 64 chunks of 16 heads are 2 MB, which one last
 // workgroup would read for longer than another launch takes.
 //
-// Infinities (fp16 overflows of cached rows) meet low halves of zero or of the other sign, so a wave whose sums
+// Infinities (fp16 overflows of cached rows) meet lower pieces of zero or of the other sign, so a wave whose sums
 // are not finite takes its channels again key by key in fp32 (plain_attention), as attention_kernel computes
-// them; the check is 33 FMAs and a ballot per wave (16.7 -> 16.9 us at 4,096 positions, a barrier more 17.3).
+// them; the check is 33 FMAs and a ballot per wave (0.2 us at 4,096 positions, with a barrier more 0.6).
 //
-// 16 query heads on one KV head: 16.9 us against 31.1 at 4,096 positions, 28.4 against 87.4 at 32,768 (of
+// 16 query heads on one KV head: 17.9 us against 31.1 at 4,096 positions, 31.7 against 88 at 32,768 (of
 // them 4.8 us the merge, 3 us the loop at 4,096, the rest the launch and the prologue's chain).  Error
 // against 64 bits 2.1e-7 at 4,096 (attention_kernel: 2.2e-7).
 // Keys per chunk (a multiple of 64) and chunks of n visible keys in at most cmax chunks.
@@ -1426,10 +1428,10 @@ typedef _Float16 h4 __attribute__((ext_vector_type(4)));
 
 __global__ __launch_bounds__(256) void attention_mfma_kernel(AttnArgs a) {
     constexpr int D = 512, QP = D + 8;  // query row stride (halves)
-    __shared__ __align__(16) _Float16 qh[16 * QP], ql[16 * QP];
+    __shared__ __align__(16) _Float16 qh[16 * QP], ql[16 * QP], qm[16 * QP];
     __shared__ __align__(16) double rsin[D / 2], rcos[D / 2];  // of the position's angles
     __shared__ __align__(16) uint16_t knew[D], vnew[D];
-    __shared__ __align__(16) _Float16 ph[4][16][16], pl[4][16][16];  // [16-key group][query][key]
+    __shared__ __align__(16) _Float16 ph[4][16][16], pl[4][16][16], pm[4][16][16];  // [16-key group][query][key]
     __shared__ float qscale[16], wmax[4][16], wsum[4][16];
 
     if (a.state && a.state[ST_STOP]) return;
@@ -1528,13 +1530,15 @@ __global__ __launch_bounds__(256) void attention_mfma_kernel(AttnArgs a) {
         const float s = query_scale(mx);  // |q s| < 32
 #pragma unroll
         for (int k = 0; k < 8; k += 4) {
-            h4 hi, lo;
+            h4 hi, lo, lm;
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const float u = o[k + j] * s;
                 hi[j] = (_Float16)u;
                 lo[j] = (_Float16)(u - (float)hi[j]);
+                lm[j] = (_Float16)(u - (float)hi[j] - (float)lo[j]);
             }
+            *reinterpret_cast<h4*>(qm + hq * QP + 64 * k + 4 * lane) = lm;
             *reinterpret_cast<h4*>(qh + hq * QP + 64 * k + 4 * lane) = hi;
             *reinterpret_cast<h4*>(ql + hq * QP + 64 * k + 4 * lane) = lo;
         }
@@ -1559,7 +1563,7 @@ __global__ __launch_bounds__(256) void attention_mfma_kernel(AttnArgs a) {
         reinterpret_cast<uint32_t*>(a.vcache + at)[tid] = reinterpret_cast<const uint32_t*>(vnew)[tid];
     }
 
-    v4f acc[8], accl[8];  // sums of the hi and of the lo products
+    v4f acc[8], accl[8];  // sums of the first pieces' products and of the others'
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc[e] = accl[e] = v4f{0.0f, 0.0f, 0.0f, 0.0f};
     float mrun = -INFINITY, lrun = 0.0f;  // of query m
@@ -1571,7 +1575,7 @@ __global__ __launch_bounds__(256) void attention_mfma_kernel(AttnArgs a) {
 #pragma unroll
             for (int s = 0; s < 16; ++s) kr[s] = *reinterpret_cast<const v4u*>(knew + 32 * s + 8 * q);
         }
-        // (eight sums of the hi products and one of the lo products: a chain of 32 additions at the score's
+        // (eight sums of the first pieces' products and one of the others': a chain of 32 additions at the score's
         // size would double the error against 64 bits)
         v4f sh[8], sv = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -1581,6 +1585,7 @@ __global__ __launch_bounds__(256) void attention_mfma_kernel(AttnArgs a) {
             const h8 A = __builtin_bit_cast(h8, kr[s]);
             sh[s % 8] = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, *reinterpret_cast<const h8*>(qh + m * QP + 32 * s + 8 * q), sh[s % 8], 0, 0, 0);
             sv = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, *reinterpret_cast<const h8*>(ql + m * QP + 32 * s + 8 * q), sv, 0, 0, 0);
+            sv = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, *reinterpret_cast<const h8*>(qm + m * QP + 32 * s + 8 * q), sv, 0, 0, 0);
         }
         sv = (((sh[0] + sh[1]) + (sh[2] + sh[3])) + ((sh[4] + sh[5]) + (sh[6] + sh[7]))) + sv;
         if (k0 + 64 < k_end) load_k(k0 + 64);
@@ -1596,7 +1601,7 @@ __global__ __launch_bounds__(256) void attention_mfma_kernel(AttnArgs a) {
         const float mn = fmaxf(fmaxf(mrun, fmaxf(wmax[0][m], wmax[1][m])), fmaxf(wmax[2][m], wmax[3][m]));
         const float al = expf(mrun - mn);  // (key k0 is visible: mn is finite, or the sums end as NaN)
         float sum = 0.0f;
-        h4 hi, lo;
+        h4 hi, lo, lm;
 #pragma unroll
         for (int e = 0; e < 4; ++e) {
             const float p = sv[e] == -INFINITY ? 0.0f : expf(sv[e] - mn);
@@ -1604,7 +1609,9 @@ __global__ __launch_bounds__(256) void attention_mfma_kernel(AttnArgs a) {
             const float u = p * 16384.0f;
             hi[e] = (_Float16)u;
             lo[e] = (_Float16)(u - (float)hi[e]);
+            lm[e] = (_Float16)(u - (float)hi[e] - (float)lo[e]);
         }
+        *reinterpret_cast<h4*>(&pm[wave][m][4 * q]) = lm;
         *reinterpret_cast<h4*>(&ph[wave][m][4 * q]) = hi;
         *reinterpret_cast<h4*>(&pl[wave][m][4 * q]) = lo;
         sum = row_total(sum);
@@ -1626,7 +1633,7 @@ __global__ __launch_bounds__(256) void attention_mfma_kernel(AttnArgs a) {
                 if (key >= k_end) vr[g][i] = v4u{0u, 0u, 0u, 0u};  // (what a probability of zero multiplies must be finite)
                 else if (key == pos) vr[g][i] = *reinterpret_cast<const v4u*>(vnew + 128 * wave + 8 * m);
             }
-            const h4 bh = *reinterpret_cast<const h4*>(&ph[g][m][4 * q]), bl = *reinterpret_cast<const h4*>(&pl[g][m][4 * q]);
+            const h4 bh = *reinterpret_cast<const h4*>(&ph[g][m][4 * q]), bl = *reinterpret_cast<const h4*>(&pl[g][m][4 * q]), bm = *reinterpret_cast<const h4*>(&pm[g][m][4 * q]);
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
                 const uint32_t sel = e & 1 ? 0x07060302u : 0x05040100u;
@@ -1635,6 +1642,7 @@ __global__ __launch_bounds__(256) void attention_mfma_kernel(AttnArgs a) {
                 const h4 A = __builtin_bit_cast(h4, w);
                 acc[e] = __builtin_amdgcn_mfma_f32_16x16x16f16(A, bh, acc[e], 0, 0, 0);
                 accl[e] = __builtin_amdgcn_mfma_f32_16x16x16f16(A, bl, accl[e], 0, 0, 0);
+                accl[e] = __builtin_amdgcn_mfma_f32_16x16x16f16(A, bm, accl[e], 0, 0, 0);
             }
         }
         if (k0 + 64 < k_end) load_v(k0 + 64);
