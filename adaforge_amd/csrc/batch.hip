@@ -294,7 +294,7 @@ __global__ __launch_bounds__(512) void batch_input_kernel(BatchIn in) {
 //   FMA per token and row.
 // - Up to 8 tokens (PACK) the hi and lo halves are rows 0-7 and 8-15 of one MFMA operand, otherwise of two.
 // The waves' sums are added in LDS.  With S > 1 the ranges' sums go to planes in memory, and the last
-// workgroup of a row group to finish adds them (in split order) and writes y, unless the next kernel
+// workgroup of a row group to finish adds them and writes y, unless the next kernel
 // does (defer) or the planes are many (kFuseSplits: batch_reduce_kernel).
 //
 // Where a token has small blocks, a second form of the loop multiplies by their factors (3840 -> 15360, 32
@@ -378,6 +378,19 @@ __device__ __forceinline__ void spread_lanes(uint32_t v, uint32_t (&o)[4]) {
     o[1] = a[1];
     o[2] = b[0];
     o[3] = b[1];
+}
+
+// u[0] + ... + u[N - 1] (N a power of two), halves first: the rounding errors of log2 N additions in a row, not N - 1.
+template <int N>
+__device__ __forceinline__ float tree_sum(const float (&u)[N]) {
+    if constexpr (N == 1) {
+        return u[0];
+    } else {
+        float h[N / 2];
+#pragma unroll
+        for (int k = 0; k < N / 2; ++k) h[k] = u[2 * k] + u[2 * k + 1];
+        return tree_sum(h);
+    }
 }
 
 template <int G, bool PACK, int P, int RW, int W>
@@ -612,13 +625,13 @@ __global__ __launch_bounds__(64 * W) void batch_gemm_kernel(BatchGemm a, uint32_
         for (int p = 0; p < P; ++p) {
             float s = 0.0f;
             if (t < a.T) {
+                float u[KW];
 #pragma unroll
                 for (int k = 0; k < KW; ++k) {
                     const float* at = red + (size_t)k * TR * NR + t * NR + col + 16 * p;
-                    const float u = PACK ? at[0] + at[8 * NR] : at[0];
-                    s = k ? s + u : u;
+                    u[k] = PACK ? at[0] + at[8 * NR] : at[0];
                 }
-                s *= fabsf(inv[t]);
+                s = tree_sum(u) * fabsf(inv[t]);
             }
             v[j][p] = s;
         }
@@ -684,16 +697,14 @@ __global__ __launch_bounds__(64 * W) void batch_gemm_kernel(BatchGemm a, uint32_
             float s[P];
 #pragma unroll
             for (int p = 0; p < P; ++p) {
-                s[p] = u[j][p][0];
-#pragma unroll
-                for (uint32_t k = 1; k < FS; ++k) s[p] += u[j][p][k];
+                s[p] = tree_sum(u[j][p]);
             }
             if (t < a.T && row < a.w.rows) put(t, s);
         }
     }
 }
 
-// y from S split-K partial planes, summed in split order; one thread per (t, row).
+// y from S split-K partial planes; one thread per (t, row).
 template <int P>
 __global__ __launch_bounds__(256) void batch_reduce_kernel(BatchGemm a, uint32_t S, uint32_t Tp) {
     const uint32_t rows = a.w.rows, i = blockIdx.x * 256 + threadIdx.x;
@@ -703,8 +714,13 @@ __global__ __launch_bounds__(256) void batch_reduce_kernel(BatchGemm a, uint32_t
     float v[P];
 #pragma unroll
     for (int q = 0; q < P; ++q) {
-        float s = a.part[((size_t)q * Tp + t) * prow + row];
-        for (uint32_t k = 1; k < S; ++k) s += a.part[((size_t)(k * P + q) * Tp + t) * prow + row];
+        float s = 0.0f;  // four planes at a time
+        for (uint32_t k = 0; k < S; k += 4) {
+            float u[4];
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i) u[i] = k + i < S ? a.part[((size_t)((k + i) * P + q) * Tp + t) * prow + row] : 0.0f;
+            s += tree_sum(u);
+        }
         v[q] = s;
     }
     float* y = a.y + (size_t)t * a.y_stride + row;
