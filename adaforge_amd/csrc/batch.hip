@@ -1367,14 +1367,16 @@ __global__ __launch_bounds__(256, D == 256 ? 2 : 1) void wide_attention_kernel(B
         v4f sv[KT];
 #pragma unroll
         for (int kt = 0; kt < KT; ++kt) {
-            v4f x = {0.0f, 0.0f, 0.0f, 0.0f};
+            // (the small products in a sum of their own: fewer additions round at the score's size.  A layer's error
+            // against 64 bits over 512 positions 3.8e-7, with one sum 4.3e-7)
+            v4f x = {0.0f, 0.0f, 0.0f, 0.0f}, xl = x;
 #pragma unroll
             for (int s = 0; s < DS; ++s) {
                 const v8h A = *reinterpret_cast<const v8h*>(ks + (16 * kt + m) * KP + 32 * s + 8 * q);
                 x = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, qh[s], x, 0, 0, 0);
-                x = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, ql[s], x, 0, 0, 0);
+                xl = __builtin_amdgcn_mfma_f32_16x16x32_f16(A, ql[s], xl, 0, 0, 0);
             }
-            sv[kt] = x;
+            sv[kt] = x + xl;
         }
         float mx = -INFINITY;
 #pragma unroll

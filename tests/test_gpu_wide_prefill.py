@@ -149,6 +149,29 @@ def test_batched_trace_of_tiny_queries(batch):
     oracle.check_layer_stack(model, ids, outputs, kv, threads=THREADS, positions=[0, 1, 31, 32, 63, 64, 99])
 
 
+def test_wide_pass_is_no_less_exact_than_narrow_ones():
+    """A layer's error against the oracle over 512 positions: in one pass no larger than in passes of 32 (scores
+    summed in one chain made it 3 % larger)."""
+    model = synth.model(name="exact", layers=1, hidden=1024, intermediate=2048, q_heads=16, kv_heads=8, head_width=256,
+                        vocabulary=2048, window=1024, global_every=2)
+    n = 512
+    ids = np.array(synth.prompt_ids(n, model.vocabulary, name="exact.ids"), np.uint32)
+    emb = np.concatenate([oracle.embedding(model.table, 1024, 2048, ids[i:i + 256]) for i in (0, 256)]).reshape(n, -1)
+    table, error = oracle.layer_table(model), []
+    for batch in (32, 512):
+        with open_with_env(model, n + 8, AF_TRACE_BATCH=batch) as s:
+            out, kv, _, _ = s.trace(ids, kv_rows=8 * 256, logits=False, hidden=False)
+        num = den = 0.0
+        for t in range(1, n, 3):
+            k, v = (np.ascontiguousarray(kv[:t + 1, 0, i]) for i in (0, 1))
+            ref = oracle.layer_forward(model, table, 0, emb[t], k, v, t, given_kv=True, threads=THREADS)[0].astype(np.float64)
+            num += ((out[t, 0] - ref) ** 2).sum()
+            den += (ref ** 2).sum()
+        error.append((num / den) ** 0.5)
+    print(f"layer error over {n} positions: {error[0]:.3e} in passes of 32, {error[1]:.3e} in one", flush=True)
+    assert error[1] <= error[0]
+
+
 def test_wide_prefill_ids_match_one_position_at_a_time():
     """Greedy ids after a 300-token prompt: one wide pass against one step-kernel launch per position, and
     again on a follow-up turn whose pass starts in the middle of the ring."""
