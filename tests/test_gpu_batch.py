@@ -157,13 +157,13 @@ def test_batched_trace_long_chunks_teacher_forced(width):
 
 
 def test_batched_prefill_generation_matches_oracle_and_resumes():
-    """Generation with the default batched prefill: greedy ids equal the oracle's for a 75-token prompt
+    """Generation with a prefill batched 32 positions at a time: greedy ids equal the oracle's for a 75-token prompt
     (three batches, the local ring wrapping), then a follow-up turn on the cached prefix (its pending
     tokens prefilled in a batch) continues exactly as the oracle does."""
     model = batch_model(16, 8, 16, name="batch-gen")
     prompt = [int(i) for i in synth.prompt_ids(75, model.vocabulary, name="batch-gen.prompt")]
     stop = [model.vocabulary - 1]
-    with open_with_env(model, 160) as s:
+    with open_with_env(model, 160, AF_PREFILL_BATCH=32) as s:
         first = s.generate(prompt, stop, 8)
         turn2 = prompt + first.ids + [int(i) for i in synth.prompt_ids(40, model.vocabulary, name="batch-gen.more")]
         second = s.generate(turn2, stop, 8)

@@ -116,15 +116,17 @@ def test_session_prefix_reset_stop_and_budget_stack_rs_1887():
         assert again.stats.cached_tokens == 1 and again.stats.prompt_tokens == 1
 
 
-@pytest.mark.parametrize("step_kernel", ["1", "0"])
-def test_graph_matches_direct_for_changing_tokens_positions_and_reset_stack_rs_1980(step_kernel):
+@pytest.mark.parametrize("fall_back", [False, True])
+def test_graph_matches_direct_for_changing_tokens_positions_and_reset_stack_rs_1980(fall_back):
     """Graph replays and direct launches leave bit-identical caches: after generating from each
     sequence, a trace of one more token (which reads every cached K/V row of the sliding
-    window) returns identical layer outputs, appended K/V and logits on both sessions.  Both the
-    persistent step kernel (with the head, one graph per token) and the per-operation kernels."""
+    window) returns identical layer outputs, appended K/V and logits on both sessions.  The steps that are
+    replayed are the per-operation kernels': from the session's opening, or captured when a step-kernel launch
+    timed out (forced from the host at layer 0's down projection) in the middle of a generation."""
     model = fixture_model(packed_table(), 8, 2)
-    graph = open_with_env(model, 8, AF_STEP_KERNEL=step_kernel)
-    direct = open_with_env(model, 8, AF_STEP_KERNEL=step_kernel, AF_DISABLE_GRAPHS=1)
+    env = {"AF_STEP_FAIL_PHASE": 4} if fall_back else {"AF_STEP_KERNEL": "0"}
+    graph = open_with_env(model, 8, **env)
+    direct = open_with_env(model, 8, AF_DISABLE_GRAPHS=1, **env)
     try:
         for seq in ([0, 3, 1, 2], [4, 2, 0, 1]):
             a = graph.generate(seq[:3], [4], 2)
@@ -136,9 +138,28 @@ def test_graph_matches_direct_for_changing_tokens_positions_and_reset_stack_rs_1
                 assert np.array_equal(x, y)
             graph.reset()
             direct.reset()
+        assert not ran_step_kernel(graph, [0, 3])
     finally:
         graph.close()
         direct.close()
+
+
+def test_step_kernel_matches_per_operation_graph_for_changing_tokens_positions_and_reset():
+    """The step kernel's direct launches against the per-operation kernels' graph on the same sequences: the same ids,
+    and caches, layer outputs and logits of a further token to the rounding of their sums."""
+    model = fixture_model(packed_table(), 8, 2)
+    step, graph = open_with_env(model, 8), open_with_env(model, 8, AF_STEP_KERNEL="0")
+    try:
+        for seq in ([0, 3, 1, 2], [4, 2, 0, 1]):
+            assert step.generate(seq[:3], [4], 2).ids == graph.generate(seq[:3], [4], 2).ids
+            for x, y in zip(step.trace([seq[3]], kv_rows=256), graph.trace([seq[3]], kv_rows=256)):
+                assert np.abs(x - y).max() <= 1e-4 + 1e-3 * np.abs(y).max()
+            step.reset()
+            graph.reset()
+        assert ran_step_kernel(step, [0, 3])
+    finally:
+        step.close()
+        graph.close()
 
 
 def test_fixture_model_tokens_and_logits_match_oracle():

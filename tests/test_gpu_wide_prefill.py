@@ -38,6 +38,27 @@ def test_wide_trace_teacher_forced(q_heads, kv_heads, window, intermediate, n, b
     oracle.compare(oracle.q6_matvec(model.table, model.hidden, model.vocabulary, nrm, threads=THREADS), logits)
 
 
+@pytest.mark.parametrize("hidden,intermediate,n", [
+    (1024, 4128, 33),     # two octets per thread in the down projection's image, the second nearly empty; 64-token tile
+    (1024, 8192, 64),     # both whole
+    (1024, 15360, 65),    # four octets per thread, the last not whole; splits of a long K, 128-token tiles
+    (3840, 15360, 128),   # the 12B shape
+    (1024, 16384, 200),   # the longest K
+    (3840, 15360, 512),   # the largest pass
+])
+def test_wide_trace_long_columns(hidden, intermediate, n):
+    """Down projections of 4,128 to 16,384 columns (the image's wider forms, more splits of K) per layer against the oracle."""
+    model = synth.model(name=f"long{hidden}x{intermediate}", layers=1, hidden=hidden, intermediate=intermediate, q_heads=16,
+                        kv_heads=8, head_width=256, vocabulary=2048, window=1024, global_every=2)
+    ids = [int(i) for i in synth.prompt_ids(n, model.vocabulary, name=f"long{n}.ids")]
+    with open_with_env(model, n + 8, AF_TRACE_BATCH=512) as s:
+        outputs, kv, _, _ = s.trace(ids, kv_rows=8 * 256, logits=False, hidden=False)
+    positions = sorted({p for p in (0, 15, 16, 31, 32, 63, 64, 127, 128, 255, 256, n - 1) if p < n})
+    ratio, ulps, differ = oracle.check_layer_stack(model, ids, outputs, kv, threads=THREADS, positions=positions)
+    print(f"long columns {hidden}x{intermediate} n={n}: layer ratio {ratio:.3f}, K/V ratio {ulps:.3f}, {differ} fp16 "
+          f"values differ", flush=True)
+
+
 def test_wide_trace_gemma4_width_512_shared_v():
     """The 512-wide global layer (16 query heads on one KV head, V from K's weights) in wide passes."""
     model = synth.gemma4_model(name="gemma4-wide", layers=6, hidden=1024, intermediate=2048, local_q=(16, 8, 256),
