@@ -1515,29 +1515,33 @@ uint32_t batch_padded(uint32_t tokens) {
 // - 64 tokens: eight waves, four along K: a CU's 240 places hold a 15360-row gate/up pair once, and four waves
 //   in one place leave it waiting (3840 -> 2 x 15360: 50 us against 113 with four waves of 64 x 256).
 // - 128 tokens: eight waves, two along K, one workgroup per CU; or four waves, none along K, two workgroups
-//   per CU, which hide each other's barriers but need twice the splits.  The latter for grids of several
-//   rounds (512 tokens, the pair: 286 us against 323) and where they fill the places better; equal, the
-//   former, whose splits are fewer or none (128 tokens, 4096 -> 3840: 21.6 us against 25.5; 512 tokens, qkv:
-//   no partial sums), but for two or three splits (512 tokens, 15360 -> 3840: 145 us against 155).
+//   per CU, which hide each other's barriers but need twice the splits: the cheaper by wide_cost.
 // A gate/up pair is not split (its epilogue needs whole sums).
 struct WidePlan {
     uint32_t wk, mtiles, groups, S;
 };
+// Time in us of a 128-token form's `items` x S workgroups on 256 CUs, each S-th of K's blocks long, from rates
+// measured over 96 cases (1,024 to 15,360 rows and columns, 96 to 512 tokens), partial sums included: a step of a
+// CU's two workgroups of four waves 1.0 (one block each), of one alone 0.78, of one of eight waves 1.25 (two
+// blocks); 11 more to start and end the former; planes written and read back at 5 TB/s.  The cheaper of
+// the two by it was the faster but in 5 of the 96 (by 2-8 %): 4096 -> 3840, 512 tokens 52.2 us with eight waves (two
+// splits) against 54.2 (four), 15360 -> 3840 148.6 against 137.4; 128 tokens 28.5 against 33.0 and 48.4 against 49.8; 512
+// tokens, 3840 -> 8192 76.1 (no split) against 83.2, the 15360-row pair 300.9 against 253.7.
+static double wide_cost(uint32_t wk, uint32_t items, uint32_t S, uint32_t rows, uint32_t blocks, uint32_t tokens) {
+    const uint32_t steps = (blocks + S * wk - 1) / (S * wk), per = (items * S + 255) / 256;
+    const double planes = S > 1 ? (double)S * tokens * rows * 4 / 5e6 : 0.0;
+    return planes + (wk == 2 ? steps * 1.25 * per : steps * (per / 2 + 0.78 * (per % 2)) + 11.0);
+}
 static WidePlan wide_plan(uint32_t rows, uint32_t blocks, uint32_t tokens, bool pair) {
-    constexpr uint32_t kCus = 256, kRounds = 384;
+    constexpr uint32_t kCus = 256;
     const uint32_t m = wide_tokens(tokens), mtiles = (tokens + m - 1) / m, vrows = pair ? (rows + 31) / 32 * 64 : rows;
     const uint32_t groups = (vrows + 127) / 128, items = mtiles * groups;
     const auto splits = [&](uint32_t wk, uint32_t places) {
         return pair ? 1u : std::max<uint32_t>(1, std::min({places / items, kDeferParts, blocks / (kWideChain * wk)}));
     };
-    const auto used = [&](uint32_t S, uint32_t places) {  // share of the places of the rounds it takes
-        const uint32_t n = items * S;
-        return (double)n / ((n + places - 1) / places * places);
-    };
     if (m == 64) return WidePlan{4, mtiles, groups, splits(4, kCus)};
     const uint32_t S1 = splits(1, 2 * kCus), S2 = splits(2, kCus);
-    const double u1 = used(S1, 2 * kCus), u2 = used(S2, kCus);
-    const bool two = items < kRounds && (u2 > u1 + 0.02 || (u2 > u1 - 0.02 && S2 != 2 && S2 != 3));
+    const bool two = wide_cost(2, items, S2, rows, blocks, tokens) < wide_cost(1, items, S1, rows, blocks, tokens);
     return WidePlan{two ? 2u : 1u, mtiles, groups, two ? S2 : S1};
 }
 
