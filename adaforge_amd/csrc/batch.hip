@@ -318,23 +318,28 @@ constexpr uint32_t kFuseSplits = 4;
 // the weight stream, a range's input halves fit LDS and each wave has a super-tile.
 // - Up to 8 tokens W 8, RW 1: the halves are cheap to make (8 KB per 1,024 columns), so a workgroup per 64 rows
 //   makes its own (16 waves, 15360 -> 3840, 5 tokens: 15.6 us against 14.9; 4096 -> 3840: 11.0 against 8.9).
-// - Above, W 16 and RW 2 or 4 (up to 16 tokens, or 32) share them among more rows, where the matrix has
-//   kGemmLarge units of 64 rows x 128 columns, one wave's share of a super-tile, or more; below, such
-//   workgroups would leave most CUs idle and their sums take longer to add: W 8, RW 1, and two groups
-//   of 16 tokens (tg) that read the weights twice rather than one of 32.  4096 -> 3840, 32 tokens: 12.7 us
-//   against 17.0 with W 16, RW 4; 1024 -> 1000, 30 tokens: 7.1 against 9.3 with one group of 32.
+// - Above, the same with 16 tokens per workgroup (two groups tg of them above 16 tokens, which read the weights twice
+//   rather than share one workgroup: 1024 -> 1000, 30 tokens: 7.1 us against 9.3), where its workgroups fit the 256
+//   CUs in one round; their halves leave no room for a second one on a CU, so past that the grid takes two rounds,
+//   and W 16 and RW 2 or 4 (up to 16 tokens, or 32) share the halves among more rows instead.  Over 29 shapes of
+//   1,024 to 65,536 rows and 256 to 16,384 columns by 9 to 32 tokens the line lies there: 256 workgroups (8192 rows,
+//   3840 columns, 9 tokens) 11.2 us against 11.8 with W 16, 288 (6144, 3840) 16.4 against 11.5, 320 (5120, 4096, 24
+//   tokens) 21.6 against 15.1.  The one shape better on the other side is 15360 -> 3840 by 9 to 16 tokens (480; 23.8
+//   against 25.7).
 struct GemmPlan {
     uint32_t rw, waves, tg, groups, S;
 };
-constexpr uint32_t kGemmLarge = 3200;
 GemmPlan gemm_plan(uint32_t rows, uint32_t blocks, uint32_t T, bool pair) {
     const uint32_t tiles = (rows + 15) / 16 * (pair ? 2 : 1), nst = (blocks + 3) / 4;
-    const bool large = T > 8 && (uint64_t)tiles * nst >= 4 * kGemmLarge;
-    const uint32_t rw = !large ? 1 : T <= 16 ? 2 : 4, waves = large ? 16 : 8, tg = !large && T > 16 ? 2 : 1;
-    const uint32_t groups = (tiles + 4 * rw - 1) / (4 * rw) * tg;
-    const uint32_t most = kGemmLds / (4096u * (T <= 8 ? 1 : T <= 16 || tg == 2 ? 2 : 4));  // super-tiles of a range
-    const uint32_t need = (nst + most - 1) / most, want = std::max(1u, std::min((256 + groups / 2) / groups, large ? nst / (waves / rw) : (nst + 7) / 8));
-    return GemmPlan{rw, waves, tg, groups, std::max(need, std::min(want, kDeferParts))};
+    const auto form = [&](uint32_t rw, uint32_t waves, uint32_t tg) {
+        const uint32_t groups = (tiles + 4 * rw - 1) / (4 * rw) * tg;
+        const uint32_t most = kGemmLds / (4096u * (T <= 8 ? 1 : T <= 16 || tg == 2 ? 2 : 4));  // super-tiles of a range
+        const uint32_t need = (nst + most - 1) / most, each = waves == 16 ? nst / (waves / rw) : (nst + 7) / 8;
+        const uint32_t want = std::max(1u, std::min((256 + groups / 2) / groups, each));
+        return GemmPlan{rw, waves, tg, groups, std::max(need, std::min(want, kDeferParts))};
+    };
+    const GemmPlan p = form(1, 8, T > 16 ? 2 : 1);
+    return T <= 8 || p.groups * p.S <= 256 ? p : T <= 16 ? form(2, 16, 1) : form(4, 16, 1);
 }
 
 // Super-tiles [s0, s1) of range k of S.

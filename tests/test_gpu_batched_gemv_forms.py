@@ -23,6 +23,9 @@ pytestmark = pytest.mark.gpu
     (3840, 15360, 16), (15360, 3856, 13),          # 16 waves, 2 row waves
     (3840, 15361, 17), (3872, 15360, 32),          # 16 waves, 4 row waves, the last workgroup adds
     (15360, 3844, 31),                             # and with a reduce launch
+    (512, 16384, 16), (512, 16385, 16), (512, 16384, 17),  # 256 workgroups of 8 waves, and past one round of them
+    (256, 20480, 9), (32, 16400, 32),              # 16 waves, fewer super-tiles than waves along K
+    (4096, 5120, 16), (4096, 5120, 17),
 ])
 def test_forms_match_oracle(columns, rows, tokens):
     w = synth.q4(f"forms{columns}x{rows}", columns, rows, signed=True)
