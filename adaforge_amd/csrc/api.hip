@@ -393,7 +393,7 @@ float median_of(std::vector<float> t) {
     return n % 2 ? t[n / 2] : 0.5f * (t[n / 2 - 1] + t[n / 2]);
 }
 
-// Scratch for the standalone head / attention entry points (grown on demand, never shrunk).
+// Scratch for the standalone head, attention and batched GEMV entry points (grown on demand, never shrunk).
 struct Scratch {
     std::mutex mu;
     DevMem head_partial, head_counter, attn_part, attn_counters;
@@ -2174,7 +2174,7 @@ int generate_core(af_session* s, const uint32_t* prompt, size_t n_prompt, const 
     if (n_stop) HIP_OK(hipMemcpyAsync(s->STOPS.p, stop, n_stop * 4, hipMemcpyHostToDevice, st), "stop ids upload");
     std::memset(s->records + P, 0, (size_t)(s->capacity + 2 - P) * sizeof(StepRecord));
     // Positions consumed .. P - 2 fill the KV caches: in batches through the batched layers, or one
-    // step-kernel launch (graph replay) each; the decode steps then start at position P - 1.
+    // prefill step each; the decode steps then start at position P - 1.
     const bool batched = s->prefill_batch > 1 && pend > 1 && !timer;
     int rc = s->set_state(batched ? P - 1 : pend == 0 ? s->consumed - 1 : s->consumed, (uint32_t)n_stop);
     if (rc) return rc;
@@ -2206,7 +2206,7 @@ int generate_core(af_session* s, const uint32_t* prompt, size_t n_prompt, const 
     // Steps k0 .. k1 - 1 onto the stream.  At most kDecodeAhead steps are queued ahead of the one
     // being read back: the GPU never waits for the host (a step takes milliseconds, a launch
     // microseconds), and a call of many steps does not put thousands of kernel dispatches in flight
-    // at once (a 128-step call of a model whose decode graph holds 49 kernels would queue 6,272).
+    // at once (a 128-step call of a model whose step is 49 kernels would queue 6,272).
     uint32_t queued = 0;
     auto enqueue_range = [&](uint32_t k0, uint32_t k1) -> int {
         s->timer = timer;

@@ -9,14 +9,14 @@
 // it by the weight stream.  512 tokens through six layers of the 12B shape: 14.3 ms in 16 passes of 32,
 // 4.86 ms in one.
 //
-// Up to kBatchMax tokens each token's GEMM input is written as two fp16 halves per 32-element block: with u the block
-// scaled by 2^(14 - e) (e = ilogb of the block's max |x|, so that |u| < 2^15), hi = fp16(u) and
-// lo = fp16(u - hi), both rounded to nearest even; hi + lo holds u to about 2^-23 of the block's max.  The GEMM runs on the
-// fp16 matrix cores with the tokens in the MFMA's M dimension: v_mfma_f32_16x16x32_f16 with A = the
-// hi (then the lo) halves of 16 tokens over one 32-weight block (k) and B = the block's weights
-// n - 8 of 16 rows as fp16 (exact: each nibble placed in the mantissa of 1024 + n, then 1032
-// subtracted), both MFMAs accumulating into one fp32 tile, so D[t][r] = sum_j u_j(t) (n_rj - 8) with
-// every product exact.  Each lane adds d_r 2^(e - 14) D[t][r] to its fp32 partial per block.
+// The products run on the fp16 matrix cores (v_mfma_f32_16x16x32_f16) with the tokens in the M dimension: A =
+// a token's inputs over one 32-weight block (k) as two fp16 halves, B = the block's weights n - 8 of 16 rows as
+// fp16 (exact: each nibble placed in the mantissa of 1024 + n, then 1032 subtracted), so that D[t][r] =
+// sum_j u_j(t) (n_rj - 8) with every product exact.  The halves are of u, the inputs scaled by 2^(14 - e), e the
+// ilogb of the largest |x| of the token (a wide pass) or of the token's range of K (up to kBatchMax tokens):
+// |u| < 2^15, hi = fp16(u) and lo = fp16(u - hi), both rounded to nearest even, hold u to 2^-23 of itself, or to
+// 2^-25 where that is more; a block far below the largest has a scale of its own (block_spread).  Each lane adds d_r
+// D[t][r] to its fp32 sum per block, and the sum is multiplied by 2^(e - 14) once at the end.
 #include "device.h"
 
 namespace af {
@@ -103,8 +103,8 @@ __device__ __forceinline__ void wide_halves(const float (&v)[8], int sh, uint32_
 // float4), and every global load of the token (x, res and both norm weights) is issued before the
 // first reduction, so the kernel waits for memory once.
 // PS: x comes from in.parts split-K partial planes (NO == 1 only).
-// WIDE: the wide GEMM's image, one scale per token but for small blocks (block_spread); no padding tokens are written (their rows of the
-// product are never stored).  Workgroup b takes token (b % 8) ceil(T / 8) + b / 8, so that the 16
+// WIDE: the wide GEMM's image, one scale per token but for small blocks (block_spread); no padding tokens are
+// written (their rows of the product are never stored).  Workgroup b takes token (b % 8) ceil(T / 8) + b / 8, so that the 16
 // tokens whose halves share a 256-byte run of the image are mostly written through one XCD's L2.
 template <int NO, bool PS, bool WIDE>
 __global__ __launch_bounds__(512) void batch_input_kernel(BatchIn in) {
@@ -300,9 +300,9 @@ __global__ __launch_bounds__(512) void batch_input_kernel(BatchIn in) {
 // Where a token has small blocks, a second form of the loop multiplies by their factors (3840 -> 15360, 32
 // tokens: 22.7 us against 20.6; 15360 -> 3840, 5 tokens: 17.2 against 14.5).
 //
-// 3840 -> 15360, 32 tokens: 21.9 us against 34.3 us for the separate input-image, GEMM and reduce launches
+// 3840 -> 15360, 32 tokens: 20.4 us against 34.3 us for the separate input-image, GEMM and reduce launches
 // this replaced (16 operations per eight weights, a per-block input scale, operands from L2 one block
-// ahead); 15360 -> 3840, 5 tokens: 15.0 against 26.2 us.
+// ahead); 15360 -> 3840, 5 tokens: 14.5 against 26.2 us.
 
 namespace {
 
@@ -399,7 +399,8 @@ __device__ __forceinline__ float tree_sum(const float (&u)[N]) {
 }
 
 template <int G, bool PACK, int P, int RW, int W>
-__global__ __launch_bounds__(64 * W) void batch_gemm_kernel(BatchGemm a, uint32_t S, uint32_t groups, uint32_t tgroups, uint32_t fuse) {
+__global__ __launch_bounds__(64 * W) void batch_gemm_kernel(BatchGemm a, uint32_t S, uint32_t groups, uint32_t tgroups,
+                                                            uint32_t fuse) {
     constexpr int KW = W / RW, kTokens = PACK ? 8 : 16 * G;
     constexpr int NF = PACK ? 1 : 2 * G;        // 1 KB operands per block: [token group][hi, lo], or one packed
     constexpr uint32_t TR = 16 * G;             // operand rows (tokens; PACK: hi, then lo of eight tokens)
@@ -407,8 +408,8 @@ __global__ __launch_bounds__(64 * W) void batch_gemm_kernel(BatchGemm a, uint32_
     static_assert(W <= kTokens, "a wave per token in the input stage, or several tokens");
     constexpr int TW = kTokens / W;             // tokens per wave there
     constexpr int NO = kGemmLds / (4096 * NF) / 4;  // octet rounds of 64 lanes per token
-    constexpr int kAhead = W == 16 ? 1 : 2;     // super-tiles requested ahead (16 waves have 128 registers each)
-    //                   // super-tiles requested ahead of the one being multiplied
+    // super-tiles requested ahead of the one being multiplied (16 waves have 128 registers each)
+    constexpr int kAhead = W == 16 ? 1 : 2;
     extern __shared__ __align__(16) v4u smem[]; // input halves [block][NF][64 lanes], later sums [KW][TR][NR] f32
     __shared__ float inv[32];                   // the tokens' scales 2^(e - 14), negative with small blocks
     __shared__ __align__(16) float factor[1024];  // of those tokens' blocks (block_spread) [block][kTokens]
@@ -451,14 +452,16 @@ __global__ __launch_bounds__(64 * W) void batch_gemm_kernel(BatchGemm a, uint32_
         const size_t at = in ? st : 0;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(cp[i]) + at * 1024, 0, in ? 1024 : 0, 0x00020000);
-            const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(dp[i]) + at * 64, 0, in ? 128 : 0, 0x00020000);
+            const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint8_t*>(cp[i]) + at * 1024, 0,
+                                                                                 in ? 1024 : 0, 0x00020000);
+            const __amdgpu_buffer_rsrc_t rd = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(dp[i]) + at * 64, 0,
+                                                                                 in ? 128 : 0, 0x00020000);
             wc[u][i] = __builtin_amdgcn_raw_buffer_load_b128(rc, lane * 16, 0, 2);
             wd[u][i] = __builtin_amdgcn_raw_buffer_load_b16(rd, lane * 2, 0, 2);
         }
     };
 
-    // ---- inputs: token t = wave + 8 k, octet o = (block o / 4, part o % 4) of the range
+    // ---- inputs: token t = wave + W k, octet o = (block o / 4, part o % 4) of the range
     const uint32_t no = (s1 - s0) * 16;  // octets of the range, those past the last block zero
     v4f x[TW][NO][2];
 #pragma unroll
@@ -738,13 +741,13 @@ __global__ __launch_bounds__(256) void batch_reduce_kernel(BatchGemm a, uint32_t
 // y[t][r] = sum_b d_rb sum_j (n_rbj - 8) x_tbj for more than kBatchMax tokens.  A workgroup takes M = 64 WM
 // tokens x 64 WN rows over K range `split`, WM x WN waves of 64 x 64 (4 x 4 MFMA tiles) for each of WK
 // 32-weight blocks (one MFMA depth) per step: the tokens' halves are copied from the image, which
-// is laid out as the MFMAs read it, by LDS DMA two steps ahead, and the weights unpacked once per
-// workgroup into LDS while the step before is multiplied.  The WK waves of a tile add their sums in LDS at the end.  The block's d_rb differs from the next one's, so each block's 16 x 16
-// products are folded into fp32 sums on their own (one FMA per product and lane: half as many VALU
-// cycles as the two MFMAs take; the token's scale waits for the epilogue, so that the fold has no other
-// factor, unless a token of the tile has small blocks with scales of their own: then a second form of the
-// loop multiplies by the blocks' factors).  Sums run over kWideChain blocks, then join a total, so that no chain of fp32 additions is
-// longer than K / 32 / kWideChain + kWideChain.
+// is laid out as the MFMAs read it, by LDS DMA two steps ahead (one where WK is 4), and the weights unpacked once per
+// workgroup into LDS while the step before is multiplied.  The WK waves of a tile add their sums in LDS at the
+// end.  The block's d_rb differs from the next one's, so each block's 16 x 16 products are folded into fp32 sums on
+// their own (one FMA per product and lane: half as many VALU cycles as the two MFMAs take; the token's scale waits
+// for the epilogue, so that the fold has no other factor, unless a token of the tile has small blocks with scales
+// of their own: then a second form of the loop multiplies by the blocks' factors).  Sums run over kWideChain blocks,
+// then join a total, so that no chain of fp32 additions is longer than K / 32 / kWideChain + kWideChain.
 //
 // Work items (split, row group, token tile), token tile fastest, go to the XCDs in contiguous
 // shares (workgroup b runs on XCD b % 8), so that the workgroups that unpack the same weights share
@@ -753,7 +756,9 @@ constexpr uint32_t kWideChain = 8;
 typedef __attribute__((address_space(3))) void* lds_ptr;
 
 template <int WM, int WN, int WK, int P>
-__global__ __launch_bounds__(64 * WM * WN * WK, 2 / WK ? 2 / WK : 1) void wide_gemm_kernel(BatchGemm a, uint32_t S, uint32_t mtiles, uint32_t ngroups) {
+__global__ __launch_bounds__(64 * WM * WN * WK, 2 / WK ? 2 / WK : 1) void wide_gemm_kernel(BatchGemm a, uint32_t S,
+                                                                                             uint32_t mtiles,
+                                                                                             uint32_t ngroups) {
     constexpr int MG = 4 * WM, NT = 4 * WN;       // 16-token groups and 16-row tiles of the workgroup
     constexpr int W = WM * WN * WK, TH = 64 * W;  // waves, threads
     constexpr int SA = 8 / WN, SB = 4 / WM;       // 16-byte pieces of the image and code dwords per thread and step
@@ -1665,14 +1670,16 @@ static hipError_t wide_launch(const BatchGemm& a, hipStream_t s, uint32_t* parts
     else if (p.wk == 2) hipLaunchKernelGGL((wide_gemm_kernel<2, 2, 2, P>), grid, dim3(512), 0, s, a, S, p.mtiles, p.groups);
     else hipLaunchKernelGGL((wide_gemm_kernel<2, 2, 1, P>), grid, dim3(256), 0, s, a, S, p.mtiles, p.groups);
     hipError_t e = hipGetLastError();
-    if (e != hipSuccess || S == 1) return e;
-    if (a.defer) {
+    if (e != hipSuccess || S == 1) return e;  // (S is 1 for a pair)
+    if constexpr (P == 1) {
+        if (!a.defer) {
+            const uint32_t n = a.T * a.w.rows;
+            hipLaunchKernelGGL((batch_reduce_kernel<1>), dim3((n + 255) / 256), dim3(256), 0, s, a, S, 16 * wide_groups(a.T));
+            return hipGetLastError();
+        }
         if (parts) *parts = S;
-        return hipSuccess;
     }
-    const uint32_t n = a.T * a.w.rows;
-    hipLaunchKernelGGL((batch_reduce_kernel<P>), dim3((n + 255) / 256), dim3(256), 0, s, a, S, 16 * wide_groups(a.T));
-    return hipGetLastError();
+    return hipSuccess;
 }
 
 hipError_t launch_batch_gemm(const BatchGemm& a, bool gelu_pair, hipStream_t s, uint32_t* parts) {

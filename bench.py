@@ -5,9 +5,8 @@ Workload (the `value`): a 48-layer Gemma-3-12B-shaped model with seeded random w
 3840, FFN 15360, 16 q / 8 kv heads of width 256, 5:1 local(window 1024):global layers, Q4_0
 projections, tied Q6_K embedding/lm-head over 262144 ids); a 128-token random prompt is
 prefilled, then W warm-up and K timed greedy decode steps run through
-GenerationSession::generate (per token: one persistent launch for all 48 layers, one launch for
-the Q6_K head + greedy argmax, replayed as one hipGraph; ids come back through mapped host
-memory).  A "step" is one decoded token; `value` is tokens per second over the K timed steps.
+GenerationSession::generate (per token: one persistent launch for all 48 layers and one launch for
+the Q6_K head + greedy argmax; ids come back through mapped host memory).  A "step" is one decoded token; `value` is tokens per second over the K timed steps.
 
 After the timed region, PROFILE_STEPS more decode steps run with a hipEvent pair around every
 launch on the session stream (af_session_profile): the first half launch the step kernel plainly
@@ -23,8 +22,8 @@ CPU baseline: the C oracle (a port of the reference's FP64 CPU path), on this ho
 all of the box's CPU share (16 threads at most) and on one core, configs 0-3 in both modes.
 
 Beside the headline (`prefill`, `long_context`, `speculative` and `gemma4` in the JSON line): a
-512-id prompt prefilled on the config-4 model through the batched layers (32 positions per weight
-pass) and one step-kernel launch per position; config-4 decode after a 7620-id prompt; greedy
+512-id prompt prefilled on the config-4 model through the batched layers (in one weight pass, the
+default, and 32 positions per pass) and one step-kernel launch per position; config-4 decode after a 7620-id prompt; greedy
 speculative decoding with prompt-lookup drafts on a copying
 workload (config-4 shapes, local layers only, a prompt that repeats the model's own continuation),
 against plain decoding of the same prompt; and a full-size Gemma-4-shaped model (the reference's own
@@ -385,23 +384,23 @@ def open_env(model, capacity, **env):
 
 
 def prefill_leg(model, stop, tokens=512):
-    """Prefill of a `tokens`-id prompt on the config-4 model: batched (32 positions per weight pass,
-    the default) against one step-kernel launch per position (AF_PREFILL_BATCH=0); the first generated
-    id must agree."""
+    """Prefill of a `tokens`-id prompt on the config-4 model: batched (up to 512 positions per weight pass,
+    the default), 32 positions per pass, and one step-kernel launch per position (AF_PREFILL_BATCH=0); the
+    first generated id must agree."""
     from adaforge_amd import synth
     prompt = [int(i) for i in synth.prompt_ids(tokens, model.vocabulary, name="config4.prefill")]
     out = {"prompt_tokens": tokens}
     first = {}
-    for name, batch in (("batched", 32), ("stepwise", 0)):
-        with open_env(model, tokens + 8, AF_PREFILL_BATCH=batch) as s:
-            s.generate(prompt[:40], stop, 1)  # allocations and graph warm-up
+    for name, env in (("batched", {}), ("passes_of_32", {"AF_PREFILL_BATCH": 32}), ("stepwise", {"AF_PREFILL_BATCH": 0})):
+        with open_env(model, tokens + 8, **env) as s:
+            s.generate(prompt[:40], stop, 1)  # allocations
             s.reset()
             r = s.generate(prompt, stop, 1)
         ms = r.stats.prefill_ms
         first[name] = r.ids
         out[name] = {"ms": round(ms, 2), "tok_s": round((tokens - 1) / ms * 1000.0, 1)}
         log(f"prefill {tokens} tokens ({name}): {ms:.1f} ms -> {out[name]['tok_s']} tok/s")
-    out["same_first_id"] = first["batched"] == first["stepwise"]
+    out["same_first_id"] = first["batched"] == first["passes_of_32"] == first["stepwise"]
     return out
 
 
@@ -641,8 +640,7 @@ def main():
         "config": {
             "workload": "config4: 48-layer Gemma-3-12B-shaped decode loop, Q4_0 projections + tied Q6_K "
                         "embedding/lm-head (vocab 262144), 128-token prompt prefill then greedy decode steps "
-                        "(one persistent launch for the 48 layers + one head launch per token, replayed as a "
-                        "hipGraph), fp16 KV cache",
+                        "(one persistent launch for the 48 layers + one head launch per token), fp16 KV cache",
             "hidden": 3840, "intermediate": 15360, "layers": 48, "q_heads": 16, "kv_heads": 8, "head_width": 256,
             "prompt_tokens": PROMPT, "decode_tokens": a.warmup + produced, "batch": 1,
             "algorithmic_bytes_per_token": round(per_token_bytes),
