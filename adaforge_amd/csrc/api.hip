@@ -507,11 +507,11 @@ int af_q4_gemm(const af_q4* m, const float* x, uint32_t tokens, float* y, void* 
         return rc;
     const size_t tickets = batch_gemm_counters(w.rows, false), had = g_scratch.batch_counters.bytes;
     if ((rc = grow(g_scratch.batch_counters, tickets * 8, true, "batch counters"))) return rc;
-    if (const char* left = std::getenv("AF_GEMM_TICKETS_LEFT"); left && g_scratch.batch_counters.bytes != had) {
-        // (for tests: what calls that overlapped may leave)
-        const std::vector<uint64_t> v(tickets, std::strtoull(left, nullptr, 10));
-        HIP_OK(hipMemcpy(g_scratch.batch_counters.p, v.data(), tickets * 8, hipMemcpyHostToDevice), "batch counters");
-    }
+    if (g_scratch.batch_counters.bytes != had)
+        if (const char* left = std::getenv("AF_GEMM_TICKETS_LEFT")) {  // (for tests: what calls that overlapped may leave)
+            const std::vector<uint64_t> v(tickets, std::strtoull(left, nullptr, 10));
+            HIP_OK(hipMemcpy(g_scratch.batch_counters.p, v.data(), tickets * 8, hipMemcpyHostToDevice), "batch counters");
+        }
     // (whatever this call's y: a later call in place, under graph capture for instance, allocates nothing)
     if ((rc = grow(g_scratch.batch_x, (size_t)kBatchMax * w.blocks * 128, false, "batch vectors"))) return rc;
     const hipStream_t s = (hipStream_t)stream;
