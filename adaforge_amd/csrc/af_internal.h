@@ -245,7 +245,8 @@ struct BatchGemm {
     uint32_t T;
     float* y;               // y[t * y_stride + r], r < w.rows (gate/up: f32(gelu(gate)) * up)
     size_t y_stride;
-    float* part;            // split-K partials (batch_gemm_part_bytes)
+    float* part;            // split-K partials of part_bytes bytes (batch_gemm_part_bytes)
+    size_t part_bytes;
     uint64_t* counters;     // batch_gemm_counters tickets, zero between launches
     uint64_t epoch;         // tickets count from here: kEpochStep more than the launch's before it, or 0 where
                             // no two launches on these counters ever overlap
@@ -277,6 +278,8 @@ uint32_t batch_padded(uint32_t tokens);
 // Largest input image of a batch of at most `tokens` tokens.
 size_t batch_image_bytes(uint32_t blocks, uint32_t tokens);
 hipError_t launch_batch_attention(BatchAttn a, uint32_t head_width, hipStream_t s);
+// Bytes of split-K partials: of a launch of exactly `tokens` tokens, and the most of any of up to `tokens`.
+size_t batch_gemm_part_need(uint32_t rows, uint32_t blocks, uint32_t tokens, bool gelu_pair);
 size_t batch_gemm_part_bytes(uint32_t rows, uint32_t blocks, uint32_t tokens, bool gelu_pair);
 size_t batch_gemm_counters(uint32_t rows, bool gelu_pair);
 hipError_t launch_batch_input(const BatchIn& in, hipStream_t s);

@@ -530,6 +530,7 @@ int af_q4_gemm(const af_q4* m, const float* x, uint32_t tokens, float* y, void* 
     g.y = y;
     g.y_stride = w.rows;
     g.part = g_scratch.batch_part.as<float>();
+    g.part_bytes = g_scratch.batch_part.bytes;
     g.counters = g_scratch.batch_counters.as<uint64_t>();
     g.epoch = g_scratch.batch_epoch += kEpochStep;
     HIP_OK(launch_batch_gemm(g, false, s), "batched GEMV launch");
@@ -1414,6 +1415,7 @@ struct af_session {
         g.y = y;
         g.y_stride = y_stride;
         g.part = BGEMM.as<float>();
+        g.part_bytes = BGEMM.bytes;
         g.counters = BTICKETS.as<uint64_t>();
         g.defer = parts != nullptr;
         return launch_batch_gemm(g, m2 != nullptr, stream, parts);

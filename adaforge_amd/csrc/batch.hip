@@ -1553,7 +1553,9 @@ static WidePlan wide_plan(uint32_t rows, uint32_t blocks, uint32_t tokens, bool 
     };
     if (m == 64) return WidePlan{4, mtiles, groups, splits(4, kCus)};
     const uint32_t S1 = splits(1, 2 * kCus), S2 = splits(2, kCus);
-    const bool two = wide_cost(2, items, S2, rows, blocks, tokens) < wide_cost(1, items, S1, rows, blocks, tokens);
+    // (of whole tiles: every pass of as many takes the same plan, for which batch_gemm_part_bytes sizes the planes)
+    const uint32_t whole = mtiles * m;
+    const bool two = wide_cost(2, items, S2, rows, blocks, whole) < wide_cost(1, items, S1, rows, blocks, whole);
     return WidePlan{two ? 2u : 1u, mtiles, groups, two ? S2 : S1};
 }
 
@@ -1562,17 +1564,20 @@ size_t batch_image_bytes(uint32_t blocks, uint32_t tokens) {
     return tokens > kBatchMax ? std::max(floats, ((size_t)blocks * (2048 + 64) + 64) * ((tokens + 127) / 128 * 8)) : floats;
 }
 
+size_t batch_gemm_part_need(uint32_t rows, uint32_t blocks, uint32_t tokens, bool gelu_pair) {
+    const bool wide = tokens > kBatchMax;
+    const uint32_t S = wide ? wide_plan(rows, blocks, tokens, gelu_pair).S : gemm_plan(rows, blocks, tokens, gelu_pair).S;
+    const size_t planes = S * (wide || !gelu_pair ? 1u : 2u), prow = (rows + 15) / 16 * 16;  // (a wide pair is not split)
+    return S > 1 ? planes * batch_padded(tokens) * prow * 4 : 0;
+}
+
 size_t batch_gemm_part_bytes(uint32_t rows, uint32_t blocks, uint32_t tokens, bool gelu_pair) {
-    size_t most = 0;  // the largest over the passes of up to `tokens` tokens
-    const size_t prow = (rows + 15) / 16 * 16;
-    for (uint32_t t : {8u, 16u, 32u}) {
-        const uint32_t T = std::min(t, tokens), S = gemm_plan(rows, blocks, T, gelu_pair).S;
-        if (S > 1) most = std::max(most, (size_t)S * (gelu_pair ? 2 : 1) * padded_tokens(T) * prow * 4);
-    }
-    for (uint32_t t = 64; t < tokens + 64 && tokens > kBatchMax; t += 64) {
-        const uint32_t T = std::min(t, tokens), S = wide_plan(rows, blocks, T, gelu_pair).S;
-        if (S > 1) most = std::max(most, (size_t)S * 16 * wide_groups(T) * prow * 4);
-    }
+    size_t most = 0;  // the largest over the passes of up to `tokens` tokens: one of each plan
+    for (uint32_t t : {8u, 16u, 32u, 64u})
+        if (t <= 32 || tokens > kBatchMax)
+            most = std::max(most, batch_gemm_part_need(rows, blocks, std::min(t, tokens), gelu_pair));
+    for (uint32_t t = 128; t < tokens + 128 && tokens > 64; t += 128)
+        most = std::max(most, batch_gemm_part_need(rows, blocks, std::min(t, tokens), gelu_pair));
     return most;
 }
 
@@ -1639,7 +1644,7 @@ static hipError_t gemm_launch(const BatchGemm& a, hipStream_t s, uint32_t* parts
     const bool defer = a.defer && P == 1 && p.S > 1;
     const uint64_t planes = (uint64_t)p.S * P * Tp * ((a.w.rows + 15) / 16 * 16) * 4;
     const bool fuse = p.S > 1 && !defer && a.counters && p.S <= (G == 2 ? kFuseSplits : kDeferParts) && planes < 0x7FFFFFFFu;
-    if (p.S > 1 && !a.part) return hipErrorInvalidValue;
+    if (p.S > 1 && (!a.part || a.part_bytes < planes)) return hipErrorInvalidValue;
     const uint32_t range = (a.w.nst + p.S - 1) / p.S;  // super-tiles, at most
     const size_t lds = std::max<size_t>((size_t)range * 4096 * (PACK ? 1 : 2 * G), 256 * p.waves * TR);  // (operands, later the waves' sums)
     const dim3 grid((p.groups * p.S + 7) / 8 * 8);
@@ -1666,7 +1671,7 @@ template <int P>
 static hipError_t wide_launch(const BatchGemm& a, hipStream_t s, uint32_t* parts) {
     const WidePlan p = wide_plan(a.w.rows, a.w.blocks, a.T, P == 2);
     const uint32_t S = p.S;
-    if (S > 1 && !a.part) return hipErrorInvalidValue;
+    if (S > 1 && (!a.part || a.part_bytes < batch_gemm_part_need(a.w.rows, a.w.blocks, a.T, P == 2))) return hipErrorInvalidValue;
     const dim3 grid((p.mtiles * p.groups * S + 7) / 8 * 8);
     if (p.wk == 4) hipLaunchKernelGGL((wide_gemm_kernel<1, 2, 4, P>), grid, dim3(512), 0, s, a, S, p.mtiles, p.groups);
     else if (p.wk == 2) hipLaunchKernelGGL((wide_gemm_kernel<2, 2, 2, P>), grid, dim3(512), 0, s, a, S, p.mtiles, p.groups);
