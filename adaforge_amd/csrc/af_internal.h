@@ -300,8 +300,8 @@ uint32_t attention_block_heads(uint32_t group, uint32_t head_width);
 // Decode attention of 512-wide heads on the matrix cores (attention_mfma_kernel), with kAttnMfmaGroup or more
 // query heads per KV head and more than kAttnMfmaSpan visible positions: its two launches take 16-18 us up to
 // 4,096 positions of one KV head, attention_kernel 9-15 us up to 1,024 and 19-31 from 1,025 on (4 to 16 query
-// heads); with more KV heads the distance grows (8 of 4 query heads, 4,096 positions: 24 us against 54; 512 of
-// them, 1,025 positions: 0.25 ms against 1.05).
+// heads); with more KV heads the distance grows (8 of 4 query heads, 4,096 positions: 25 us against 54; 512 of
+// them, 1,025 positions: 0.26 ms against 1.05).
 // a.cmax from attention_mfma_chunks, a.part of kv_heads cmax group rows (attn_part_row).
 constexpr uint32_t kAttnMfmaGroup = 4, kAttnMfmaSpan = 1024, kAttnMfmaChunks = 256;
 bool attention_mfma(uint32_t group, uint32_t head_width, uint32_t span);

@@ -1414,9 +1414,8 @@ __global__ __launch_bounds__(D) void attention_kernel(AttnArgs a) {
 // are not finite takes its channels again key by key in fp32 (plain_attention), as attention_kernel computes
 // them; the check is 33 FMAs and a ballot per wave (0.2 us at 4,096 positions, with a barrier more 0.6).
 //
-// 16 query heads on one KV head: 17.9 us against 31.1 at 4,096 positions, 31.7 against 88 at 32,768 (of
-// them 4.8 us the merge, 3 us the loop at 4,096, the rest the launch and the prologue's chain).  Error
-// against 64 bits 2.1e-7 at 4,096 (attention_kernel: 2.2e-7).
+// 16 query heads on one KV head: 17.9 us against 31.1 at 4,096 positions (of them 4.1 us the merge, the rest the
+// launch, the prologue's chain and 64 keys per workgroup), 32.0 against 88 at 32,768.
 // Keys per chunk (a multiple of 64) and chunks of n visible keys in at most cmax chunks.
 __host__ __device__ inline uint32_t attn_mfma_span(uint32_t n, uint32_t cmax) {
     const uint32_t tiles = (n + 63) / 64;
